@@ -1113,46 +1113,41 @@ __global__ __launch_bounds__(kThreads) void sig_freq_gemm_kernel(const T* __rest
 // tree per k, FP64), with Im(zsec_mm) <= 0 after every k: the reference clips
 // after every (k, band block) call (S/m_sxcf_gemm.f90:599-608).  The partials
 // of k are [kstart[k], kstart[k+1]) when kstart is given, else
-// [k*chunks, (k+1)*chunks).  One block per output element.
+// [k*chunks, (k+1)*chunks).  One wave per output element, no barriers (a
+// 256-thread tree per element and k took 10 us for 8 k of 7 partials).
 template <class T>
 __global__ __launch_bounds__(256) void sig_final_reduce_kernel(const T* __restrict__ part, int nk, int chunks,
                                                                const int* __restrict__ kstart, int ntq,
                                                                cd* __restrict__ zsec, int64_t ldz) {
-  __shared__ double sr[256], si[256];
   const int np = ntq * ntq;
-  const int p = blockIdx.x;
+  const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (p >= np) return;
   const int m = p % ntq, mp = p / ntq;
   cd* z = zsec + m + ldz * mp;
   const cd z0 = *z;
-  double zr = z0.re, zi = z0.im;  // running value (thread 0's copy is the one written)
+  double zr = z0.re, zi = z0.im;
   for (int k = 0; k < nk; ++k) {
     const int q0 = kstart ? kstart[k] : k * chunks, q1 = kstart ? kstart[k + 1] : (k + 1) * chunks;
     double a = 0.0, c = 0.0;
-    for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
+    for (int q = q0 + lane; q < q1; q += 64) {
       double xr, xi;
       ld_c2(part + (int64_t)np * q + p, xr, xi);
       a += xr;
       c += xi;
     }
-    sr[threadIdx.x] = a;
-    si[threadIdx.x] = c;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) {
-        sr[threadIdx.x] += sr[threadIdx.x + w];
-        si[threadIdx.x] += si[threadIdx.x + w];
-      }
-      __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) {
+      a += __shfl_xor(a, o);
+      c += __shfl_xor(c, o);
     }
-    zr += sr[0];
-    zi += si[0];
+    zr += a;
+    zi += c;
     if (m == mp && zi > 0.0) zi = 0.0;
-    __syncthreads();
   }
-  if (threadIdx.x == 0) *z = cd{zr, zi};
+  if (lane == 0) *z = cd{zr, zi};
 }
 
-// Split-K partials of the final product (S/m_sxcf_gemm.f90:599):
+// Split-K partials of the final product (S/m_sxcf_gemm.f90:599) on the GEMM
+// engine (FP64 and FP32 forms, and more than kSigFinalMax end states):
 // part[chunk][b] (ntq x ntq) = cz_b(chunk rows)^H zmel_b(chunk rows) for gb
 // internal k-points of R = n*nm rows each (per-k strides zs), chunks of KC rows.
 constexpr int SIG_KC = 2048;
@@ -1216,7 +1211,9 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_CZ, cz_bytes_per * group, (void**)&cz));
   // final product: split-K partials of czmelwc^H zmel (K = n*nm per internal k)
   const int64_t R = (int64_t)n * nm;
-  const int chunks = sig_chunks(R);
+  const bool direct = MODE == MBF3 && ntq <= kSigFinalMax;
+  const int KC = direct ? sig_final_chunk(R * nbatch) : SIG_KC;
+  const int chunks = (int)((R + KC - 1) / KC);
   const int np = ntq * ntq;
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_PART, sizeof(T) * (size_t)np * chunks * nbatch, (void**)&part));
   const int64_t wstride = ldw * n * nw1;
@@ -1249,10 +1246,14 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
     }
     if (rp)  // czmelwc += real-axis pole columns (S/m_sxcf_gemm.f90:586-589)
       ECALJ_TRY(real_plan_into_cz(h, rp, *rs, MODE == M64 ? M64 : M32, zmel, n, nm, ntq, b0, b0 + gb, cz));
-    ECALJ_TRY((sig_final_partials<MODE, T>(h, cz, zmel + (int64_t)n * ncol * b0, R, (int64_t)n * ncol, gb, ntq,
-                                            part + (int64_t)np * chunks * b0)));
+    if (direct)
+      ECALJ_TRY(sig_final_bf3(h, (const cf*)cz, (const cf*)zmel + (int64_t)n * ncol * b0, R, (int64_t)n * ncol, chunks,
+                              nullptr, gb, (int64_t)chunks * gb, KC, ntq, (cf*)part + (int64_t)np * chunks * b0));
+    else
+      ECALJ_TRY((sig_final_partials<MODE, T>(h, cz, zmel + (int64_t)n * ncol * b0, R, (int64_t)n * ncol, gb, ntq,
+                                              part + (int64_t)np * chunks * b0)));
   }
-  hipLaunchKernelGGL((sig_final_reduce_kernel<T>), dim3(np), dim3(256), 0, h->stream, part, nbatch, chunks,
+  hipLaunchKernelGGL((sig_final_reduce_kernel<T>), dim3((np + 3) / 4), dim3(256), 0, h->stream, part, nbatch, chunks,
                      (const int*)nullptr, ntq, zsec, ldz);
   ECALJ_HIP(hipGetLastError());
   return ECALJ_OK;
@@ -1298,14 +1299,31 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
   }
   maxg = std::max(maxg, acc);
   gstart.push_back(nk);
-  int64_t nparts = 0;
-  for (int k = 0; k < nk; ++k) nparts += nm[k] ? sig_chunks((int64_t)n * nm[k]) : 0;
+  // chunks of the final product per k
+  const bool direct = ntq <= kSigFinalMax;
+  int64_t rows = 0, nparts = 0;
+  for (int k = 0; k < nk; ++k) rows += (int64_t)n * nm[k];
+  const int KC = direct ? sig_final_chunk(rows) : SIG_KC;
+  std::vector<SigFinalK> tab(nk);
+  std::vector<int> kst(nk + 1, 0);
+  for (int k = 0; k < nk; ++k) {
+    const int64_t R = (int64_t)n * nm[k];
+    tab[k] = SigFinalK{(int64_t)n * zoff[k], R, nparts};
+    nparts += (R + KC - 1) / KC;
+    if (nparts > 0x7fffffff) return ECALJ_ERR_DIM;
+    kst[k + 1] = (int)nparts;
+  }
+  const size_t tb = sizeof(SigFinalK) * nk;
+  std::vector<unsigned char> blob(tb + sizeof(int) * (nk + 1));
+  memcpy(blob.data(), tab.data(), tb);
+  memcpy(blob.data() + tb, kst.data(), sizeof(int) * (nk + 1));
+  unsigned char* dtab;
+  ECALJ_TRY(upload_blob(h, ecalj_ctx::S_KST, blob, &dtab));
   unsigned char* wh;
   cf* part;
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_WH, maxg, (void**)&wh));
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_PART, sizeof(cf) * (size_t)np * std::max<int64_t>(nparts, 1),
                         (void**)&part));
-  int64_t pofs = 0;
   for (size_t gi = 0; gi + 1 < gstart.size(); ++gi) {
     const int k0 = gstart[gi], k1 = gstart[gi + 1];
     std::vector<int> ncol(k1 - k0);
@@ -1321,26 +1339,22 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
     ECALJ_TRY((h->sigc_fp8 ? sig_f8_grouped : sig_bf3_grouped)(h, k1 - k0, ncol.data(), z + (int64_t)n * zoff[k0],
                                                                n, nw1, wc + wstride * k0, ldw, wstride,
                                                                wgt + nw1 * zoff[k0], cz, as, bs));
+    if (direct) {
+      ECALJ_TRY(sig_final_bf3(h, cz, z + (int64_t)n * zoff[k0], 0, 0, 0, (const SigFinalK*)dtab + k0, k1 - k0,
+                              kst[k1] - kst[k0], KC, ntq, part + (int64_t)np * kst[k0]));
+      continue;
+    }
     int64_t cofs = 0;
     for (int k = k0; k < k1; ++k) {
       if (nm[k] == 0) continue;
       const int64_t R = (int64_t)n * nm[k];
       ECALJ_TRY((sig_final_partials<MBF3, cf>(h, cz + cofs, z + (int64_t)n * zoff[k], R, 0, 1, ntq,
-                                              part + (int64_t)np * pofs)));
-      cofs += (int64_t)n * nm[k] * ntq;
-      pofs += sig_chunks(R);
+                                              part + (int64_t)np * kst[k])));
+      cofs += R * ntq;
     }
   }
-  std::vector<unsigned char> ks(sizeof(int) * (nk + 1));
-  {
-    int* kp = reinterpret_cast<int*>(ks.data());
-    kp[0] = 0;
-    for (int k = 0; k < nk; ++k) kp[k + 1] = kp[k] + (nm[k] ? sig_chunks((int64_t)n * nm[k]) : 0);
-  }
-  unsigned char* dks;
-  ECALJ_TRY(upload_blob(h, ecalj_ctx::S_KST, ks, &dks));
-  hipLaunchKernelGGL((sig_final_reduce_kernel<cf>), dim3(np), dim3(256), 0, h->stream, part, nk, 0,
-                     (const int*)dks, ntq, zsec, ldz);
+  hipLaunchKernelGGL((sig_final_reduce_kernel<cf>), dim3((np + 3) / 4), dim3(256), 0, h->stream, part, nk, 0,
+                     (const int*)(dtab + tb), ntq, zsec, ldz);
   ECALJ_HIP(hipGetLastError());
   return ECALJ_OK;
 }

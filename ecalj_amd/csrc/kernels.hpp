@@ -99,6 +99,16 @@ ecalj_status sig3m_grouped_prep(ecalj_ctx* h, int nk, const int* ncol, const cf*
                                 int64_t ldw, int64_t w_stride, unsigned short* as, cf* zp);
 ecalj_status sig3m_grouped_run(ecalj_ctx* h, int wm, int nk, const int* ncol, int n, int nw1,
                                const unsigned short* as, const cf* zp, const double* wgt, cf* cz);
+// Split-K partials of the bf16x3 final product (sigfinal.hip), up to
+// kSigFinalMax end states; one entry per k of the grouped form.
+constexpr int kSigFinalMax = 64;
+struct SigFinalK {
+  int64_t off, R;  // zmel / czmelwc of the k (elements), its rows
+  int64_t p0;      // its first chunk
+};
+int sig_final_chunk(int64_t rows);
+ecalj_status sig_final_bf3(ecalj_ctx* h, const cf* cz, const cf* z, int64_t R, int64_t zs, int chunks,
+                           const SigFinalK* tab, int nk, int64_t nblk, int KC, int ntq, cf* part);
 // x0gemm in the bf16x3 form: per-bin entry lists on the host (bin b: entries
 // cnt[b]..cnt[b+1]-1 with zmel column offsets col[] and weights wt[]), output
 // slice slice[b] of rcxq (npr x npr_col, complex64, slice stride slice_elems)
