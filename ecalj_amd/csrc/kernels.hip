@@ -1186,6 +1186,11 @@ static ecalj_status sig_final_partials(ecalj_ctx* h, const T* cz, const T* zmel,
   return ECALJ_OK;
 }
 
+// Scratch of one group of internal k-points (operands + czmelwc).  The mode
+// form keeps the planes of every group of columns and takes twice as much, so
+// that a launch still holds several k (C3: 6 of 12).
+constexpr size_t kSigScratch = (size_t)8 << 30, kSigModeScratch = (size_t)16 << 30;
+
 template <int MODE, class T>
 static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int n, int nm, int ntq, int niw,
                                    const cd* wc, int64_t ldw, const double* wgt, cd* zsec, int64_t ldz,
@@ -1203,10 +1208,15 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   T *wh, *cz, *part;
   // W unpacked (or, for bf16x3, split into bf16 planes) per internal k;
   // processed in groups to bound scratch memory
-  const size_t wh_bytes_per = (MODE == MBF3) ? sig_bf3_bytes_per_k(n, ncol, nw1) : sizeof(T) * nn * nw1;
+  const bool modes = MODE == MBF3 && sig_modes_pays(h, n, (int64_t)ncol * nbatch, nbatch, nw1);
+  const size_t wh_bytes_per = modes ? sig_modes_bytes(n, nm, ntq, nw1)
+                              : (MODE == MBF3) ? sig_bf3_bytes_per_k(n, ncol, nw1) : sizeof(T) * nn * nw1;
   const size_t cz_bytes_per = sizeof(T) * (size_t)n * ncol;
-  int group = (int)std::max<size_t>(1, std::min<size_t>(nbatch, ((size_t)8 << 30) / (wh_bytes_per + cz_bytes_per)));
+  const size_t cap = modes ? kSigModeScratch : kSigScratch;
+  int group = (int)std::max<size_t>(1, std::min<size_t>(nbatch, cap / (wh_bytes_per + cz_bytes_per)));
   group = std::min(group, 65535);
+  if (modes) group = (nbatch + (nbatch + group - 1) / group - 1) / ((nbatch + group - 1) / group);  // even parts
+  const std::vector<int> nms(modes ? group : 0, nm);
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_WH, wh_bytes_per * group, (void**)&wh));
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_CZ, cz_bytes_per * group, (void**)&cz));
   // final product: split-K partials of czmelwc^H zmel (K = n*nm per internal k)
@@ -1221,7 +1231,10 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   const int ublocks = (int)std::min<int64_t>((tot + 255) / 256, 65536);
   for (int b0 = 0; b0 < nbatch; b0 += group) {
     const int gb = std::min(group, nbatch - b0);
-    if constexpr (MODE == MBF3) {
+    if (MODE == MBF3 && modes) {
+      ECALJ_TRY(sig_modes(h, gb, nms.data(), ntq, (const cf*)zmel + (int64_t)n * ncol * b0, n, nw1, wc + wstride * b0,
+                          ldw, wstride, wgt + (int64_t)nw1 * ncol * b0, (cf*)cz, (unsigned char*)wh));
+    } else if constexpr (MODE == MBF3) {
       unsigned short* as = reinterpret_cast<unsigned short*>(wh);
       unsigned short* bs = as + sig_bf3_a_elems_per_k(n, nw1) * gb;
       ECALJ_TRY((h->sigc_fp8 ? sig_f8 : sig_bf3)(h, gb, (const cf*)zmel + (int64_t)n * ncol * b0,
@@ -1284,13 +1297,17 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
   }
   const cf* z = (const cf*)zmel;
   const int np = ntq * ntq;
-  // scratch groups of consecutive k under 8 GB
+  // scratch groups of consecutive k
+  const bool modes = sig_modes_pays(h, n, zoff[nk], nk, nw1);
+  const size_t cap = modes ? kSigModeScratch : kSigScratch;
   std::vector<int> gstart{0};
   size_t acc = 0;
   size_t maxg = 0;
   for (int k = 0; k < nk; ++k) {
-    const size_t b = sig_bf3_bytes_per_k(n, std::max(nm[k] * ntq, 1), nw1) + sizeof(cf) * (size_t)n * nm[k] * ntq;
-    if (acc > 0 && acc + b > ((size_t)8 << 30)) {
+    const size_t b = (modes ? sig_modes_bytes(n, nm[k], ntq, nw1)
+                            : sig_bf3_bytes_per_k(n, std::max(nm[k] * ntq, 1), nw1)) +
+                     sizeof(cf) * (size_t)n * nm[k] * ntq;
+    if (acc > 0 && acc + b > cap) {
       gstart.push_back(k);
       maxg = std::max(maxg, acc);
       acc = 0;
@@ -1326,19 +1343,28 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
                         (void**)&part));
   for (size_t gi = 0; gi + 1 < gstart.size(); ++gi) {
     const int k0 = gstart[gi], k1 = gstart[gi + 1];
-    std::vector<int> ncol(k1 - k0);
-    size_t a_elems = sig_bf3_a_elems_per_k(n, nw1) * (k1 - k0);
-    size_t b_bytes = 0;
-    for (int k = k0; k < k1; ++k) {
-      ncol[k - k0] = nm[k] * ntq;
-      b_bytes += sig_bf3_bytes_per_k(n, std::max(ncol[k - k0], 1), nw1) - 2 * sig_bf3_a_elems_per_k(n, nw1);
+    cf* cz;
+    if (modes) {
+      size_t b = 0;
+      for (int k = k0; k < k1; ++k) b += sig_modes_bytes(n, nm[k], ntq, nw1);
+      cz = reinterpret_cast<cf*>(wh + b);
+      ECALJ_TRY(sig_modes(h, k1 - k0, nm + k0, ntq, z + (int64_t)n * zoff[k0], n, nw1, wc + wstride * k0, ldw, wstride,
+                          wgt + nw1 * zoff[k0], cz, wh));
+    } else {
+      std::vector<int> ncol(k1 - k0);
+      size_t a_elems = sig_bf3_a_elems_per_k(n, nw1) * (k1 - k0);
+      size_t b_bytes = 0;
+      for (int k = k0; k < k1; ++k) {
+        ncol[k - k0] = nm[k] * ntq;
+        b_bytes += sig_bf3_bytes_per_k(n, std::max(ncol[k - k0], 1), nw1) - 2 * sig_bf3_a_elems_per_k(n, nw1);
+      }
+      unsigned short* as = reinterpret_cast<unsigned short*>(wh);
+      unsigned short* bs = as + a_elems;
+      cz = reinterpret_cast<cf*>(reinterpret_cast<unsigned char*>(bs) + b_bytes);
+      ECALJ_TRY((h->sigc_fp8 ? sig_f8_grouped : sig_bf3_grouped)(h, k1 - k0, ncol.data(), z + (int64_t)n * zoff[k0],
+                                                                 n, nw1, wc + wstride * k0, ldw, wstride,
+                                                                 wgt + nw1 * zoff[k0], cz, as, bs));
     }
-    unsigned short* as = reinterpret_cast<unsigned short*>(wh);
-    unsigned short* bs = as + a_elems;
-    cf* cz = reinterpret_cast<cf*>(reinterpret_cast<unsigned char*>(bs) + b_bytes);
-    ECALJ_TRY((h->sigc_fp8 ? sig_f8_grouped : sig_bf3_grouped)(h, k1 - k0, ncol.data(), z + (int64_t)n * zoff[k0],
-                                                               n, nw1, wc + wstride * k0, ldw, wstride,
-                                                               wgt + nw1 * zoff[k0], cz, as, bs));
     if (direct) {
       ECALJ_TRY(sig_final_bf3(h, cz, z + (int64_t)n * zoff[k0], 0, 0, 0, (const SigFinalK*)dtab + k0, k1 - k0,
                               kst[k1] - kst[k0], KC, ntq, part + (int64_t)np * kst[k0]));

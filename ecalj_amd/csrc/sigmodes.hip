@@ -1,0 +1,557 @@
+// sigmodes.hip -- the bf16x3 Sigma_c frequency contraction in frequency modes.
+//
+//   czmelwc(I,c) = sum_v sum_J Wt_v(I,J) wgt(v,c) zmel(J,c)
+//
+// costs one product of a W with zmel per frequency.  The weights of a range
+// of middle states are smooth in the energy difference to the end state, so
+// their vectors over the frequencies span far fewer dimensions than there
+// are frequencies: with an orthonormal basis Q (nw1 x R) of the weights of a
+// group of columns,
+//   wgt(v,c) = sum_r (Q_vr / s_v) g_r(c),  g_r(c) = sum_v Q_vr s_v wgt(v,c),
+//   czmelwc(I,c) = sum_r sum_J [sum_v Q_vr / s_v Wt_v](I,J) g_r(c) zmel(J,c),
+// R products instead of nw1.  s_v is the Frobenius norm of W_v, so that a
+// column's error is weighed as it enters the product.  R is the number of
+// steps of a pivoted Gram-Schmidt after which the residual of EVERY column of
+// the group is at most kModeTol = 2^-25 of that column's norm, the rounding
+// of a weight to FP32 (which every form of the contraction does); weights
+// that span all frequencies give R = nw1 and the plain contraction.
+// R is found and used on the device: no host wait, and a captured graph
+// replays with the ranks of its present inputs.
+//
+// Grouping: a column's weights depend on the distance |e_n - omega_m| of its
+// middle and end states, and columns of like distance span few dimensions, so
+// the columns of a k are sorted by it (by the weight at the highest frequency,
+// which grows with it; whatever the weights are, the order only decides how
+// low the ranks get) and taken in groups of whole column tiles.  C3, 21
+// frequencies: mean rank 17 for one group, 8.8 for 4, 6.8 for 8, 6.0 for 12;
+// groups of consecutive middle states instead of sorted columns: 10.6 for 8.
+// More groups mean more modes to form and write; one mode costs about as much
+// as 1.5 column tiles at one rank.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <vector>
+
+#include "sig3mtile.hpp"
+
+namespace ecalj {
+
+constexpr int kModeMax = Q3NW;    // frequencies, and therefore modes, of one launch
+constexpr int kModeChunks = 16;   // partial sums of one W norm
+constexpr int kModePool = 4;      // planes kept per k, in units of its frequencies
+constexpr int kModeSort = 16384;  // columns of one sort (128 KB of LDS)
+constexpr double kModeTol = 1.0 / 33554432.0;
+
+// Columns c0 .. c0+cnt-1 of one internal k, sorted together.
+struct SigModeSort {
+  int64_t gsrc;   // weights of the k (elements of wgtim)
+  int64_t cbase;  // first position in the sorted order of all k
+  int c0, cnt, ncp, pad;
+};
+// One group: positions cbase .. cbase+ncp-1 of the sorted order, the first
+// ncol of them columns, the rest padding (perm = -1).
+struct SigMode {
+  int64_t cbase;
+  int64_t gsrc;   // weights of the k
+  int64_t zsrc;   // zmel and czmelwc of the k (elements)
+  int64_t wbase;  // plane pool of the k (16-bit elements)
+  int k, ncol, ncp, pad;
+};
+struct SigModeTile {
+  int grp, ct0, cnt, pad;  // up to 32 consecutive column tiles of one group
+};
+// What the device finds for a group: modes, modes whose planes it forms, first plane in the pool
+struct SigModeRank {
+  int rank, form, poff, raw;
+};
+
+// ---------------------------------------------------------------- order of the columns
+// Bitonic sort in LDS, one block per entry; keys (|weight at the highest
+// frequency| as bits, column), so the order is unique.
+__global__ __launch_bounds__(1024) void mode_sort_kernel(const SigModeSort* __restrict__ so,
+                                                         const double* __restrict__ wgt, int nw1,
+                                                         int* __restrict__ perm) {
+  __shared__ unsigned long long key[kModeSort];
+  const SigModeSort s = so[blockIdx.x];
+  const int t = threadIdx.x;
+  int M = 128;
+  while (M < s.cnt) M *= 2;
+  for (int i = t; i < M; i += 1024) {
+    unsigned long long x = ~0ull;
+    if (i < s.cnt) {
+      const float g = fabsf((float)wgt[s.gsrc + (int64_t)nw1 * (s.c0 + i) + nw1 - 1]);
+      x = ((unsigned long long)__float_as_uint(g) << 32) | (unsigned)i;
+    }
+    key[i] = x;
+  }
+  __syncthreads();
+  for (int k = 2; k <= M; k *= 2)
+    for (int j = k / 2; j > 0; j /= 2) {
+      for (int q = t; q < M / 2; q += 1024) {
+        const int i = 2 * q - (q & (j - 1)), l = i + j;  // bit j of i clear
+        const unsigned long long x = key[i], y = key[l];
+        if ((x > y) == ((i & k) == 0)) {
+          key[i] = y;
+          key[l] = x;
+        }
+      }
+      __syncthreads();
+    }
+  for (int i = t; i < s.ncp; i += 1024)
+    perm[s.cbase + i] = i < s.cnt ? s.c0 + (int)(unsigned)(key[i] & 0xffffffffu) : -1;
+}
+
+// ---------------------------------------------------------------- norms of W
+// part[(k*nw1 + v)*kModeChunks + ch]: sum |W_v(I,J)|^2, I <= J, over every
+// kModeChunks-th column: one pass over the upper triangles, bound by HBM.
+__global__ __launch_bounds__(256) void mode_norm_kernel(const cd* __restrict__ w, int64_t ldw, int64_t w_stride,
+                                                        int n, int nw1, double* __restrict__ part) {
+  __shared__ double red[4];
+  const int kv = blockIdx.y, k = kv / nw1, v = kv % nw1;
+  const cd* W = w + w_stride * k + ldw * n * v;
+  double s = 0.0;
+  for (int J = blockIdx.x; J < n; J += kModeChunks) {
+    const cd* col = W + ldw * J;
+    for (int I = threadIdx.x; I <= J; I += 256) {
+      const cd x = col[I];
+      s += x.re * x.re + x.im * x.im;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) part[(int64_t)kv * kModeChunks + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+}
+
+// ---------------------------------------------------------------- modes of one group
+// One block per group.  X (nw1 x ncp, scratch) holds the residuals of the
+// normalised columns, nrm their norms.  Each step takes the column of largest
+// residual as the next basis vector and removes it from every column; the
+// coefficients are those of the Gram-Schmidt, so the representation holds to
+// the residual whatever rounding does to the basis' orthogonality.
+// gm: mode weights (FP32, mode-major, ncp each); coef: kModeMax x kModeMax
+// per group, coef[r*kModeMax + v] = Q_vr / s_v; rank >= 1.
+// Latency-bound: 8-15 steps, each one pass over X in L2.
+__global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restrict__ grp, const int* __restrict__ perm,
+                                                         const double* __restrict__ wgt,
+                                                         const double* __restrict__ part, int nw1,
+                                                         double* __restrict__ xs, double* __restrict__ nrms,
+                                                         float* __restrict__ gms, float* __restrict__ coef,
+                                                         SigModeRank* __restrict__ rank) {
+  __shared__ double sv[kModeMax], q[kModeMax];
+  __shared__ double bval[8];
+  __shared__ int bcol[8];
+  const SigMode g = grp[blockIdx.x];
+  const int t = threadIdx.x, ncp = g.ncp;
+  const int64_t cbase = g.cbase;
+  double* X = xs + cbase * nw1;
+  double* nrm = nrms + cbase;
+  float* gm = gms + cbase * nw1;
+  float* cf_ = coef + (int64_t)blockIdx.x * kModeMax * kModeMax;
+  if (t < kModeMax) {
+    double s = 0.0;
+    if (t < nw1)
+      for (int c = 0; c < kModeChunks; ++c) s += part[((int64_t)g.k * nw1 + t) * kModeChunks + c];
+    s = sqrt(s);
+    // below FP32's normal range W rounds to zero or nearly so; a W with infinities
+    // or NaN goes unscaled, so that they reach every mode and the result
+    sv[t] = (s < 1e-36) ? 0.0 : (s < 1e300 ? s : 1.0);
+  }
+  for (int e = t; e < kModeMax * kModeMax; e += 512) cf_[e] = 0.f;
+  __syncthreads();
+  double best = 0.0;
+  int bc = 0;
+  for (int c = t; c < ncp; c += 512) {
+    double x[kModeMax], n2 = 0.0;
+    if (c < g.ncol) {
+      const double* src = wgt + g.gsrc + (int64_t)nw1 * perm[cbase + c];
+#pragma unroll
+      for (int v = 0; v < kModeMax; ++v) {
+        x[v] = v < nw1 ? sv[v] * src[v] : 0.0;
+        n2 += x[v] * x[v];
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < kModeMax; ++v) x[v] = 0.0;
+    }
+    const double nr = sqrt(n2), inv = n2 > 0.0 ? 1.0 / nr : 0.0;
+    double r2 = 0.0;
+#pragma unroll
+    for (int v = 0; v < kModeMax; ++v)
+      if (v < nw1) {
+        const double y = x[v] * inv;
+        X[(int64_t)v * ncp + c] = y;
+        r2 += y * y;
+      }
+    nrm[c] = nr;
+    gm[c] = n2 < 1e300 ? 0.f : __builtin_nanf("");  // (stays where no mode is found)
+    if (r2 > best) {
+      best = r2;
+      bc = c;
+    }
+  }
+  int r = 0;
+  for (; r < nw1; ++r) {
+    // column of the largest residual (the lower index on a tie)
+    for (int o = 32; o > 0; o >>= 1) {
+      const double ov = __shfl_xor(best, o);
+      const int oc = __shfl_xor(bc, o);
+      if (ov > best || (ov == best && oc < bc)) {
+        best = ov;
+        bc = oc;
+      }
+    }
+    if ((t & 63) == 0) {
+      bval[t >> 6] = best;
+      bcol[t >> 6] = bc;
+    }
+    __syncthreads();
+    best = bval[0];
+    bc = bcol[0];
+#pragma unroll
+    for (int w = 1; w < 8; ++w)
+      if (bval[w] > best || (bval[w] == best && bcol[w] < bc)) {
+        best = bval[w];
+        bc = bcol[w];
+      }
+    if (!(best > kModeTol * kModeTol)) break;
+    if (t < nw1) {
+      const double x = X[(int64_t)t * ncp + bc] / sqrt(best);
+      q[t] = x;
+      cf_[r * kModeMax + t] = sv[t] > 0.0 ? (float)(x / sv[t]) : 0.f;
+    }
+    __syncthreads();
+    best = 0.0;
+    bc = 0;
+    for (int c = t; c < ncp; c += 512) {
+      double x[kModeMax], d = 0.0, r2 = 0.0;
+#pragma unroll
+      for (int v = 0; v < kModeMax; ++v) {
+        x[v] = 0.0;
+        if (v < nw1) {
+          x[v] = X[(int64_t)v * ncp + c];
+          d += q[v] * x[v];
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < kModeMax; ++v)
+        if (v < nw1) {
+          const double y = x[v] - d * q[v];
+          X[(int64_t)v * ncp + c] = y;
+          r2 += y * y;
+        }
+      gm[(int64_t)r * ncp + c] = (float)(d * nrm[c]);
+      if (r2 > best) {
+        best = r2;
+        bc = c;
+      }
+    }
+  }
+  if (t == 0) rank[blockIdx.x].raw = max(r, 1);  // all weights zero: one mode of weight 0
+}
+
+// Places of the groups' modes in the plane pool of their k (one block per
+// group).  When they do not fit, every group of the k takes the W planes of
+// the frequencies themselves (formed once, by the first group) with the
+// weights as they are: the plain contraction.
+__global__ __launch_bounds__(256) void mode_pack_kernel(const SigMode* __restrict__ grp, const int* __restrict__ kgrp,
+                                                        const int* __restrict__ perm, const double* __restrict__ wgt,
+                                                        int nw1, float* __restrict__ gms, float* __restrict__ coef,
+                                                        SigModeRank* __restrict__ rank) {
+  const SigMode g = grp[blockIdx.x];
+  const int g0 = kgrp[g.k], g1 = kgrp[g.k + 1];
+  int tot = 0, before = 0;
+  for (int i = g0; i < g1; ++i) {
+    if (i == (int)blockIdx.x) before = tot;
+    tot += rank[i].raw;
+  }
+  SigModeRank* r = rank + blockIdx.x;
+  if (tot <= kModePool * nw1) {
+    if (threadIdx.x == 0) {
+      r->rank = r->form = r->raw;
+      r->poff = before;
+    }
+    return;
+  }
+  if (threadIdx.x == 0) {
+    r->rank = nw1;
+    r->form = (int)blockIdx.x == g0 ? nw1 : 0;
+    r->poff = 0;
+  }
+  for (int e = threadIdx.x; e < g.ncp * nw1; e += 256) {
+    const int c = e % g.ncp, v = e / g.ncp;
+    gms[g.cbase * nw1 + e] = c < g.ncol ? (float)wgt[g.gsrc + (int64_t)nw1 * perm[g.cbase + c] + v] : 0.f;
+  }
+  float* cf_ = coef + (int64_t)blockIdx.x * kModeMax * kModeMax;
+  for (int e = threadIdx.x; e < kModeMax * kModeMax; e += 256) cf_[e] = e / kModeMax == e % kModeMax ? 1.f : 0.f;
+}
+
+// ---------------------------------------------------------------- W planes of the modes
+// Per internal k and tile pair (a, b), a <= b, of W's upper triangle: the nw1
+// frequencies of a 32 x 32 tile are read from HBM once and held in registers
+// (FP32), then every mode of every group of the k is formed, split and written
+// as the two output tiles it feeds (row tile a, k slice b) and, through LDS,
+// (row tile b, k slice a), in the layout of split_w6_kernel.  Bound by the
+// writes of the planes (12 bytes per element, mode and triangle half).
+template <int NV>
+__global__ __launch_bounds__(512, 4) void mode_planes_kernel(const cd* __restrict__ w, int64_t ldw, int64_t w_stride,
+                                                             int n, int nw1, int MP, int NS,
+                                                             const SigMode* __restrict__ grp,
+                                                             const int* __restrict__ kgrp,
+                                                             const float* __restrict__ coef,
+                                                             const SigModeRank* __restrict__ rank,
+                                                             unsigned short* __restrict__ as) {
+  __shared__ float2 tr[2][32][33];
+  const int64_t tri = blockIdx.x;
+  int b = (int)((sqrt(8.0 * (double)tri + 1.0) - 1.0) * 0.5);
+  while ((int64_t)(b + 1) * (b + 2) / 2 <= tri) ++b;
+  while ((int64_t)b * (b + 1) / 2 > tri) --b;
+  const int a = (int)(tri - (int64_t)b * (b + 1) / 2);
+  const int k = blockIdx.y;
+  const int I0 = a * 32, J0 = b * 32;
+  // thread: row r of an output tile, k values 2 kp and 2 kp + 1 of its slice
+  const int r = threadIdx.x >> 4, kp = threadIdx.x & 15;
+  const cd* W = w + w_stride * k;
+  float xr[NV][2], xi[NV][2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int I = I0 + r, J = J0 + 2 * kp + e;
+    const bool low = I > J;  // below the diagonal (diagonal tiles only): conj(W(J, I))
+    const int64_t o = low ? J + ldw * I : I + ldw * J;
+    const bool in = I < n && J < n;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const cd x = (in && v < nw1) ? W[o + ldw * n * v] : cd{0.0, 0.0};
+      xr[v][e] = (float)x.re;
+      xi[v][e] = low ? -(float)x.im : (float)x.im;
+    }
+  }
+  const int64_t pst = (int64_t)MP * QBK;
+  const bool put1 = a < MP / 32 && b < NS, put2 = a < b && b < MP / 32 && a < NS;
+  auto put = [&](unsigned short* A, float r0, float i0, float r1, float i1) {
+    const HiLo2 h0 = split2_bf16_alu(r0, r1), h1 = split2_bf16_alu(i0, i1), h2 = split2_bf16_alu(r0 + i0, r1 + i1);
+    unsigned* p = reinterpret_cast<unsigned*>(A);
+    const int64_t ps = pst / 2;
+    p[0] = h0.hi;
+    p[ps] = h0.lo;
+    p[2 * ps] = h1.hi;
+    p[3 * ps] = h1.lo;
+    p[4 * ps] = h2.hi;
+    p[5 * ps] = h2.lo;
+  };
+  // element offsets of this thread's pair in a (row tile, k slice) tile
+  const int ch = kp >> 2, in8 = 2 * (kp & 3);
+  const int64_t o1 = (int64_t)b * Q3PL * pst + (int64_t)(I0 + r) * QBK + 8 * chunk_slot(I0 + r, ch) + in8;
+  const int64_t o2 = (int64_t)a * Q3PL * pst + (int64_t)(J0 + r) * QBK + 8 * chunk_slot(J0 + r, ch) + in8;
+  int it = 0;
+  for (int gi = kgrp[k]; gi < kgrp[k + 1]; ++gi) {
+    const int R = rank[gi].form;
+    unsigned short* A = as + grp[gi].wbase + (int64_t)rank[gi].poff * NS * Q3PL * pst;
+    const float* cg = coef + (int64_t)gi * kModeMax * kModeMax;
+    for (int m = 0; m < R; ++m, ++it) {
+      const float* c = cg + m * kModeMax;
+      float ar[2] = {0.f, 0.f}, ai[2] = {0.f, 0.f};
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const float f = c[v];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          ar[e] = fmaf(f, xr[v][e], ar[e]);
+          ai[e] = fmaf(f, xi[v][e], ai[e]);
+        }
+      }
+      unsigned short* Am = A + (int64_t)m * NS * Q3PL * pst;
+      if (put1) put(Am + o1, ar[0], ai[0], ar[1], ai[1]);
+      if (a < b) {  // uniform: the block's tiles
+        float2(*T)[33] = tr[it & 1];
+        T[r][2 * kp] = float2{ar[0], ai[0]};
+        T[r][2 * kp + 1] = float2{ar[1], ai[1]};
+        __syncthreads();  // the other buffer was last read before this barrier's predecessor
+        const float2 x0 = T[2 * kp][r], x1 = T[2 * kp + 1][r];
+        if (put2) put(Am + o2, x0.x, -x0.y, x1.x, -x1.y);
+      }
+    }
+  }
+}
+
+// zp[p * NP + J] = zmel(J, column perm[p]), zero beyond n and for padding columns
+__global__ __launch_bounds__(256) void mode_pad_kernel(const SigMode* __restrict__ grp, const int* __restrict__ perm,
+                                                       const cf* __restrict__ z, int n, int NP, cf* __restrict__ zp) {
+  const SigMode g = grp[blockIdx.y];
+  for (int p = blockIdx.x; p < g.ncp; p += gridDim.x) {
+    const int c = perm[g.cbase + p];
+    const cf* src = z + g.zsrc + (int64_t)n * max(c, 0);
+    cf* dst = zp + (g.cbase + p) * NP;
+    for (int J = threadIdx.x; J < NP; J += 256) dst[J] = (c >= 0 && J < n) ? src[J] : cf{0.f, 0.f};
+  }
+}
+
+// ---------------------------------------------------------------- contraction
+// 1-D grid, block p on XCD p % 8: XCD x's j-th block belongs to super-tile
+// (j / G)*8 + x, a (run of up to G column tiles of one group, row tile), so
+// the blocks that read the same planes run together on one XCD and share them
+// through its L2.  The runs come in the order of the groups within their k,
+// the nearest columns (the highest ranks) first, so the short blocks end the launch.
+__global__ __launch_bounds__(512, 1) void sig3m_modes_kernel(const SigMode* __restrict__ grp,
+                                                             const SigModeTile* __restrict__ runs, int nrun, int G,
+                                                             const SigModeRank* __restrict__ rank,
+                                                             const int* __restrict__ perm,
+                                                             const unsigned short* __restrict__ as,
+                                                             const cf* __restrict__ zp, const float* __restrict__ gms,
+                                                             int n, int nw1, int MP, int NS, int NP,
+                                                             cf* __restrict__ cz) {
+  __shared__ Sig3Smem s;
+  const int p = blockIdx.x, x = p & 7, j = p >> 3, R = MP / QBM;
+  const int sigma = (j / G) * 8 + x, loc = j % G;
+  if (sigma >= nrun * R) return;
+  const SigModeTile t = runs[sigma / R];
+  if (loc >= t.cnt) return;
+  const SigMode g = grp[t.grp];
+  const int c0 = (t.ct0 + loc) * Q3BN, nwg = __builtin_amdgcn_readfirstlane(rank[t.grp].rank);
+  const int64_t poff = __builtin_amdgcn_readfirstlane(rank[t.grp].poff);
+  const float* gm = gms + g.cbase * nw1 + c0;
+  const int* pm = perm + g.cbase + c0;
+  sig3m_tile<2>(
+      s, as + g.wbase + poff * NS * Q3PL * MP * QBK, zp + g.cbase * NP,
+      [&](int v, int e) { return gm[(int64_t)v * g.ncp + e]; }, [&](int e) { return pm[e]; }, n, 0, nwg, MP, NS, NP,
+      (sigma % R) * QBM, c0, 0, cz + g.zsrc, (int64_t)n);
+}
+
+// ---------------------------------------------------------------- host
+// Column tiles of the groups of one sort of T tiles: sqrt(1.6 T) equal groups,
+// about the least of rank sum x tiles + 1.5 tiles per mode (23 tiles: 6
+// groups, 90 tiles: 12), at most 16.
+static int mode_group_tiles(int T) {
+  const int G = std::max(1, std::min(16, (int)(std::sqrt(1.6 * T) + 0.5)));
+  return (T + G - 1) / G;
+}
+
+// Whether the mode form is taken.  Frequencies: one launch holds kModeMax;
+// fewer than 8 leave too little to save.  Columns: below about 1000 per k the
+// basis and the extra launches cost what the ranks save.
+bool sig_modes_pays(const ecalj_ctx* h, int n, int64_t cols, int nk, int nw1) {
+  return h->tune_mode == 0 && !h->sigc_fp8 && nw1 >= 8 && nw1 <= kModeMax && n >= 128 && cols >= 1000LL * nk;
+}
+
+static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Scratch of one k: plane pool, padded zmel, order, residuals, weights
+size_t sig_modes_bytes(int n, int nm, int ntq, int nw1) {
+  if (nm == 0) return al256((size_t)nw1 * kModeChunks * 8);  // its norms only
+  const int64_t NP = pad_to(n, QBK), ncol = (int64_t)nm * ntq, ncp = (ncol + Q3BN - 1) / Q3BN * Q3BN;
+  const int64_t groups = 16 * (ncol / kModeSort + 1);
+  return al256(kModePool * sig3m_a_elems_per_k(n, nw1) * 2 + (size_t)ncp * (sizeof(cf) * NP + 12 * nw1 + 12) +
+               (kModeMax * kModeMax * 4 + sizeof(SigModeRank)) * groups + (size_t)nw1 * kModeChunks * 8 + 4096);
+}
+
+// czmelwc of nk internal k-points (zmel, wgt, cz packed per k: n x nm[k] x ntq
+// and nw1 x nm[k] x ntq); scratch: the sum of sig_modes_bytes.
+ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* zmel, int n, int nw1, const cd* wc,
+                       int64_t ldw, int64_t w_stride, const double* wgt, cf* cz, unsigned char* scratch) {
+  const int MP = pad_to(n, QBM), NP = pad_to(n, QBK), NS = NP / QBK, R = MP / QBM;
+  const int64_t pool = kModePool * (int64_t)sig3m_a_elems_per_k(n, nw1);
+  std::vector<SigModeSort> sorts;
+  std::vector<SigMode> grp;
+  std::vector<int> kgrp(nk + 1, 0);
+  int64_t cols = 0, co = 0, pools = 0;
+  int maxg = 0;
+  for (int k = 0; k < nk; ++k) {
+    const int64_t N = (int64_t)nm[k] * ntq;
+    if (N > 0x7fffffff / 2) return ECALJ_ERR_DIM;
+    const int T = (int)((N + Q3BN - 1) / Q3BN), per = kModeSort / Q3BN, parts = (T + per - 1) / per;
+    const int tp = parts ? (T + parts - 1) / parts : 0;  // column tiles of one sort
+    for (int t0 = 0; t0 < T; t0 += tp) {
+      const int tn = std::min(tp, T - t0), cnt = (int)std::min<int64_t>(N - (int64_t)t0 * Q3BN, (int64_t)tn * Q3BN);
+      sorts.push_back({co * nw1, cols, t0 * Q3BN, cnt, tn * Q3BN, 0});
+      const int gt = mode_group_tiles(tn);
+      for (int g0 = 0; g0 < tn; g0 += gt) {
+        const int gn = std::min(gt, tn - g0);
+        grp.push_back({cols + g0 * Q3BN, co * nw1, co * n, pools, k, std::min(gn * Q3BN, cnt - g0 * Q3BN),
+                       gn * Q3BN, 0});
+      }
+      cols += (int64_t)tn * Q3BN;
+    }
+    co += N;
+    if (N > 0) pools += pool;
+    kgrp[k + 1] = (int)grp.size();
+    maxg = std::max(maxg, kgrp[k + 1] - kgrp[k]);
+  }
+  const int ng = (int)grp.size();
+  if (ng == 0) return ECALJ_OK;
+  // runs of column tiles, group index within the k outermost
+  std::vector<SigModeTile> runs;
+  int G = 1, ncpmax = 0;
+  for (int gi = 0; gi < maxg; ++gi)
+    for (int k = 0; k < nk; ++k) {
+      if (kgrp[k] + gi >= kgrp[k + 1]) continue;
+      const SigMode& m = grp[kgrp[k] + gi];
+      const int ct = m.ncp / Q3BN, parts = (ct + 31) / 32, per = (ct + parts - 1) / parts;
+      for (int c = 0; c < ct; c += per) runs.push_back({kgrp[k] + gi, c, std::min(per, ct - c), 0});
+      G = std::max(G, per);
+      ncpmax = std::max(ncpmax, m.ncp);
+    }
+  const int64_t T = std::max(MP / 32, NS), npair = T * (T + 1) / 2;
+  const int64_t blocks = 8LL * G * (((int64_t)runs.size() * R + 7) / 8);
+  if (blocks > 0x7fffffff || npair > 0x7fffffff || nk > 65535 || (int64_t)nw1 * nk > 65535 || ng > 65535)
+    return ECALJ_ERR_DIM;
+  unsigned char* q = scratch;
+  auto take = [&](size_t bytes) {
+    unsigned char* r = q;
+    q += al256(bytes);
+    return r;
+  };
+  unsigned short* as = (unsigned short*)take((size_t)pools * 2);
+  cf* zp = (cf*)take(sizeof(cf) * (size_t)cols * NP);
+  double* xs = (double*)take(sizeof(double) * (size_t)cols * nw1);
+  double* nrm = (double*)take(sizeof(double) * (size_t)cols);
+  float* gm = (float*)take(sizeof(float) * (size_t)cols * nw1);
+  int* perm = (int*)take(sizeof(int) * (size_t)cols);
+  float* coef = (float*)take(sizeof(float) * kModeMax * kModeMax * (size_t)ng);
+  double* part = (double*)take(sizeof(double) * kModeChunks * (size_t)nw1 * nk);
+  SigModeRank* rank = (SigModeRank*)take(sizeof(SigModeRank) * (size_t)ng);
+  // tables
+  const size_t b0 = sizeof(SigModeSort) * sorts.size(), b1 = sizeof(SigMode) * grp.size();
+  const size_t b2 = sizeof(SigModeTile) * runs.size(), b3 = sizeof(int) * kgrp.size();
+  std::vector<unsigned char> blob(b0 + b1 + b2 + b3);
+  std::memcpy(blob.data(), sorts.data(), b0);
+  std::memcpy(blob.data() + b0, grp.data(), b1);
+  std::memcpy(blob.data() + b0 + b1, runs.data(), b2);
+  std::memcpy(blob.data() + b0 + b1 + b2, kgrp.data(), b3);
+  unsigned char* d;
+  ECALJ_TRY(upload_blob(h, ecalj_ctx::S_GTAB, blob, &d));
+  const SigModeSort* ds = (const SigModeSort*)d;
+  const SigMode* dg = (const SigMode*)(d + b0);
+  const SigModeTile* dr = (const SigModeTile*)(d + b0 + b1);
+  const int* dk = (const int*)(d + b0 + b1 + b2);
+
+  hipLaunchKernelGGL(mode_sort_kernel, dim3((unsigned)sorts.size()), dim3(1024), 0, h->stream, ds, wgt, nw1, perm);
+  ECALJ_HIP(hipGetLastError());
+  hipLaunchKernelGGL(mode_norm_kernel, dim3(kModeChunks, nw1 * nk), dim3(256), 0, h->stream, wc, ldw, w_stride, n, nw1,
+                     part);
+  ECALJ_HIP(hipGetLastError());
+  hipLaunchKernelGGL(mode_basis_kernel, dim3(ng), dim3(512), 0, h->stream, dg, perm, wgt, part, nw1, xs, nrm, gm, coef,
+                     rank);
+  ECALJ_HIP(hipGetLastError());
+  hipLaunchKernelGGL(mode_pack_kernel, dim3(ng), dim3(256), 0, h->stream, dg, dk, perm, wgt, nw1, gm, coef, rank);
+  ECALJ_HIP(hipGetLastError());
+  auto planes = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)npair, nk), dim3(512), 0, h->stream, wc, ldw, w_stride, n, nw1, MP, NS, dg,
+                       dk, coef, rank, as);
+  };
+  if (nw1 <= 12) planes(mode_planes_kernel<12>);
+  else if (nw1 <= 18) planes(mode_planes_kernel<18>);
+  else planes(mode_planes_kernel<24>);
+  ECALJ_HIP(hipGetLastError());
+  hipLaunchKernelGGL(mode_pad_kernel, dim3(std::min(ncpmax, 4096), ng), dim3(256), 0, h->stream, dg, perm, zmel, n, NP,
+                     zp);
+  ECALJ_HIP(hipGetLastError());
+  int tev = -1;
+  ECALJ_TRY(timing_begin(h, 0, &tev));
+  hipLaunchKernelGGL(sig3m_modes_kernel, dim3((unsigned)blocks), dim3(512), 0, h->stream, dg, dr, (int)runs.size(), G,
+                     rank, perm, as, zp, gm, n, nw1, MP, NS, NP, cz);
+  ECALJ_HIP(hipGetLastError());
+  ECALJ_TRY(timing_end(h, 0, tev));
+  return ECALJ_OK;
+}
+
+}  // namespace ecalj

@@ -1,0 +1,180 @@
+"""Sigma_c in frequency modes (sigmodes.hip), the bf16x3 form of calls with
+1000 and more columns per internal k and 8 to 24 frequencies, against the FP64
+oracle and the plain three-product contraction (a forced tuner variant)."""
+import numpy as np
+import pytest
+
+from ecalj_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+# Every product of the bf16x3 form errs by at most ~2^-16 of its factors (the
+# dropped lo*lo term and the two lo roundings) and the sums average it; the
+# mode form adds 2^-25 of a column's weights.  2e-5 is that bound with no averaging.
+TOL = 2e-5
+
+
+@pytest.fixture(scope="module")
+def orc():
+    import oracle
+
+    oracle.build()
+    return oracle
+
+
+def crand(rng, *sh):
+    return np.asfortranarray(rng.standard_normal(sh) + 1j * rng.standard_normal(sh))
+
+
+def relerr(a, b):
+    return np.abs(a - b).max() / np.abs(b).max()
+
+
+def physical_weights(orc, rng, nm, ntq, nf):
+    t, w = np.polynomial.legendre.leggauss(nf)
+    x, wx = 0.5 * (t + 1.0), 0.5 * w
+    om = (1.0 - x) / x
+    no = max(1, nm // 10)
+    ek = np.concatenate([np.sort(rng.uniform(-12, 0, no)), np.sort(rng.uniform(0.5, 60, nm - no))]) / synth.RYDBERG_EV
+    eq = np.sort(rng.uniform(-11, 12, ntq)) / synth.RYDBERG_EV
+    return orc.wgtim(eq, ek, 0.003, 0.25, x, wx, np.exp(-om ** 2))
+
+
+def case(orc, seed, ngb, nm, ntq, nf, weights):
+    rng = np.random.default_rng(seed)
+    z = crand(rng, ngb, nm, ntq)
+    w = crand(rng, ngb, ngb, nf + 1) / (1.0 + np.arange(nf + 1)) ** 2  # used through the upper triangle
+    if weights == "physical":
+        g = physical_weights(orc, rng, nm, ntq, nf)
+    elif weights == "random":  # every frequency needed: the plane pool overflows, plain contraction
+        g = rng.standard_normal((nf + 1, nm, ntq))
+    elif weights == "rank1":
+        g = rng.standard_normal((nf + 1, 1, 1)) * rng.standard_normal((1, nm, ntq))
+    else:
+        g = np.zeros((nf + 1, nm, ntq))
+        g[:, nm // 2, 0] = 1.0
+    return z, np.asfortranarray(w), np.asfortranarray(g)
+
+
+# rows: tile remainders and a full tile; columns: a whole number of tiles, one
+# more, one group and several; frequencies: both ends and the plane kernel's edges
+@pytest.mark.parametrize("weights", ["physical", "random", "rank1", "one_column"])
+@pytest.mark.parametrize("ngb,nm,ntq,nf", [(128, 128, 8, 7), (161, 129, 9, 11), (130, 67, 16, 12), (200, 113, 10, 17),
+                                           (257, 150, 7, 18), (131, 80, 33, 23)])
+def test_modes_against_oracle(orc, weights, ngb, nm, ntq, nf):
+    import ecalj_amd
+
+    z, w, g = case(orc, ngb + nf, ngb, nm, ntq, nf, weights)
+    ref = orc.sigc_imag(z, w, g)
+    h = ecalj_amd.Handle(0, "bf16x3")
+    try:
+        got = h.sigc(z, w, g)
+        again = h.sigc(z, w, g)
+        h.set_tuning(6)
+        plain = h.sigc(z, w, g)
+    finally:
+        h.close()
+    print(weights, ngb, nm, ntq, nf, relerr(got, ref), relerr(plain, ref), flush=True)
+    assert relerr(got, ref) < TOL
+    assert np.array_equal(got, again)
+    # against the plain form: both roundings, averaged over the columns
+    assert relerr(got, plain) < TOL
+
+
+@pytest.mark.parametrize("nms", [[140, 0, 70, 211], [200]])
+def test_modes_grouped(orc, nms):
+    import ecalj_amd
+
+    ngb, ntq, nf = 150, 11, 14
+    zs, ws, gs = zip(*[case(orc, 7 + k, ngb, max(nm, 1), ntq, nf, "physical") for k, nm in enumerate(nms)])
+    ref = np.zeros((ntq, ntq), complex, order="F")
+    for nm, z, w, g in zip(nms, zs, ws, gs):
+        if nm:
+            ref = orc.sigc_imag(z, w, g, ref)
+    h = ecalj_amd.Handle(0, "bf16x3")
+    try:
+        cat = lambda xs: np.concatenate([x.ravel(order="F") for nm, x in zip(nms, xs) if nm])
+        dz, dg = h.to_dev(cat(zs).astype(np.complex64)), h.to_dev(cat(gs))
+        dw = h.to_dev(np.concatenate([w.ravel(order="F") for w in ws]))
+        s = h.array((ntq, ntq))
+        s.zero()
+        h.sigc_grouped_dev(nms, dz, ngb, ntq, nf, dw, dg, s)
+        got = s.download()
+    finally:
+        h.close()
+    print(nms, relerr(got, ref), flush=True)
+    assert relerr(got, ref) < TOL
+
+
+def test_modes_more_columns_than_one_sort(orc):
+    """17 000 columns: two sorts per k; the oracle's contraction is linear in
+    the columns of one middle state, so a few states are compared."""
+    import ecalj_amd
+
+    ngb, nm, ntq, nf = 128, 1000, 17, 8
+    z, w, g = case(orc, 3, ngb, nm, ntq, nf, "physical")
+    keep = np.zeros(nm, bool)
+    keep[[0, 3, 499, 963, 964, 999]] = True
+    g[:, ~keep, :] = 0.0
+    ref = orc.sigc_imag(np.asfortranarray(z[:, keep]), w, np.asfortranarray(g[:, keep]))
+    h = ecalj_amd.Handle(0, "bf16x3")
+    try:
+        got = h.sigc(z, w, g)
+    finally:
+        h.close()
+    print(relerr(got, ref), flush=True)
+    assert relerr(got, ref) < TOL
+
+
+def test_modes_non_finite_inputs_reach_the_result(orc):
+    import ecalj_amd
+
+    z, w, g = case(orc, 5, 130, 130, 8, 9, "physical")
+    h = ecalj_amd.Handle(0, "bf16x3")
+    try:
+        for bad in (np.inf, np.nan):
+            w2 = w.copy(order="F")
+            w2[3, 70, 4] = bad
+            assert not np.isfinite(h.sigc(z, w2, g)).any()
+            g2 = g.copy(order="F")
+            g2[2, 11, 5] = bad
+            s = h.sigc(z, w, g2)
+            assert not np.isfinite(s[5]).any() and np.isfinite(np.delete(s, 5, axis=0)).all()
+        assert np.array_equal(h.sigc(z, w, np.zeros_like(g)), np.zeros((8, 8)))
+    finally:
+        h.close()
+
+
+def test_modes_graph_replay_follows_its_inputs(orc):
+    """The ranks are found on the device: a captured call replays with those of
+    the weights it meets, also when they need more modes than at capture."""
+    import ecalj_amd
+
+    ngb, nm, ntq, nf = 130, 130, 9, 12
+    z, w, g1 = case(orc, 21, ngb, nm, ntq, nf, "rank1")
+    h = ecalj_amd.Handle(0, "bf16x3")
+    try:
+        dz, dw, dg, s = h.to_dev(z.astype(np.complex64)), h.to_dev(w), h.to_dev(g1), h.array((ntq, ntq))
+
+        def call():
+            s.zero()
+            h.sigc_dev(1, dz, ngb, nm, ntq, nf, dw, dg, s)
+
+        call()
+        h.graph_begin()
+        try:
+            call()
+        finally:
+            gr = h.graph_end()
+        for weights in ("rank1", "physical", "random", "rank1"):
+            g = case(orc, 21, ngb, nm, ntq, nf, weights)[2]
+            dg.upload(g)
+            call()
+            eager = s.download()
+            gr.launch()
+            h.sync()
+            assert np.array_equal(s.download(), eager)
+            assert relerr(eager, orc.sigc_imag(z, w, g)) < TOL
+        gr.close()
+    finally:
+        h.close()
