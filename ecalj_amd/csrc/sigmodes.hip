@@ -60,9 +60,9 @@ struct SigMode {
 struct SigModeTile {
   int grp, ct0, cnt, pad;  // up to 32 consecutive column tiles of one group
 };
-// What the device finds for a group: modes, modes whose planes it forms, first plane in the pool
+// What the device finds for a group: its modes, the first of them in the pool, the basis' size
 struct SigModeRank {
-  int rank, form, poff, raw;
+  int rank, poff, raw, pad;
 };
 
 // ---------------------------------------------------------------- order of the columns
@@ -251,13 +251,14 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
 }
 
 // Places of the groups' modes in the plane pool of their k (one block per
-// group).  When they do not fit, every group of the k takes the W planes of
-// the frequencies themselves (formed once, by the first group) with the
-// weights as they are: the plain contraction.
+// group): coefp[(k kModePool nw1 + p) kModeMax + v] for plane p, nplane[k]
+// planes.  When they do not fit, every group of the k takes the W planes of
+// the frequencies themselves with the weights as they are: the plain contraction.
 __global__ __launch_bounds__(256) void mode_pack_kernel(const SigMode* __restrict__ grp, const int* __restrict__ kgrp,
                                                         const int* __restrict__ perm, const double* __restrict__ wgt,
-                                                        int nw1, float* __restrict__ gms, float* __restrict__ coef,
-                                                        SigModeRank* __restrict__ rank) {
+                                                        int nw1, float* __restrict__ gms,
+                                                        const float* __restrict__ coef, float* __restrict__ coefp,
+                                                        int* __restrict__ nplane, SigModeRank* __restrict__ rank) {
   const SigMode g = grp[blockIdx.x];
   const int g0 = kgrp[g.k], g1 = kgrp[g.k + 1];
   int tot = 0, before = 0;
@@ -265,51 +266,52 @@ __global__ __launch_bounds__(256) void mode_pack_kernel(const SigMode* __restric
     if (i == (int)blockIdx.x) before = tot;
     tot += rank[i].raw;
   }
+  const bool fits = tot <= kModePool * nw1;
   SigModeRank* r = rank + blockIdx.x;
-  if (tot <= kModePool * nw1) {
-    if (threadIdx.x == 0) {
-      r->rank = r->form = r->raw;
-      r->poff = before;
-    }
-    return;
-  }
+  const int R = fits ? r->raw : nw1;
+  float* cp = coefp + ((int64_t)g.k * kModePool * nw1 + (fits ? before : 0)) * kModeMax;
   if (threadIdx.x == 0) {
-    r->rank = nw1;
-    r->form = (int)blockIdx.x == g0 ? nw1 : 0;
-    r->poff = 0;
+    r->rank = R;
+    r->poff = fits ? before : 0;
+    if ((int)blockIdx.x == g0) nplane[g.k] = fits ? tot : nw1;
   }
-  for (int e = threadIdx.x; e < g.ncp * nw1; e += 256) {
-    const int c = e % g.ncp, v = e / g.ncp;
-    gms[g.cbase * nw1 + e] = c < g.ncol ? (float)wgt[g.gsrc + (int64_t)nw1 * perm[g.cbase + c] + v] : 0.f;
-  }
-  float* cf_ = coef + (int64_t)blockIdx.x * kModeMax * kModeMax;
-  for (int e = threadIdx.x; e < kModeMax * kModeMax; e += 256) cf_[e] = e / kModeMax == e % kModeMax ? 1.f : 0.f;
+  if (fits || (int)blockIdx.x == g0)
+    for (int e = threadIdx.x; e < R * kModeMax; e += 256)
+      cp[e] = fits ? coef[(int64_t)blockIdx.x * kModeMax * kModeMax + e] : (e / kModeMax == e % kModeMax ? 1.f : 0.f);
+  if (!fits)
+    for (int e = threadIdx.x; e < g.ncp * nw1; e += 256) {
+      const int c = e % g.ncp, v = e / g.ncp;
+      gms[g.cbase * nw1 + e] = c < g.ncol ? (float)wgt[g.gsrc + (int64_t)nw1 * perm[g.cbase + c] + v] : 0.f;
+    }
 }
 
 // ---------------------------------------------------------------- W planes of the modes
 // Per internal k and tile pair (a, b), a <= b, of W's upper triangle: the nw1
 // frequencies of a 32 x 32 tile are read from HBM once and held in registers
-// (FP32), then every mode of every group of the k is formed, split and written
-// as the two output tiles it feeds (row tile a, k slice b) and, through LDS,
-// (row tile b, k slice a), in the layout of split_w6_kernel.  Bound by the
-// writes of the planes (12 bytes per element, mode and triangle half).
+// (FP32), then every mode of the k is formed and, through LDS, split and
+// written as the two output tiles it feeds, (row tile a, k slice b) and (row
+// tile b, k slice a), in the layout of split_w6_kernel.  Two modes per
+// barrier: 512 threads are then 2 modes x 2 tiles x 32 rows x 4 chunks, one
+// 16-byte store per plane each.  Rows beyond the last tile of n are not
+// written: they only reach output rows that do not exist.  Bound by the writes
+// of the planes (12 bytes per element and mode).
 template <int NV>
 __global__ __launch_bounds__(512, 4) void mode_planes_kernel(const cd* __restrict__ w, int64_t ldw, int64_t w_stride,
-                                                             int n, int nw1, int MP, int NS,
-                                                             const SigMode* __restrict__ grp,
-                                                             const int* __restrict__ kgrp,
-                                                             const float* __restrict__ coef,
-                                                             const SigModeRank* __restrict__ rank,
+                                                             int n, int nw1, int MP, int NS, int64_t pool,
+                                                             const int* __restrict__ kpool,
+                                                             const float* __restrict__ coefp,
+                                                             const int* __restrict__ nplane,
                                                              unsigned short* __restrict__ as) {
-  __shared__ float2 tr[2][32][33];
+  __shared__ __align__(16) float2 tr[2][2][32][34];
   const int64_t tri = blockIdx.x;
   int b = (int)((sqrt(8.0 * (double)tri + 1.0) - 1.0) * 0.5);
   while ((int64_t)(b + 1) * (b + 2) / 2 <= tri) ++b;
   while ((int64_t)b * (b + 1) / 2 > tri) --b;
   const int a = (int)(tri - (int64_t)b * (b + 1) / 2);
   const int k = blockIdx.y;
+  if (kpool[k] < 0) return;  // no columns
   const int I0 = a * 32, J0 = b * 32;
-  // thread: row r of an output tile, k values 2 kp and 2 kp + 1 of its slice
+  // thread: row r of the tile, k values 2 kp and 2 kp + 1 of its slice
   const int r = threadIdx.x >> 4, kp = threadIdx.x & 15;
   const cd* W = w + w_stride * k;
   float xr[NV][2], xi[NV][2];
@@ -326,30 +328,20 @@ __global__ __launch_bounds__(512, 4) void mode_planes_kernel(const cd* __restric
       xi[v][e] = low ? -(float)x.im : (float)x.im;
     }
   }
-  const int64_t pst = (int64_t)MP * QBK;
-  const bool put1 = a < MP / 32 && b < NS, put2 = a < b && b < MP / 32 && a < NS;
-  auto put = [&](unsigned short* A, float r0, float i0, float r1, float i1) {
-    const HiLo2 h0 = split2_bf16_alu(r0, r1), h1 = split2_bf16_alu(i0, i1), h2 = split2_bf16_alu(r0 + i0, r1 + i1);
-    unsigned* p = reinterpret_cast<unsigned*>(A);
-    const int64_t ps = pst / 2;
-    p[0] = h0.hi;
-    p[ps] = h0.lo;
-    p[2 * ps] = h1.hi;
-    p[3 * ps] = h1.lo;
-    p[4 * ps] = h2.hi;
-    p[5 * ps] = h2.lo;
-  };
-  // element offsets of this thread's pair in a (row tile, k slice) tile
-  const int ch = kp >> 2, in8 = 2 * (kp & 3);
-  const int64_t o1 = (int64_t)b * Q3PL * pst + (int64_t)(I0 + r) * QBK + 8 * chunk_slot(I0 + r, ch) + in8;
-  const int64_t o2 = (int64_t)a * Q3PL * pst + (int64_t)(J0 + r) * QBK + 8 * chunk_slot(J0 + r, ch) + in8;
-  int it = 0;
-  for (int gi = kgrp[k]; gi < kgrp[k + 1]; ++gi) {
-    const int R = rank[gi].form;
-    unsigned short* A = as + grp[gi].wbase + (int64_t)rank[gi].poff * NS * Q3PL * pst;
-    const float* cg = coef + (int64_t)gi * kModeMax * kModeMax;
-    for (int m = 0; m < R; ++m, ++it) {
-      const float* c = cg + m * kModeMax;
+  // writing: mode wm of the pair, tile wo (0: row tile a, 1: row tile b), row wr, chunk wc
+  const int wc = threadIdx.x & 3, wr = (threadIdx.x >> 2) & 31, wo = (threadIdx.x >> 7) & 1, wm = threadIdx.x >> 8;
+  const int64_t pst = (int64_t)MP * QBK, plane = (int64_t)NS * Q3PL * pst;
+  const int row = (wo ? J0 : I0) + wr;
+  unsigned short* A = as + pool * kpool[k] + (int64_t)(wo ? a : b) * Q3PL * pst + (int64_t)row * QBK +
+                      8 * chunk_slot(row, wc);
+  const bool put = wo == 0 || a < b;
+  const int P = nplane[k];
+  const float* c0 = coefp + (int64_t)k * kModePool * nw1 * kModeMax;
+  for (int p = 0; p < P; p += 2) {
+    float2(*T)[32][34] = tr[(p >> 1) & 1];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const float* c = c0 + min(p + m, P - 1) * kModeMax;
       float ar[2] = {0.f, 0.f}, ai[2] = {0.f, 0.f};
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
@@ -360,16 +352,32 @@ __global__ __launch_bounds__(512, 4) void mode_planes_kernel(const cd* __restric
           ai[e] = fmaf(f, xi[v][e], ai[e]);
         }
       }
-      unsigned short* Am = A + (int64_t)m * NS * Q3PL * pst;
-      if (put1) put(Am + o1, ar[0], ai[0], ar[1], ai[1]);
-      if (a < b) {  // uniform: the block's tiles
-        float2(*T)[33] = tr[it & 1];
-        T[r][2 * kp] = float2{ar[0], ai[0]};
-        T[r][2 * kp + 1] = float2{ar[1], ai[1]};
-        __syncthreads();  // the other buffer was last read before this barrier's predecessor
-        const float2 x0 = T[2 * kp][r], x1 = T[2 * kp + 1][r];
-        if (put2) put(Am + o2, x0.x, -x0.y, x1.x, -x1.y);
+      *reinterpret_cast<f4*>(&T[m][r][2 * kp]) = f4{ar[0], ai[0], ar[1], ai[1]};
+    }
+    __syncthreads();  // the other buffer was last read before the previous barrier
+    if (put && p + wm < P) {
+      u4q h[Q3PL];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f4 x;
+        if (wo) {
+          const float2 u = T[wm][8 * wc + 2 * q][wr], v = T[wm][8 * wc + 2 * q + 1][wr];
+          x = f4{u.x, -u.y, v.x, -v.y};
+        } else {
+          x = *reinterpret_cast<const f4*>(&T[wm][wr][8 * wc + 2 * q]);
+        }
+        const HiLo2 s0 = split2_bf16_alu(x[0], x[2]), s1 = split2_bf16_alu(x[1], x[3]),
+                    s2 = split2_bf16_alu(x[0] + x[1], x[2] + x[3]);
+        h[0][q] = s0.hi;
+        h[1][q] = s0.lo;
+        h[2][q] = s1.hi;
+        h[3][q] = s1.lo;
+        h[4][q] = s2.hi;
+        h[5][q] = s2.lo;
       }
+      unsigned short* d = A + (p + wm) * plane;
+#pragma unroll
+      for (int q = 0; q < Q3PL; ++q) *reinterpret_cast<u4q*>(d + q * pst) = h[q];
     }
   }
 }
@@ -437,11 +445,13 @@ static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Scratch of one k: plane pool, padded zmel, order, residuals, weights
 size_t sig_modes_bytes(int n, int nm, int ntq, int nw1) {
-  if (nm == 0) return al256((size_t)nw1 * kModeChunks * 8);  // its norms only
+  // norms, coefficients and counts of a k, also of one without columns
+  const size_t per_k = (size_t)nw1 * (kModeChunks * 8 + kModePool * kModeMax * 4) + 4;
+  if (nm == 0) return al256(per_k);
   const int64_t NP = pad_to(n, QBK), ncol = (int64_t)nm * ntq, ncp = (ncol + Q3BN - 1) / Q3BN * Q3BN;
   const int64_t groups = 16 * (ncol / kModeSort + 1);
   return al256(kModePool * sig3m_a_elems_per_k(n, nw1) * 2 + (size_t)ncp * (sizeof(cf) * NP + 12 * nw1 + 12) +
-               (kModeMax * kModeMax * 4 + sizeof(SigModeRank)) * groups + (size_t)nw1 * kModeChunks * 8 + 4096);
+               (kModeMax * kModeMax * 4 + sizeof(SigModeRank)) * groups + per_k + 4096);
 }
 
 // czmelwc of nk internal k-points (zmel, wgt, cz packed per k: n x nm[k] x ntq
@@ -452,8 +462,9 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
   const int64_t pool = kModePool * (int64_t)sig3m_a_elems_per_k(n, nw1);
   std::vector<SigModeSort> sorts;
   std::vector<SigMode> grp;
-  std::vector<int> kgrp(nk + 1, 0);
-  int64_t cols = 0, co = 0, pools = 0;
+  std::vector<int> kgrp(2 * nk + 1, 0);  // first group of each k, then its pool (-1: no columns)
+  int64_t cols = 0, co = 0;
+  int pools = 0;
   int maxg = 0;
   for (int k = 0; k < nk; ++k) {
     const int64_t N = (int64_t)nm[k] * ntq;
@@ -466,13 +477,13 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
       const int gt = mode_group_tiles(tn);
       for (int g0 = 0; g0 < tn; g0 += gt) {
         const int gn = std::min(gt, tn - g0);
-        grp.push_back({cols + g0 * Q3BN, co * nw1, co * n, pools, k, std::min(gn * Q3BN, cnt - g0 * Q3BN),
+        grp.push_back({cols + g0 * Q3BN, co * nw1, co * n, pools * pool, k, std::min(gn * Q3BN, cnt - g0 * Q3BN),
                        gn * Q3BN, 0});
       }
       cols += (int64_t)tn * Q3BN;
     }
     co += N;
-    if (N > 0) pools += pool;
+    kgrp[nk + 1 + k] = N > 0 ? pools++ : -1;
     kgrp[k + 1] = (int)grp.size();
     maxg = std::max(maxg, kgrp[k + 1] - kgrp[k]);
   }
@@ -490,7 +501,7 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
       G = std::max(G, per);
       ncpmax = std::max(ncpmax, m.ncp);
     }
-  const int64_t T = std::max(MP / 32, NS), npair = T * (T + 1) / 2;
+  const int64_t npair = (int64_t)NS * (NS + 1) / 2;
   const int64_t blocks = 8LL * G * (((int64_t)runs.size() * R + 7) / 8);
   if (blocks > 0x7fffffff || npair > 0x7fffffff || nk > 65535 || (int64_t)nw1 * nk > 65535 || ng > 65535)
     return ECALJ_ERR_DIM;
@@ -500,7 +511,7 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
     q += al256(bytes);
     return r;
   };
-  unsigned short* as = (unsigned short*)take((size_t)pools * 2);
+  unsigned short* as = (unsigned short*)take((size_t)(pool * pools) * 2);
   cf* zp = (cf*)take(sizeof(cf) * (size_t)cols * NP);
   double* xs = (double*)take(sizeof(double) * (size_t)cols * nw1);
   double* nrm = (double*)take(sizeof(double) * (size_t)cols);
@@ -509,6 +520,8 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
   float* coef = (float*)take(sizeof(float) * kModeMax * kModeMax * (size_t)ng);
   double* part = (double*)take(sizeof(double) * kModeChunks * (size_t)nw1 * nk);
   SigModeRank* rank = (SigModeRank*)take(sizeof(SigModeRank) * (size_t)ng);
+  float* coefp = (float*)take(sizeof(float) * kModeMax * kModePool * (size_t)nw1 * nk);
+  int* nplane = (int*)take(sizeof(int) * (size_t)nk);
   // tables
   const size_t b0 = sizeof(SigModeSort) * sorts.size(), b1 = sizeof(SigMode) * grp.size();
   const size_t b2 = sizeof(SigModeTile) * runs.size(), b3 = sizeof(int) * kgrp.size();
@@ -532,14 +545,16 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
   hipLaunchKernelGGL(mode_basis_kernel, dim3(ng), dim3(512), 0, h->stream, dg, perm, wgt, part, nw1, xs, nrm, gm, coef,
                      rank);
   ECALJ_HIP(hipGetLastError());
-  hipLaunchKernelGGL(mode_pack_kernel, dim3(ng), dim3(256), 0, h->stream, dg, dk, perm, wgt, nw1, gm, coef, rank);
+  hipLaunchKernelGGL(mode_pack_kernel, dim3(ng), dim3(256), 0, h->stream, dg, dk, perm, wgt, nw1, gm, coef,
+                     coefp, nplane, rank);
   ECALJ_HIP(hipGetLastError());
   auto planes = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)npair, nk), dim3(512), 0, h->stream, wc, ldw, w_stride, n, nw1, MP, NS, dg,
-                       dk, coef, rank, as);
+    hipLaunchKernelGGL(kern, dim3((unsigned)npair, nk), dim3(512), 0, h->stream, wc, ldw, w_stride, n, nw1, MP, NS,
+                       pool, dk + nk + 1, coefp, nplane, as);
   };
-  if (nw1 <= 12) planes(mode_planes_kernel<12>);
-  else if (nw1 <= 18) planes(mode_planes_kernel<18>);
+  if (nw1 <= 13) planes(mode_planes_kernel<13>);
+  else if (nw1 <= 17) planes(mode_planes_kernel<17>);
+  else if (nw1 <= 21) planes(mode_planes_kernel<21>);
   else planes(mode_planes_kernel<24>);
   ECALJ_HIP(hipGetLastError());
   hipLaunchKernelGGL(mode_pad_kernel, dim3(std::min(ncpmax, 4096), ng), dim3(256), 0, h->stream, dg, perm, zmel, n, NP,
