@@ -1208,8 +1208,8 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   T *wh, *cz, *part;
   // W unpacked (or, for bf16x3, split into bf16 planes) per internal k;
   // processed in groups to bound scratch memory
-  const bool modes = MODE == MBF3 && sig_modes_pays(h, n, (int64_t)ncol * nbatch, nbatch, nw1);
-  const size_t wh_bytes_per = modes ? sig_modes_bytes(n, nm, ntq, nw1)
+  const bool modes = sig_modes_pays(h, MODE, n, (int64_t)ncol * nbatch, nw1);
+  const size_t wh_bytes_per = modes ? sig_modes_bytes(MODE, n, nm, ntq, nw1)
                               : (MODE == MBF3) ? sig_bf3_bytes_per_k(n, ncol, nw1) : sizeof(T) * nn * nw1;
   const size_t cz_bytes_per = sizeof(T) * (size_t)n * ncol;
   const size_t cap = modes ? kSigModeScratch : kSigScratch;
@@ -1231,9 +1231,9 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   const int ublocks = (int)std::min<int64_t>((tot + 255) / 256, 65536);
   for (int b0 = 0; b0 < nbatch; b0 += group) {
     const int gb = std::min(group, nbatch - b0);
-    if (MODE == MBF3 && modes) {
-      ECALJ_TRY(sig_modes(h, gb, nms.data(), ntq, (const cf*)zmel + (int64_t)n * ncol * b0, n, nw1, wc + wstride * b0,
-                          ldw, wstride, wgt + (int64_t)nw1 * ncol * b0, (cf*)cz, (unsigned char*)wh));
+    if (modes) {
+      ECALJ_TRY(sig_modes(h, MODE, gb, nms.data(), ntq, zmel + (int64_t)n * ncol * b0, n, nw1, wc + wstride * b0, ldw,
+                          wstride, wgt + (int64_t)nw1 * ncol * b0, cz, (unsigned char*)wh));
     } else if constexpr (MODE == MBF3) {
       unsigned short* as = reinterpret_cast<unsigned short*>(wh);
       unsigned short* bs = as + sig_bf3_a_elems_per_k(n, nw1) * gb;
@@ -1298,13 +1298,13 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
   const cf* z = (const cf*)zmel;
   const int np = ntq * ntq;
   // scratch groups of consecutive k
-  const bool modes = sig_modes_pays(h, n, zoff[nk], nk, nw1);
+  const bool modes = sig_modes_pays(h, MBF3, n, zoff[nk], nw1);
   const size_t cap = modes ? kSigModeScratch : kSigScratch;
   std::vector<int> gstart{0};
   size_t acc = 0;
   size_t maxg = 0;
   for (int k = 0; k < nk; ++k) {
-    const size_t b = (modes ? sig_modes_bytes(n, nm[k], ntq, nw1)
+    const size_t b = (modes ? sig_modes_bytes(MBF3, n, nm[k], ntq, nw1)
                             : sig_bf3_bytes_per_k(n, std::max(nm[k] * ntq, 1), nw1)) +
                      sizeof(cf) * (size_t)n * nm[k] * ntq;
     if (acc > 0 && acc + b > cap) {
@@ -1346,9 +1346,9 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
     cf* cz;
     if (modes) {
       size_t b = 0;
-      for (int k = k0; k < k1; ++k) b += sig_modes_bytes(n, nm[k], ntq, nw1);
+      for (int k = k0; k < k1; ++k) b += sig_modes_bytes(MBF3, n, nm[k], ntq, nw1);
       cz = reinterpret_cast<cf*>(wh + b);
-      ECALJ_TRY(sig_modes(h, k1 - k0, nm + k0, ntq, z + (int64_t)n * zoff[k0], n, nw1, wc + wstride * k0, ldw, wstride,
+      ECALJ_TRY(sig_modes(h, MBF3, k1 - k0, nm + k0, ntq, z + (int64_t)n * zoff[k0], n, nw1, wc + wstride * k0, ldw, wstride,
                           wgt + nw1 * zoff[k0], cz, wh));
     } else {
       std::vector<int> ncol(k1 - k0);

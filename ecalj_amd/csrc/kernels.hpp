@@ -109,12 +109,14 @@ struct SigFinalK {
 int sig_final_chunk(int64_t rows);
 ecalj_status sig_final_bf3(ecalj_ctx* h, const cf* cz, const cf* z, int64_t R, int64_t zs, int chunks,
                            const SigFinalK* tab, int nk, int64_t nblk, int KC, int ntq, cf* part);
-// The bf16x3 contraction in frequency modes (sigmodes.hip): rule, scratch
-// bytes of one k, and the contraction of nk k-points packed one after the other.
-bool sig_modes_pays(const ecalj_ctx* h, int n, int64_t cols, int nk, int nw1);
-size_t sig_modes_bytes(int n, int nm, int ntq, int nw1);
-ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* zmel, int n, int nw1, const cd* wc,
-                       int64_t ldw, int64_t w_stride, const double* wgt, cf* cz, unsigned char* scratch);
+// The contraction in frequency modes (sigmodes.hip): rule, scratch bytes of
+// one k, and czmelwc of nk k-points packed one after the other.
+constexpr int kTuneModes = 13;  // tuner mode that asks for it
+bool sig_modes_pays(const ecalj_ctx* h, int mode, int n, int64_t cols, int nw1);
+size_t sig_modes_bytes(int mode, int n, int nm, int ntq, int nw1);
+ecalj_status sig_modes(ecalj_ctx* h, int mode, int nk, const int* nm, int ntq, const void* zmel, int n, int nw1,
+                       const cd* wc, int64_t ldw, int64_t w_stride, const double* wgt, void* cz,
+                       unsigned char* scratch);
 // x0gemm in the bf16x3 form: per-bin entry lists on the host (bin b: entries
 // cnt[b]..cnt[b+1]-1 with zmel column offsets col[] and weights wt[]), output
 // slice slice[b] of rcxq (npr x npr_col, complex64, slice stride slice_elems)

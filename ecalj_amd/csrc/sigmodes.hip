@@ -1,4 +1,4 @@
-// sigmodes.hip -- the bf16x3 Sigma_c frequency contraction in frequency modes.
+// sigmodes.hip -- the Sigma_c frequency contraction in frequency modes.
 //
 //   czmelwc(I,c) = sum_v sum_J Wt_v(I,J) wgt(v,c) zmel(J,c)
 //
@@ -12,8 +12,8 @@
 // R products instead of nw1.  s_v is the Frobenius norm of W_v, so that a
 // column's error is weighed as it enters the product.  R is the number of
 // steps of a pivoted Gram-Schmidt after which the residual of EVERY column of
-// the group is at most kModeTol = 2^-25 of that column's norm, the rounding
-// of a weight to FP32 (which every form of the contraction does); weights
+// the group is at most the rounding of its weights (2^-25 of their norm in the
+// mixed forms, which take them in FP32, 2^-51 in FP64); weights
 // that span all frequencies give R = nw1 and the plain contraction.
 // R is found and used on the device: no host wait, and a captured graph
 // replays with the ranks of its present inputs.
@@ -38,9 +38,15 @@ namespace ecalj {
 
 constexpr int kModeMax = Q3NW;    // frequencies, and therefore modes, of one launch
 constexpr int kModeChunks = 16;   // partial sums of one W norm
-constexpr int kModePool = 4;      // planes kept per k, in units of its frequencies
+// Planes kept per k, in units of its frequencies: the mean rank times the
+// groups (C3: 12 groups of 6 modes; FP64 at C2: 13 of 11), with room to spare
+template <class WT>
+__host__ __device__ constexpr int mode_pool_planes() { return sizeof(WT) == 4 ? 6 : 11; }
 constexpr int kModeSort = 16384;  // columns of one sort (128 KB of LDS)
-constexpr double kModeTol = 1.0 / 33554432.0;
+// Largest residual of a column's weights, relative: 2^-25, the rounding of a
+// weight to FP32; FP64: 2^-51, the weights' own rounding with that of the steps.
+template <class G>
+__host__ __device__ constexpr double mode_tol() { return sizeof(G) == 4 ? 0x1p-25 : 0x1p-51; }
 
 // Columns c0 .. c0+cnt-1 of one internal k, sorted together.
 struct SigModeSort {
@@ -132,12 +138,14 @@ __global__ __launch_bounds__(256) void mode_norm_kernel(const cd* __restrict__ w
 // gm: mode weights (FP32, mode-major, ncp each); coef: kModeMax x kModeMax
 // per group, coef[r*kModeMax + v] = Q_vr / s_v; rank >= 1.
 // Latency-bound: 8-15 steps, each one pass over X in L2.
+template <class WT>
 __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restrict__ grp, const int* __restrict__ perm,
                                                          const double* __restrict__ wgt,
                                                          const double* __restrict__ part, int nw1,
                                                          double* __restrict__ xs, double* __restrict__ nrms,
-                                                         float* __restrict__ gms, float* __restrict__ coef,
+                                                         WT* __restrict__ gms, WT* __restrict__ coef,
                                                          SigModeRank* __restrict__ rank) {
+  constexpr double kTol2 = mode_tol<WT>() * mode_tol<WT>();
   __shared__ double sv[kModeMax], q[kModeMax];
   __shared__ double bval[8];
   __shared__ int bcol[8];
@@ -146,8 +154,8 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
   const int64_t cbase = g.cbase;
   double* X = xs + cbase * nw1;
   double* nrm = nrms + cbase;
-  float* gm = gms + cbase * nw1;
-  float* cf_ = coef + (int64_t)blockIdx.x * kModeMax * kModeMax;
+  WT* gm = gms + cbase * nw1;
+  WT* cf_ = coef + (int64_t)blockIdx.x * kModeMax * kModeMax;
   if (t < kModeMax) {
     double s = 0.0;
     if (t < nw1)
@@ -157,7 +165,7 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
     // or NaN goes unscaled, so that they reach every mode and the result
     sv[t] = (s < 1e-36) ? 0.0 : (s < 1e300 ? s : 1.0);
   }
-  for (int e = t; e < kModeMax * kModeMax; e += 512) cf_[e] = 0.f;
+  for (int e = t; e < kModeMax * kModeMax; e += 512) cf_[e] = 0;
   __syncthreads();
   double best = 0.0;
   int bc = 0;
@@ -184,7 +192,7 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
         r2 += y * y;
       }
     nrm[c] = nr;
-    gm[c] = n2 < 1e300 ? 0.f : __builtin_nanf("");  // (stays where no mode is found)
+    gm[c] = n2 < 1e300 ? (WT)0 : (WT)__builtin_nanf("");  // (stays where no mode is found)
     if (r2 > best) {
       best = r2;
       bc = c;
@@ -214,11 +222,11 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
         best = bval[w];
         bc = bcol[w];
       }
-    if (!(best > kModeTol * kModeTol)) break;
+    if (!(best > kTol2)) break;
     if (t < nw1) {
       const double x = X[(int64_t)t * ncp + bc] / sqrt(best);
       q[t] = x;
-      cf_[r * kModeMax + t] = sv[t] > 0.0 ? (float)(x / sv[t]) : 0.f;
+      cf_[r * kModeMax + t] = sv[t] > 0.0 ? (WT)(x / sv[t]) : (WT)0;
     }
     __syncthreads();
     best = 0.0;
@@ -240,7 +248,7 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
           X[(int64_t)v * ncp + c] = y;
           r2 += y * y;
         }
-      gm[(int64_t)r * ncp + c] = (float)(d * nrm[c]);
+      gm[(int64_t)r * ncp + c] = (WT)(d * nrm[c]);
       if (r2 > best) {
         best = r2;
         bc = c;
@@ -251,13 +259,14 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
 }
 
 // Places of the groups' modes in the plane pool of their k (one block per
-// group): coefp[(k kModePool nw1 + p) kModeMax + v] for plane p, nplane[k]
+// group): coefp[(k pool planes + p) kModeMax + v] for plane p, nplane[k]
 // planes.  When they do not fit, every group of the k takes the W planes of
 // the frequencies themselves with the weights as they are: the plain contraction.
+template <class WT>
 __global__ __launch_bounds__(256) void mode_pack_kernel(const SigMode* __restrict__ grp, const int* __restrict__ kgrp,
                                                         const int* __restrict__ perm, const double* __restrict__ wgt,
-                                                        int nw1, float* __restrict__ gms,
-                                                        const float* __restrict__ coef, float* __restrict__ coefp,
+                                                        int nw1, WT* __restrict__ gms,
+                                                        const WT* __restrict__ coef, WT* __restrict__ coefp,
                                                         int* __restrict__ nplane, SigModeRank* __restrict__ rank) {
   const SigMode g = grp[blockIdx.x];
   const int g0 = kgrp[g.k], g1 = kgrp[g.k + 1];
@@ -266,10 +275,10 @@ __global__ __launch_bounds__(256) void mode_pack_kernel(const SigMode* __restric
     if (i == (int)blockIdx.x) before = tot;
     tot += rank[i].raw;
   }
-  const bool fits = tot <= kModePool * nw1;
+  const bool fits = tot <= mode_pool_planes<WT>() * nw1;
   SigModeRank* r = rank + blockIdx.x;
   const int R = fits ? r->raw : nw1;
-  float* cp = coefp + ((int64_t)g.k * kModePool * nw1 + (fits ? before : 0)) * kModeMax;
+  WT* cp = coefp + ((int64_t)g.k * mode_pool_planes<WT>() * nw1 + (fits ? before : 0)) * kModeMax;
   if (threadIdx.x == 0) {
     r->rank = R;
     r->poff = fits ? before : 0;
@@ -277,11 +286,11 @@ __global__ __launch_bounds__(256) void mode_pack_kernel(const SigMode* __restric
   }
   if (fits || (int)blockIdx.x == g0)
     for (int e = threadIdx.x; e < R * kModeMax; e += 256)
-      cp[e] = fits ? coef[(int64_t)blockIdx.x * kModeMax * kModeMax + e] : (e / kModeMax == e % kModeMax ? 1.f : 0.f);
+      cp[e] = fits ? coef[(int64_t)blockIdx.x * kModeMax * kModeMax + e] : (e / kModeMax == e % kModeMax ? (WT)1 : (WT)0);
   if (!fits)
     for (int e = threadIdx.x; e < g.ncp * nw1; e += 256) {
       const int c = e % g.ncp, v = e / g.ncp;
-      gms[g.cbase * nw1 + e] = c < g.ncol ? (float)wgt[g.gsrc + (int64_t)nw1 * perm[g.cbase + c] + v] : 0.f;
+      gms[g.cbase * nw1 + e] = c < g.ncol ? (WT)wgt[g.gsrc + (int64_t)nw1 * perm[g.cbase + c] + v] : (WT)0;
     }
 }
 
@@ -336,7 +345,7 @@ __global__ __launch_bounds__(512, 4) void mode_planes_kernel(const cd* __restric
                       8 * chunk_slot(row, wc);
   const bool put = wo == 0 || a < b;
   const int P = nplane[k];
-  const float* c0 = coefp + (int64_t)k * kModePool * nw1 * kModeMax;
+  const float* c0 = coefp + (int64_t)k * mode_pool_planes<float>() * nw1 * kModeMax;
   for (int p = 0; p < P; p += 2) {
     float2(*T)[32][34] = tr[(p >> 1) & 1];
 #pragma unroll
@@ -425,41 +434,212 @@ __global__ __launch_bounds__(512, 1) void sig3m_modes_kernel(const SigMode* __re
       (sigma % R) * QBM, c0, 0, cz + g.zsrc, (int64_t)n);
 }
 
+// ---------------------------------------------------------------- FP64 and FP32 forms
+// Planes of the modes for the planar GEMM: mode p of the k as a full n x n
+// matrix W'(I,J) in the contraction's type, from the upper triangle (tile pair
+// (a, b) written as (I, J) and, through LDS, as its conjugate transpose).
+template <class T, int NV>
+__global__ __launch_bounds__(512) void mode_full_kernel(const cd* __restrict__ w, int64_t ldw, int64_t w_stride,
+                                                        int n, int nw1, int64_t pool, const int* __restrict__ kpool,
+                                                        const typename ElemT<T>::V* __restrict__ coefp,
+                                                        const int* __restrict__ nplane, T* __restrict__ as) {
+  typedef typename ElemT<T>::V V;
+  __shared__ T tr[2][32][33];
+  const int64_t tri = blockIdx.x;
+  int b = (int)((sqrt(8.0 * (double)tri + 1.0) - 1.0) * 0.5);
+  while ((int64_t)(b + 1) * (b + 2) / 2 <= tri) ++b;
+  while ((int64_t)b * (b + 1) / 2 > tri) --b;
+  const int a = (int)(tri - (int64_t)b * (b + 1) / 2);
+  const int k = blockIdx.y;
+  if (kpool[k] < 0) return;  // no columns
+  // thread: elements (I0 + i, J0 + j + 16 e)
+  const int i = threadIdx.x & 31, j = threadIdx.x >> 5;
+  const int I = a * 32 + i, I2 = b * 32 + i;
+  const cd* W = w + w_stride * k;
+  V xr[NV][2], xi[NV][2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int J = b * 32 + j + 16 * e;
+    const bool low = I > J;
+    const int64_t o = low ? J + ldw * I : I + ldw * J;
+    const bool in = I < n && J < n;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const cd x = (in && v < nw1) ? W[o + ldw * n * v] : cd{0.0, 0.0};
+      xr[v][e] = (V)x.re;
+      xi[v][e] = low ? -(V)x.im : (V)x.im;
+    }
+  }
+  const int P = nplane[k];
+  const int64_t nn = (int64_t)n * n;
+  T* A = as + pool * kpool[k];
+  const V* c0 = coefp + (int64_t)k * mode_pool_planes<V>() * nw1 * kModeMax;
+  for (int p = 0; p < P; ++p) {
+    T(*L)[33] = tr[p & 1];
+    const V* c = c0 + p * kModeMax;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      V ar = 0, ai = 0;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        ar += c[v] * xr[v][e];
+        ai += c[v] * xi[v][e];
+      }
+      const int J = b * 32 + j + 16 * e;
+      if (I < n && J < n) A[nn * p + I + (int64_t)n * J] = T{ar, ai};
+      L[j + 16 * e][i] = T{ar, -ai};
+    }
+    if (a == b) continue;  // uniform
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int J2 = a * 32 + j + 16 * e;
+      if (I2 < n && J2 < n) A[nn * p + I2 + (int64_t)n * J2] = L[i][j + 16 * e];
+    }
+  }
+}
+
+// B operand of the planar GEMM: B(kk, c') = gm_r(c') zmel(J, perm[c']), kk = r n + J.
+// A thread's columns stay the same over the stages, so their addresses are kept.
+template <class T, int BN, int BK>
+struct LdMode {
+  typedef typename ElemT<T>::V V;
+  static constexpr int R = BN * BK / kThreads, XS = kThreads / BK;
+  const T* z[R];   // column base (null: padding)
+  const V* gm;     // weights of the thread's first column
+  int n, ncp, K;
+  unsigned inv;    // ceil(2^32 / n): kk / n = umulhi(kk, inv) while kk n < 2^32, n >= 2
+  struct Regs { V re[R]; V im[R]; };
+  __device__ void init(const T* zk, const V* gms, const int* pm, int n_, int ncp_, int K_) {
+    n = n_;
+    ncp = ncp_;
+    K = K_;
+    inv = (unsigned)((0x100000000ull + n - 1) / n);
+    const int x = threadIdx.x / BK;
+    gm = gms + x;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int c = pm[x + q * XS];
+      z[q] = c >= 0 ? zk + (int64_t)n * c : nullptr;
+    }
+  }
+  __device__ void fetch(int, int k0, Regs& r) const {
+    const int kk = k0 + threadIdx.x % BK;
+    const int v = (int)__umulhi((unsigned)kk, inv), J = kk - v * n;
+    const bool in = kk < K;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      r.re[q] = 0;
+      r.im[q] = 0;
+      if (in && z[q]) {
+        const V g = gm[(int64_t)v * ncp + q * XS];
+        const T x = z[q][J];
+        r.re[q] = g * x.re;
+        r.im[q] = g * x.im;
+      }
+    }
+  }
+  template <class S>
+  __device__ void store(S& s, const Regs& r) const {
+#pragma unroll
+    for (int q = 0; q < R; ++q) s.putB(threadIdx.x % BK, threadIdx.x / BK + q * XS, r.re[q], r.im[q]);
+  }
+};
+
+// czmelwc on the planar GEMM core, 64 x 64 tiles, K = rank x n; block order as
+// sig3m_modes_kernel.
+template <int MODE, class T>
+__global__ __launch_bounds__(kThreads) void mode_gemm_kernel(const SigMode* __restrict__ grp,
+                                                             const SigModeTile* __restrict__ runs, int nrun, int G,
+                                                             const SigModeRank* __restrict__ rank,
+                                                             const int* __restrict__ perm, const T* __restrict__ as,
+                                                             const T* __restrict__ zmel,
+                                                             const typename ElemT<T>::V* __restrict__ gms, int n,
+                                                             int nw1, T* __restrict__ cz) {
+  constexpr int BK = ModeBK<MODE>::value;
+  typedef typename ElemT<T>::V V;
+  __shared__ typename StageOf<MODE, 64, 64, BK>::type s;
+  const int p = blockIdx.x, x = p & 7, j = p >> 3, R = (n + 63) / 64;
+  const int sigma = (j / G) * 8 + x, loc = j % G;
+  if (sigma >= nrun * R) return;
+  const SigModeTile t = runs[sigma / R];
+  if (loc >= t.cnt) return;
+  const SigMode g = grp[t.grp];
+  const int c0 = (t.ct0 + loc) * 64, m0 = (sigma % R) * 64, K = rank[t.grp].rank * n;
+  const int* pm = perm + g.cbase + c0;
+  Ld<AccN<T, false>, 64, BK, true, 1> la{
+      AccN<T, false>{as + g.wbase + (int64_t)rank[t.grp].poff * n * n, (int64_t)n, n, K, (V)1}};
+  LdMode<T, 64, BK> lb;
+  lb.init(zmel + g.zsrc, gms + g.cbase * nw1 + c0, pm, n, g.ncp, K);
+  Core<MODE, 64, 64, BK, false> core;
+  gemm_mainloop<MODE, 64, 64, BK, false>(la, lb, m0, 0, K, s, core);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  core.for_each(wave >> 1, wave & 1, lane, [&](int rr, int cc, double xr, double xi) {
+    const int i = m0 + rr, c = pm[cc];
+    if (i < n && c >= 0) st_c(cz + g.zsrc + i + (int64_t)n * c, xr, xi);
+  });
+}
+
 // ---------------------------------------------------------------- host
-// Column tiles of the groups of one sort of T tiles: sqrt(1.6 T) equal groups,
-// about the least of rank sum x tiles + 1.5 tiles per mode (23 tiles: 6
-// groups, 90 tiles: 12), at most 16.
-static int mode_group_tiles(int T) {
-  const int G = std::max(1, std::min(16, (int)(std::sqrt(1.6 * T) + 0.5)));
+// Column tiles of the groups of one sort of T tiles: sqrt(f T) equal groups,
+// about the least of rank sum x tiles + 1/f.. tiles per mode.  bf16x3, f = 1.6:
+// a mode costs about 1.5 tiles at one rank (23 tiles: 6 groups, 90 tiles: 12);
+// FP64 / FP32 on 64-column tiles, f = 3.5: about 0.3 (45 tiles: 13 groups).
+constexpr int kModeGroups = 16;
+static int mode_group_tiles(int T, double f) {
+  const int G = std::max(1, std::min(kModeGroups, (int)(std::sqrt(f * T) + 0.5)));
   return (T + G - 1) / G;
 }
 
 // Whether the mode form is taken.  Frequencies: one launch holds kModeMax;
-// fewer than 8 leave too little to save.  Columns: below about 1000 per k the
-// basis and the extra launches cost what the ranks save.
-bool sig_modes_pays(const ecalj_ctx* h, int n, int64_t cols, int nk, int nw1) {
-  return h->tune_mode == 0 && !h->sigc_fp8 && nw1 >= 8 && nw1 <= kModeMax && n >= 128 && cols >= 1000LL * nk;
+// fewer than 8 leave too little to save.  Work: the order, the bases and the
+// extra launches take about 0.2 ms, so the plain contraction has to take more
+// than about twice that (2e11 flop in the bf16x3 form, 4e10 in FP64 and FP32).
+// Tuner mode kTuneModes asks for it at any size.
+bool sig_modes_pays(const ecalj_ctx* h, int mode, int n, int64_t cols, int nw1) {
+  if (nw1 > kModeMax || n < 2 || n > 13000) return false;  // n: what LdMode divides by
+  if (mode == MBF3 && h->sigc_fp8) return false;
+  if (h->tune_mode == kTuneModes) return true;
+  if (mode == MBF3 && h->tune_mode != 0) return false;
+  return nw1 >= 8 && 8.0 * n * n * nw1 * (double)cols >= (mode == MBF3 ? 2e11 : 4e10);
 }
 
 static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// What one k of a call takes: elements of its plane pool, and whether its
+// zmel is copied in sorted order (bf16x3).
+static int64_t mode_planes_max(int mode, int nw1) {
+  return (int64_t)nw1 * (mode == M64 ? mode_pool_planes<double>() : mode_pool_planes<float>());
+}
+static int64_t mode_pool(int mode, int n, int nw1) {
+  return mode_planes_max(mode, nw1) * (mode == MBF3 ? (int64_t)sig3m_a_elems_per_k(n, 1) : (int64_t)n * n);
+}
+static size_t mode_pool_elem(int mode) { return mode == MBF3 ? 2 : mode == M64 ? sizeof(cd) : sizeof(cf); }
+
 // Scratch of one k: plane pool, padded zmel, order, residuals, weights
-size_t sig_modes_bytes(int n, int nm, int ntq, int nw1) {
+size_t sig_modes_bytes(int mode, int n, int nm, int ntq, int nw1) {
+  const size_t wt = mode == M64 ? 8 : 4;
   // norms, coefficients and counts of a k, also of one without columns
-  const size_t per_k = (size_t)nw1 * (kModeChunks * 8 + kModePool * kModeMax * 4) + 4;
+  const size_t per_k = (size_t)nw1 * kModeChunks * 8 + mode_planes_max(mode, nw1) * kModeMax * wt + 4;
   if (nm == 0) return al256(per_k);
   const int64_t NP = pad_to(n, QBK), ncol = (int64_t)nm * ntq, ncp = (ncol + Q3BN - 1) / Q3BN * Q3BN;
-  const int64_t groups = 16 * (ncol / kModeSort + 1);
-  return al256(kModePool * sig3m_a_elems_per_k(n, nw1) * 2 + (size_t)ncp * (sizeof(cf) * NP + 12 * nw1 + 12) +
-               (kModeMax * kModeMax * 4 + sizeof(SigModeRank)) * groups + per_k + 4096);
+  const int64_t groups = kModeGroups * (ncol / kModeSort + 1);
+  return al256(mode_pool(mode, n, nw1) * mode_pool_elem(mode) +
+               (size_t)ncp * ((mode == MBF3 ? sizeof(cf) * NP : 0) + (8 + wt) * nw1 + 12) +
+               (kModeMax * kModeMax * wt + sizeof(SigModeRank)) * groups + per_k + 4096);
 }
 
 // czmelwc of nk internal k-points (zmel, wgt, cz packed per k: n x nm[k] x ntq
-// and nw1 x nm[k] x ntq); scratch: the sum of sig_modes_bytes.
-ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* zmel, int n, int nw1, const cd* wc,
-                       int64_t ldw, int64_t w_stride, const double* wgt, cf* cz, unsigned char* scratch) {
-  const int MP = pad_to(n, QBM), NP = pad_to(n, QBK), NS = NP / QBK, R = MP / QBM;
-  const int64_t pool = kModePool * (int64_t)sig3m_a_elems_per_k(n, nw1);
+// and nw1 x nm[k] x ntq) in the storage type of the mode; scratch: the sum of
+// sig_modes_bytes.
+template <int MODE, class T, class WT>
+static ecalj_status sig_modes_t(ecalj_ctx* h, int nk, const int* nm, int ntq, const T* zmel, int n, int nw1,
+                                const cd* wc, int64_t ldw, int64_t w_stride, const double* wgt, T* cz,
+                                unsigned char* scratch) {
+  constexpr int BN = MODE == MBF3 ? Q3BN : 64;
+  constexpr double GF = MODE == MBF3 ? 1.6 : 3.5;
+  const int MP = pad_to(n, QBM), NP = pad_to(n, QBK), NS = NP / QBK, R = MODE == MBF3 ? MP / QBM : (n + 63) / 64;
+  const int64_t pool = mode_pool(MODE, n, nw1);
   std::vector<SigModeSort> sorts;
   std::vector<SigMode> grp;
   std::vector<int> kgrp(2 * nk + 1, 0);  // first group of each k, then its pool (-1: no columns)
@@ -469,18 +649,18 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
   for (int k = 0; k < nk; ++k) {
     const int64_t N = (int64_t)nm[k] * ntq;
     if (N > 0x7fffffff / 2) return ECALJ_ERR_DIM;
-    const int T = (int)((N + Q3BN - 1) / Q3BN), per = kModeSort / Q3BN, parts = (T + per - 1) / per;
-    const int tp = parts ? (T + parts - 1) / parts : 0;  // column tiles of one sort
-    for (int t0 = 0; t0 < T; t0 += tp) {
-      const int tn = std::min(tp, T - t0), cnt = (int)std::min<int64_t>(N - (int64_t)t0 * Q3BN, (int64_t)tn * Q3BN);
-      sorts.push_back({co * nw1, cols, t0 * Q3BN, cnt, tn * Q3BN, 0});
-      const int gt = mode_group_tiles(tn);
+    const int TT = (int)((N + BN - 1) / BN), per = kModeSort / BN, parts = (TT + per - 1) / per;
+    const int tp = parts ? (TT + parts - 1) / parts : 0;  // column tiles of one sort
+    for (int t0 = 0; t0 < TT; t0 += tp) {
+      const int tn = std::min(tp, TT - t0), cnt = (int)std::min<int64_t>(N - (int64_t)t0 * BN, (int64_t)tn * BN);
+      sorts.push_back({co * nw1, cols, t0 * BN, cnt, tn * BN, 0});
+      const int gt = mode_group_tiles(tn, GF);
       for (int g0 = 0; g0 < tn; g0 += gt) {
         const int gn = std::min(gt, tn - g0);
-        grp.push_back({cols + g0 * Q3BN, co * nw1, co * n, pools * pool, k, std::min(gn * Q3BN, cnt - g0 * Q3BN),
-                       gn * Q3BN, 0});
+        grp.push_back({cols + g0 * BN, co * nw1, co * n, pools * pool, k, std::min(gn * BN, cnt - g0 * BN), gn * BN,
+                       0});
       }
-      cols += (int64_t)tn * Q3BN;
+      cols += (int64_t)tn * BN;
     }
     co += N;
     kgrp[nk + 1 + k] = N > 0 ? pools++ : -1;
@@ -496,7 +676,7 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
     for (int k = 0; k < nk; ++k) {
       if (kgrp[k] + gi >= kgrp[k + 1]) continue;
       const SigMode& m = grp[kgrp[k] + gi];
-      const int ct = m.ncp / Q3BN, parts = (ct + 31) / 32, per = (ct + parts - 1) / parts;
+      const int ct = m.ncp / BN, parts = (ct + 31) / 32, per = (ct + parts - 1) / parts;
       for (int c = 0; c < ct; c += per) runs.push_back({kgrp[k] + gi, c, std::min(per, ct - c), 0});
       G = std::max(G, per);
       ncpmax = std::max(ncpmax, m.ncp);
@@ -511,16 +691,16 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
     q += al256(bytes);
     return r;
   };
-  unsigned short* as = (unsigned short*)take((size_t)(pool * pools) * 2);
-  cf* zp = (cf*)take(sizeof(cf) * (size_t)cols * NP);
+  unsigned char* as = take((size_t)(pool * pools) * mode_pool_elem(MODE));
+  cf* zp = (cf*)take(MODE == MBF3 ? sizeof(cf) * (size_t)cols * NP : 0);
   double* xs = (double*)take(sizeof(double) * (size_t)cols * nw1);
   double* nrm = (double*)take(sizeof(double) * (size_t)cols);
-  float* gm = (float*)take(sizeof(float) * (size_t)cols * nw1);
+  WT* gm = (WT*)take(sizeof(WT) * (size_t)cols * nw1);
   int* perm = (int*)take(sizeof(int) * (size_t)cols);
-  float* coef = (float*)take(sizeof(float) * kModeMax * kModeMax * (size_t)ng);
+  WT* coef = (WT*)take(sizeof(WT) * kModeMax * kModeMax * (size_t)ng);
   double* part = (double*)take(sizeof(double) * kModeChunks * (size_t)nw1 * nk);
   SigModeRank* rank = (SigModeRank*)take(sizeof(SigModeRank) * (size_t)ng);
-  float* coefp = (float*)take(sizeof(float) * kModeMax * kModePool * (size_t)nw1 * nk);
+  WT* coefp = (WT*)take(sizeof(WT) * kModeMax * (size_t)mode_planes_max(MODE, nw1) * nk);
   int* nplane = (int*)take(sizeof(int) * (size_t)nk);
   // tables
   const size_t b0 = sizeof(SigModeSort) * sorts.size(), b1 = sizeof(SigMode) * grp.size();
@@ -542,31 +722,60 @@ ecalj_status sig_modes(ecalj_ctx* h, int nk, const int* nm, int ntq, const cf* z
   hipLaunchKernelGGL(mode_norm_kernel, dim3(kModeChunks, nw1 * nk), dim3(256), 0, h->stream, wc, ldw, w_stride, n, nw1,
                      part);
   ECALJ_HIP(hipGetLastError());
-  hipLaunchKernelGGL(mode_basis_kernel, dim3(ng), dim3(512), 0, h->stream, dg, perm, wgt, part, nw1, xs, nrm, gm, coef,
-                     rank);
+  hipLaunchKernelGGL(mode_basis_kernel<WT>, dim3(ng), dim3(512), 0, h->stream, dg, perm, wgt, part, nw1, xs, nrm, gm,
+                     coef, rank);
   ECALJ_HIP(hipGetLastError());
-  hipLaunchKernelGGL(mode_pack_kernel, dim3(ng), dim3(256), 0, h->stream, dg, dk, perm, wgt, nw1, gm, coef,
-                     coefp, nplane, rank);
+  hipLaunchKernelGGL(mode_pack_kernel<WT>, dim3(ng), dim3(256), 0, h->stream, dg, dk, perm, wgt, nw1, gm, coef, coefp,
+                     nplane, rank);
   ECALJ_HIP(hipGetLastError());
-  auto planes = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)npair, nk), dim3(512), 0, h->stream, wc, ldw, w_stride, n, nw1, MP, NS,
-                       pool, dk + nk + 1, coefp, nplane, as);
-  };
-  if (nw1 <= 13) planes(mode_planes_kernel<13>);
-  else if (nw1 <= 17) planes(mode_planes_kernel<17>);
-  else if (nw1 <= 21) planes(mode_planes_kernel<21>);
-  else planes(mode_planes_kernel<24>);
-  ECALJ_HIP(hipGetLastError());
-  hipLaunchKernelGGL(mode_pad_kernel, dim3(std::min(ncpmax, 4096), ng), dim3(256), 0, h->stream, dg, perm, zmel, n, NP,
-                     zp);
-  ECALJ_HIP(hipGetLastError());
+  const dim3 pgrid((unsigned)npair, nk);
+  if constexpr (MODE == MBF3) {
+    auto planes = [&](auto kern) {
+      hipLaunchKernelGGL(kern, pgrid, dim3(512), 0, h->stream, wc, ldw, w_stride, n, nw1, MP, NS, pool, dk + nk + 1,
+                         coefp, nplane, (unsigned short*)as);
+    };
+    if (nw1 <= 13) planes(mode_planes_kernel<13>);
+    else if (nw1 <= 17) planes(mode_planes_kernel<17>);
+    else if (nw1 <= 21) planes(mode_planes_kernel<21>);
+    else planes(mode_planes_kernel<24>);
+    ECALJ_HIP(hipGetLastError());
+    hipLaunchKernelGGL(mode_pad_kernel, dim3(std::min(ncpmax, 4096), ng), dim3(256), 0, h->stream, dg, perm, zmel, n,
+                       NP, zp);
+    ECALJ_HIP(hipGetLastError());
+  } else {
+    auto planes = [&](auto kern) {
+      hipLaunchKernelGGL(kern, pgrid, dim3(512), 0, h->stream, wc, ldw, w_stride, n, nw1, pool, dk + nk + 1, coefp,
+                         nplane, (T*)as);
+    };
+    if (nw1 <= 13) planes(mode_full_kernel<T, 13>);
+    else if (nw1 <= 17) planes(mode_full_kernel<T, 17>);
+    else planes(mode_full_kernel<T, 24>);
+    ECALJ_HIP(hipGetLastError());
+  }
   int tev = -1;
   ECALJ_TRY(timing_begin(h, 0, &tev));
-  hipLaunchKernelGGL(sig3m_modes_kernel, dim3((unsigned)blocks), dim3(512), 0, h->stream, dg, dr, (int)runs.size(), G,
-                     rank, perm, as, zp, gm, n, nw1, MP, NS, NP, cz);
+  if constexpr (MODE == MBF3)
+    hipLaunchKernelGGL(sig3m_modes_kernel, dim3((unsigned)blocks), dim3(512), 0, h->stream, dg, dr, (int)runs.size(), G,
+                       rank, perm, (const unsigned short*)as, zp, gm, n, nw1, MP, NS, NP, cz);
+  else
+    hipLaunchKernelGGL((mode_gemm_kernel<MODE, T>), dim3((unsigned)blocks), dim3(kThreads), 0, h->stream, dg, dr,
+                       (int)runs.size(), G, rank, perm, (const T*)as, zmel, gm, n, nw1, cz);
   ECALJ_HIP(hipGetLastError());
   ECALJ_TRY(timing_end(h, 0, tev));
   return ECALJ_OK;
+}
+
+ecalj_status sig_modes(ecalj_ctx* h, int mode, int nk, const int* nm, int ntq, const void* zmel, int n, int nw1,
+                       const cd* wc, int64_t ldw, int64_t w_stride, const double* wgt, void* cz,
+                       unsigned char* scratch) {
+  if (mode == M64)
+    return sig_modes_t<M64, cd, double>(h, nk, nm, ntq, (const cd*)zmel, n, nw1, wc, ldw, w_stride, wgt, (cd*)cz,
+                                        scratch);
+  if (mode == M32)
+    return sig_modes_t<M32, cf, float>(h, nk, nm, ntq, (const cf*)zmel, n, nw1, wc, ldw, w_stride, wgt, (cf*)cz,
+                                       scratch);
+  return sig_modes_t<MBF3, cf, float>(h, nk, nm, ntq, (const cf*)zmel, n, nw1, wc, ldw, w_stride, wgt, (cf*)cz,
+                                      scratch);
 }
 
 }  // namespace ecalj

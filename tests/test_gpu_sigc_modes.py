@@ -1,6 +1,6 @@
-"""Sigma_c in frequency modes (sigmodes.hip), the bf16x3 form of calls with
-1000 and more columns per internal k and 8 to 24 frequencies, against the FP64
-oracle and the plain three-product contraction (a forced tuner variant)."""
+"""Sigma_c in frequency modes (sigmodes.hip), the form of large calls with 8 to
+24 frequencies, here asked for at small sizes (tuner mode 13), against the
+FP64 oracle and the plain contraction."""
 import numpy as np
 import pytest
 
@@ -8,10 +8,16 @@ from ecalj_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-# Every product of the bf16x3 form errs by at most ~2^-16 of its factors (the
-# dropped lo*lo term and the two lo roundings) and the sums average it; the
-# mode form adds 2^-25 of a column's weights.  2e-5 is that bound with no averaging.
-TOL = 2e-5
+# bf16x3: each of the two products in a row errs by at most ~2^-16 of its
+# factors (the dropped lo*lo term and the two lo roundings); the mode form adds
+# 2^-25 of a column's weights; 3.1e-5 is that bound with no averaging (one
+# element: 2.1e-5 in the plain form too).  f32:
+# 2^-24 per step of sums of up to 24 x 257 and then 257 x 150 terms of random
+# sign, 2^-24 sqrt(45 000) = 1.3e-5 (the plain form reaches 2.6e-6).  f64: the
+# same count of 2^-53 is 2.4e-14, and residuals of 2^-51.
+TOLS = {"bf16x3": 3.1e-5, "f32": 1.3e-5, "f64": 1e-13}
+TOL = TOLS["bf16x3"]
+MODES = 13
 
 
 @pytest.fixture(scope="module")
@@ -58,31 +64,34 @@ def case(orc, seed, ngb, nm, ntq, nf, weights):
 
 # rows: tile remainders and a full tile; columns: a whole number of tiles, one
 # more, one group and several; frequencies: both ends and the plane kernel's edges
+@pytest.mark.parametrize("prec", ["bf16x3", "f32", "f64"])
 @pytest.mark.parametrize("weights", ["physical", "random", "rank1", "one_column"])
 @pytest.mark.parametrize("ngb,nm,ntq,nf", [(128, 128, 8, 7), (161, 129, 9, 11), (130, 67, 16, 12), (200, 113, 10, 17),
-                                           (257, 150, 7, 18), (131, 80, 33, 23)])
-def test_modes_against_oracle(orc, weights, ngb, nm, ntq, nf):
+                                           (257, 150, 7, 18), (131, 80, 33, 23), (33, 9, 5, 9),
+                                            (1, 3, 1, 1)])
+def test_modes_against_oracle(orc, prec, weights, ngb, nm, ntq, nf):
     import ecalj_amd
 
     z, w, g = case(orc, ngb + nf, ngb, nm, ntq, nf, weights)
     ref = orc.sigc_imag(z, w, g)
-    h = ecalj_amd.Handle(0, "bf16x3")
+    h = ecalj_amd.Handle(0, prec)
     try:
+        h.set_tuning(MODES)
         got = h.sigc(z, w, g)
         again = h.sigc(z, w, g)
         h.set_tuning(6)
         plain = h.sigc(z, w, g)
     finally:
         h.close()
-    print(weights, ngb, nm, ntq, nf, relerr(got, ref), relerr(plain, ref), flush=True)
-    assert relerr(got, ref) < TOL
+    print(prec, weights, ngb, nm, ntq, nf, relerr(got, ref), relerr(plain, ref), flush=True)
+    assert relerr(got, ref) < TOLS[prec]
     assert np.array_equal(got, again)
-    # against the plain form: both roundings, averaged over the columns
-    assert relerr(got, plain) < TOL
+    assert relerr(got, plain) < TOLS[prec]
 
 
+@pytest.mark.parametrize("prec", ["bf16x3", "f32", "f64"])
 @pytest.mark.parametrize("nms", [[140, 0, 70, 211], [200]])
-def test_modes_grouped(orc, nms):
+def test_modes_grouped(orc, nms, prec):
     import ecalj_amd
 
     ngb, ntq, nf = 150, 11, 14
@@ -91,10 +100,11 @@ def test_modes_grouped(orc, nms):
     for nm, z, w, g in zip(nms, zs, ws, gs):
         if nm:
             ref = orc.sigc_imag(z, w, g, ref)
-    h = ecalj_amd.Handle(0, "bf16x3")
+    h = ecalj_amd.Handle(0, prec)
     try:
+        h.set_tuning(MODES)
         cat = lambda xs: np.concatenate([x.ravel(order="F") for nm, x in zip(nms, xs) if nm])
-        dz, dg = h.to_dev(cat(zs).astype(np.complex64)), h.to_dev(cat(gs))
+        dz, dg = h.to_dev(cat(zs).astype(np.complex128 if prec == "f64" else np.complex64)), h.to_dev(cat(gs))
         dw = h.to_dev(np.concatenate([w.ravel(order="F") for w in ws]))
         s = h.array((ntq, ntq))
         s.zero()
@@ -103,7 +113,7 @@ def test_modes_grouped(orc, nms):
     finally:
         h.close()
     print(nms, relerr(got, ref), flush=True)
-    assert relerr(got, ref) < TOL
+    assert relerr(got, ref) < TOLS[prec]
 
 
 def test_modes_more_columns_than_one_sort(orc):
@@ -119,6 +129,7 @@ def test_modes_more_columns_than_one_sort(orc):
     ref = orc.sigc_imag(np.asfortranarray(z[:, keep]), w, np.asfortranarray(g[:, keep]))
     h = ecalj_amd.Handle(0, "bf16x3")
     try:
+        h.set_tuning(MODES)
         got = h.sigc(z, w, g)
     finally:
         h.close()
@@ -132,6 +143,7 @@ def test_modes_non_finite_inputs_reach_the_result(orc):
     z, w, g = case(orc, 5, 130, 130, 8, 9, "physical")
     h = ecalj_amd.Handle(0, "bf16x3")
     try:
+        h.set_tuning(MODES)
         for bad in (np.inf, np.nan):
             w2 = w.copy(order="F")
             w2[3, 70, 4] = bad
@@ -154,6 +166,7 @@ def test_modes_graph_replay_follows_its_inputs(orc):
     z, w, g1 = case(orc, 21, ngb, nm, ntq, nf, "rank1")
     h = ecalj_amd.Handle(0, "bf16x3")
     try:
+        h.set_tuning(MODES)
         dz, dw, dg, s = h.to_dev(z.astype(np.complex64)), h.to_dev(w), h.to_dev(g1), h.array((ntq, ntq))
 
         def call():
