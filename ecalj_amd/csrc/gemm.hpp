@@ -483,6 +483,34 @@ struct GemmArgs {
   int xg, xt;
 };
 
+// Epilogue of one output element (i, j) with product (xr, xi); C at batch b.
+template <class T>
+__device__ __forceinline__ void gemm_store(const GemmArgs& g, T* Cb, int i, int j, double xr, double xi) {
+  if (i >= g.M || j >= g.N) return;
+  T* p = Cb + i + g.ldc * j;
+  // (the contraction of the products is spelled out, so that every kernel rounds alike)
+  double vr = __builtin_fma(g.alr, xr, -(g.ali * xi));
+  double vi = __builtin_fma(g.ali, xr, g.alr * xi);
+  if (g.epi == EPI_STORE) {
+    if (g.ber != 0.0 || g.bei != 0.0) {
+      double orr, oi;
+      ld_c2(p, orr, oi);
+      vr += g.ber * orr - g.bei * oi;
+      vi += g.ber * oi + g.bei * orr;
+    }
+    if (g.conjC) vi = -vi;
+    st_c(p, vr, vi);
+  } else if (g.epi == EPI_EPS) {
+    const double sc = g.svec[i] * g.svec[j];
+    st_c(p, (i == j ? 1.0 : 0.0) - sc * vr, -sc * vi);
+  } else {  // EPI_GJ
+    if (i >= g.gj_k0 && i < g.gj_k1) return;
+    double orr = 0.0, oi = 0.0;
+    if (!(j >= g.gj_k0 && j < g.gj_k1)) ld_c2(p, orr, oi);
+    st_c(p, orr - vr, oi - vi);
+  }
+}
+
 template <int MODE, class T, int BM, int BN, bool AT, bool AREAL, bool BT>
 __global__ __launch_bounds__(kThreads) void zgemm_kernel(GemmArgs g) {
   constexpr int BK = ModeBK<MODE>::value;
@@ -517,31 +545,8 @@ __global__ __launch_bounds__(kThreads) void zgemm_kernel(GemmArgs g) {
   gemm_mainloop<MODE, BM, BN, BK, AREAL>(la, lb, m0, n0, g.K, s, core);
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  core.for_each(wave >> 1, wave & 1, lane, [&](int r, int c, double xr, double xi) {
-    const int i = m0 + r, j = n0 + c;
-    if (i >= g.M || j >= g.N) return;
-    T* p = Cb + i + g.ldc * j;
-    double vr = g.alr * xr - g.ali * xi;
-    double vi = g.alr * xi + g.ali * xr;
-    if (g.epi == EPI_STORE) {
-      if (g.ber != 0.0 || g.bei != 0.0) {
-        double orr, oi;
-        ld_c2(p, orr, oi);
-        vr += g.ber * orr - g.bei * oi;
-        vi += g.ber * oi + g.bei * orr;
-      }
-      if (g.conjC) vi = -vi;
-      st_c(p, vr, vi);
-    } else if (g.epi == EPI_EPS) {
-      const double sc = g.svec[i] * g.svec[j];
-      st_c(p, (i == j ? 1.0 : 0.0) - sc * vr, -sc * vi);
-    } else {  // EPI_GJ
-      if (i >= g.gj_k0 && i < g.gj_k1) return;
-      double orr = 0.0, oi = 0.0;
-      if (!(j >= g.gj_k0 && j < g.gj_k1)) ld_c2(p, orr, oi);
-      st_c(p, orr - vr, oi - vi);
-    }
-  });
+  core.for_each(wave >> 1, wave & 1, lane,
+                [&](int r, int c, double xr, double xi) { gemm_store(g, Cb, m0 + r, n0 + c, xr, xi); });
 }
 
 }  // namespace ecalj

@@ -60,6 +60,7 @@ ecalj_status gemm(ecalj_ctx* h, const GemmCall& c) {
   const bool at = c.ta, bt = c.tb;
   switch (c.mode) {
     case M64:
+      if (!c.areal && gemm64_pays(h, g)) return gemm64(h, g, at, bt);
       if (c.N <= 32) return launch_gemm<M64, cd, 64, 32>(h, g, at, c.areal, bt);
       return launch_gemm<M64, cd, 64, 64>(h, g, at, c.areal, bt);
     case M32:

@@ -117,6 +117,10 @@ size_t sig_modes_bytes(int mode, int n, int nm, int ntq, int nw1);
 ecalj_status sig_modes(ecalj_ctx* h, int mode, int nk, const int* nm, int ntq, const void* zmel, int n, int nw1,
                        const cd* wc, int64_t ldw, int64_t w_stride, const double* wgt, void* cz,
                        unsigned char* scratch);
+// Large FP64 products (gemm64.hip): rule and launch.
+struct GemmArgs;
+bool gemm64_pays(const ecalj_ctx* h, const GemmArgs& g);
+ecalj_status gemm64(ecalj_ctx* h, const GemmArgs& g, bool at, bool bt);
 // x0gemm in the bf16x3 form: per-bin entry lists on the host (bin b: entries
 // cnt[b]..cnt[b+1]-1 with zmel column offsets col[] and weights wt[]), output
 // slice slice[b] of rcxq (npr x npr_col, complex64, slice stride slice_elems)

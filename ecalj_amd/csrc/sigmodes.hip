@@ -32,6 +32,7 @@
 #include <cstring>
 #include <vector>
 
+#include "gemm64.hpp"
 #include "sig3mtile.hpp"
 
 namespace ecalj {
@@ -435,9 +436,10 @@ __global__ __launch_bounds__(512, 1) void sig3m_modes_kernel(const SigMode* __re
 }
 
 // ---------------------------------------------------------------- FP64 and FP32 forms
-// Planes of the modes for the planar GEMM: mode p of the k as a full n x n
-// matrix W'(I,J) in the contraction's type, from the upper triangle (tile pair
-// (a, b) written as (I, J) and, through LDS, as its conjugate transpose).
+// Planes of the modes for the planar GEMM: mode p of the k as a full matrix
+// W'(I,J), I < n, J < NK = n rounded up to 8 (zero beyond n), in the
+// contraction's type, from the upper triangle (tile pair (a, b) written as
+// (I, J) and, through LDS, as its conjugate transpose).
 template <class T, int NV>
 __global__ __launch_bounds__(512) void mode_full_kernel(const cd* __restrict__ w, int64_t ldw, int64_t w_stride,
                                                         int n, int nw1, int64_t pool, const int* __restrict__ kpool,
@@ -471,7 +473,8 @@ __global__ __launch_bounds__(512) void mode_full_kernel(const cd* __restrict__ w
     }
   }
   const int P = nplane[k];
-  const int64_t nn = (int64_t)n * n;
+  const int NK = (n + 7) / 8 * 8;
+  const int64_t nn = (int64_t)n * NK;
   T* A = as + pool * kpool[k];
   const V* c0 = coefp + (int64_t)k * mode_pool_planes<V>() * nw1 * kModeMax;
   for (int p = 0; p < P; ++p) {
@@ -486,7 +489,7 @@ __global__ __launch_bounds__(512) void mode_full_kernel(const cd* __restrict__ w
         ai += c[v] * xi[v][e];
       }
       const int J = b * 32 + j + 16 * e;
-      if (I < n && J < n) A[nn * p + I + (int64_t)n * J] = T{ar, ai};
+      if (I < n && J < NK) A[nn * p + I + (int64_t)n * J] = T{ar, ai};
       L[j + 16 * e][i] = T{ar, -ai};
     }
     if (a == b) continue;  // uniform
@@ -494,12 +497,12 @@ __global__ __launch_bounds__(512) void mode_full_kernel(const cd* __restrict__ w
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const int J2 = a * 32 + j + 16 * e;
-      if (I2 < n && J2 < n) A[nn * p + I2 + (int64_t)n * J2] = L[i][j + 16 * e];
+      if (I2 < n && J2 < NK) A[nn * p + I2 + (int64_t)n * J2] = L[i][j + 16 * e];
     }
   }
 }
 
-// B operand of the planar GEMM: B(kk, c') = gm_r(c') zmel(J, perm[c']), kk = r n + J.
+// B operand of the planar GEMM: B(kk, c') = gm_r(c') zmel(J, perm[c']), kk = r NK + J.
 // A thread's columns stay the same over the stages, so their addresses are kept.
 template <class T, int BN, int BK>
 struct LdMode {
@@ -507,14 +510,15 @@ struct LdMode {
   static constexpr int R = BN * BK / kThreads, XS = kThreads / BK;
   const T* z[R];   // column base (null: padding)
   const V* gm;     // weights of the thread's first column
-  int n, ncp, K;
-  unsigned inv;    // ceil(2^32 / n): kk / n = umulhi(kk, inv) while kk n < 2^32, n >= 2
+  int n, NK, ncp, K;
+  unsigned inv;    // ceil(2^32 / NK): kk / NK = umulhi(kk, inv) while kk NK < 2^32, n >= 2
   struct Regs { V re[R]; V im[R]; };
   __device__ void init(const T* zk, const V* gms, const int* pm, int n_, int ncp_, int K_) {
     n = n_;
     ncp = ncp_;
     K = K_;
-    inv = (unsigned)((0x100000000ull + n - 1) / n);
+    NK = (n + 7) / 8 * 8;
+    inv = (unsigned)((0x100000000ull + NK - 1) / NK);
     const int x = threadIdx.x / BK;
     gm = gms + x;
 #pragma unroll
@@ -525,8 +529,8 @@ struct LdMode {
   }
   __device__ void fetch(int, int k0, Regs& r) const {
     const int kk = k0 + threadIdx.x % BK;
-    const int v = (int)__umulhi((unsigned)kk, inv), J = kk - v * n;
-    const bool in = kk < K;
+    const int v = (int)__umulhi((unsigned)kk, inv), J = kk - v * NK;
+    const bool in = kk < K && J < n;
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       r.re[q] = 0;
@@ -546,8 +550,8 @@ struct LdMode {
   }
 };
 
-// czmelwc on the planar GEMM core, 64 x 64 tiles, K = rank x n; block order as
-// sig3m_modes_kernel.
+// czmelwc of the FP32 form on the planar GEMM core, 64 x 64 tiles, K = rank x
+// NK; block order as sig3m_modes_kernel.
 template <int MODE, class T>
 __global__ __launch_bounds__(kThreads) void mode_gemm_kernel(const SigMode* __restrict__ grp,
                                                              const SigModeTile* __restrict__ runs, int nrun, int G,
@@ -565,10 +569,10 @@ __global__ __launch_bounds__(kThreads) void mode_gemm_kernel(const SigMode* __re
   const SigModeTile t = runs[sigma / R];
   if (loc >= t.cnt) return;
   const SigMode g = grp[t.grp];
-  const int c0 = (t.ct0 + loc) * 64, m0 = (sigma % R) * 64, K = rank[t.grp].rank * n;
+  const int NK = (n + 7) / 8 * 8, c0 = (t.ct0 + loc) * 64, m0 = (sigma % R) * 64, K = rank[t.grp].rank * NK;
   const int* pm = perm + g.cbase + c0;
   Ld<AccN<T, false>, 64, BK, true, 1> la{
-      AccN<T, false>{as + g.wbase + (int64_t)rank[t.grp].poff * n * n, (int64_t)n, n, K, (V)1}};
+      AccN<T, false>{as + g.wbase + (int64_t)rank[t.grp].poff * n * NK, (int64_t)n, n, K, (V)1}};
   LdMode<T, 64, BK> lb;
   lb.init(zmel + g.zsrc, gms + g.cbase * nw1 + c0, pm, n, g.ncp, K);
   Core<MODE, 64, 64, BK, false> core;
@@ -580,11 +584,84 @@ __global__ __launch_bounds__(kThreads) void mode_gemm_kernel(const SigMode* __re
   });
 }
 
+// czmelwc of the FP64 form on the 128 x 64 tile of gemm64.hpp: a lane moves 8 k
+// of one column per stage, so the gather costs one pointer per lane, and the
+// mode's weight multiplies the fragments of the lane's two columns after the
+// LDS read.  Block order as sig3m_modes_kernel.
+__global__ __launch_bounds__(D6T, 4) void mode_gemm64_kernel(const SigMode* __restrict__ grp,
+                                                             const SigModeTile* __restrict__ runs, int nrun, int G,
+                                                             const SigModeRank* __restrict__ rank,
+                                                             const int* __restrict__ perm, const cd* __restrict__ as,
+                                                             const cd* __restrict__ zmel,
+                                                             const double* __restrict__ gms, int n, int nw1,
+                                                             cd* __restrict__ cz) {
+  __shared__ D6Smem s;
+  const int p = blockIdx.x, x = p & 7, j = p >> 3, NR = (n + D6M - 1) / D6M;
+  const int sigma = (j / G) * 8 + x, loc = j % G;
+  if (sigma >= nrun * NR) return;
+  const SigModeTile t = runs[sigma / NR];
+  if (loc >= t.cnt) return;
+  const SigMode g = grp[t.grp];
+  const int NS = (n + D6K - 1) / D6K, NK = NS * D6K;
+  const int c0 = (t.ct0 + loc) * D6N, m0 = (sigma % NR) * D6M;
+  const int R = __builtin_amdgcn_readfirstlane(rank[t.grp].rank);
+  const int* pm = perm + g.cbase + c0;
+  const double* gm = gms + g.cbase * nw1 + c0;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  typedef D6Ld<D6M, false> LA;
+  typedef D6Ld<D6N, true> LB;
+  static_assert(D6M == QBM, "row tiles are counted in QBM");
+  static_assert(LB::NI == 1, "one load of B per wave and stage");
+  LA la;
+  la.init(as + g.wbase + (int64_t)rank[t.grp].poff * n * NK, n, m0, n, wave, lane);
+  // B: the lane's column (padding columns take column 0 with weight 0) and k
+  const int bx = wave * 8 + (lane >> 3), bk = (lane & 7) ^ (bx & 7);
+  const cd* bp = zmel + g.zsrc + (int64_t)n * max(pm[bx], 0);
+  int ir = 0, iks = 0;  // the next stage to issue
+  auto issue = [&](int buf) {
+    la.issue(s.a[buf], wave, (ir * NS + iks) * D6K, R * NK);
+    __builtin_amdgcn_global_load_lds((gbl_ptr_t)(bp + min(iks * D6K + bk, n - 1)), (lds_ptr_t)(s.b[buf] + wave * 64),
+                                     16, 0, 0);
+    if (iks + 1 < NS) ++iks;
+    else if (ir + 1 < R) iks = 0, ++ir;
+  };
+  D6Acc c;
+  c.zero();
+  issue(0);
+  issue(1);
+  int buf = 0;
+  for (int r = 0; r < R; ++r) {
+    double w[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) w[q] = gm[(int64_t)r * g.ncp + wn * 32 + q * 16 + (lane & 15)];
+    for (int ks = 0; ks < NS; ++ks) {
+      d6_wait<LA::NI + 1>();
+      issue(buf == 0 ? 2 : buf - 1);
+      d6_stage<LA, LB, false, true>(c, s.a[buf], s.b[buf], wm, wn, lane, 1.0, 1.0, w, D6K);
+      buf = buf == 2 ? 0 : buf + 1;
+    }
+  }
+  ECALJ_WAIT_VMCNT(0);  // the repeated stages have landed before the block's LDS is released
+#pragma unroll
+  for (int jj = 0; jj < 2; ++jj) {
+    const int col = pm[wn * 32 + jj * 16 + (lane & 15)];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        __builtin_amdgcn_sched_barrier(0);  // (one address at a time)
+        const int I = m0 + wm * 32 + i * 16 + acc_row_f64(lane, e);
+        if (I < n && col >= 0) cz[g.zsrc + I + (int64_t)n * col] = cd{c.cr[i][jj][e], c.ci[i][jj][e]};
+      }
+  }
+}
+
 // ---------------------------------------------------------------- host
 // Column tiles of the groups of one sort of T tiles: sqrt(f T) equal groups,
-// about the least of rank sum x tiles + 1/f.. tiles per mode.  bf16x3, f = 1.6:
+// about the least of rank sum x tiles + the modes' cost.  bf16x3, f = 1.6:
 // a mode costs about 1.5 tiles at one rank (23 tiles: 6 groups, 90 tiles: 12);
-// FP64 / FP32 on 64-column tiles, f = 3.5: about 0.3 (45 tiles: 13 groups).
+// FP64 / FP32 on 64-column tiles, f = 2.2: about 0.5 (45 tiles: 10 groups).
 constexpr int kModeGroups = 16;
 static int mode_group_tiles(int T, double f) {
   const int G = std::max(1, std::min(kModeGroups, (int)(std::sqrt(f * T) + 0.5)));
@@ -612,7 +689,7 @@ static int64_t mode_planes_max(int mode, int nw1) {
   return (int64_t)nw1 * (mode == M64 ? mode_pool_planes<double>() : mode_pool_planes<float>());
 }
 static int64_t mode_pool(int mode, int n, int nw1) {
-  return mode_planes_max(mode, nw1) * (mode == MBF3 ? (int64_t)sig3m_a_elems_per_k(n, 1) : (int64_t)n * n);
+  return mode_planes_max(mode, nw1) * (mode == MBF3 ? (int64_t)sig3m_a_elems_per_k(n, 1) : (int64_t)n * ((n + 7) / 8 * 8));
 }
 static size_t mode_pool_elem(int mode) { return mode == MBF3 ? 2 : mode == M64 ? sizeof(cd) : sizeof(cf); }
 
@@ -637,8 +714,8 @@ static ecalj_status sig_modes_t(ecalj_ctx* h, int nk, const int* nm, int ntq, co
                                 const cd* wc, int64_t ldw, int64_t w_stride, const double* wgt, T* cz,
                                 unsigned char* scratch) {
   constexpr int BN = MODE == MBF3 ? Q3BN : 64;
-  constexpr double GF = MODE == MBF3 ? 1.6 : 3.5;
-  const int MP = pad_to(n, QBM), NP = pad_to(n, QBK), NS = NP / QBK, R = MODE == MBF3 ? MP / QBM : (n + 63) / 64;
+  constexpr double GF = MODE == MBF3 ? 1.6 : 2.2;
+  const int MP = pad_to(n, QBM), NP = pad_to(n, QBK), NS = NP / QBK, R = MODE == M32 ? (n + 63) / 64 : MP / QBM;
   const int64_t pool = mode_pool(MODE, n, nw1);
   std::vector<SigModeSort> sorts;
   std::vector<SigMode> grp;
@@ -757,6 +834,9 @@ static ecalj_status sig_modes_t(ecalj_ctx* h, int nk, const int* nm, int ntq, co
   if constexpr (MODE == MBF3)
     hipLaunchKernelGGL(sig3m_modes_kernel, dim3((unsigned)blocks), dim3(512), 0, h->stream, dg, dr, (int)runs.size(), G,
                        rank, perm, (const unsigned short*)as, zp, gm, n, nw1, MP, NS, NP, cz);
+  else if constexpr (MODE == M64)
+    hipLaunchKernelGGL(mode_gemm64_kernel, dim3((unsigned)blocks), dim3(D6T), 0, h->stream, dg, dr, (int)runs.size(),
+                       G, rank, perm, (const cd*)as, zmel, gm, n, nw1, cz);
   else
     hipLaunchKernelGGL((mode_gemm_kernel<MODE, T>), dim3((unsigned)blocks), dim3(kThreads), 0, h->stream, dg, dr,
                        (int)runs.size(), G, rank, perm, (const T*)as, zmel, gm, n, nw1, cz);
