@@ -30,97 +30,179 @@ __device__ inline float dsilu_f(float z) {
 // ---------------------------------------------------------------- FP32 GEMM
 // C (M x N, row-major ldc) = op(A) op(B):
 //   A(i,k) = TA ? A[k*lda + i] : A[i*lda + k],  B(k,j) = TB ? B[j*ldb + k] : B[k*ldb + j].
-enum MlpEpi { ME_STORE = 0, ME_BIAS = 1, ME_BIAS_SILU = 2, ME_DSILU = 3 };
-constexpr int MT = 64, MK = 16;
+// The training step's products are tiny (256 x 256 x 256 at most in the
+// learned tail): what bounds them is the chain of loads, not the flops.  A
+// block takes a 32 x 32 tile with its k dealt out to 8 waves in chunks of 16,
+// operands go straight from memory to the MFMA lanes (the next chunk in
+// flight), and the waves' sums meet in LDS in a fixed order.  A 64 x 64 tile
+// that staged 16 k at a time took 33 us for 256^3 (16 blocks, 16 load round trips).
+enum MlpEpi { ME_STORE = 0, ME_BIAS = 1, ME_BIAS_SILU = 2, ME_DSILU = 3, ME_MSE = 4 };
+constexpr int MT = 64;              // tile of the inference kernel
+constexpr int GT = 32, GW = 8;      // tile and waves of the training kernel
+
+// Lane l, chunk at k0: element e belongs to k = k0 + 4 (l / 16) + e of both
+// operands; MFMA step e takes element e of every lane group, an order of k
+// that A and B share.
+struct MlpGemm {
+  int M, N, K;
+  const float *A, *B;
+  int lda, ldb;
+  float* C;
+  int ldc;
+  const float* bias;   // ME_BIAS, ME_BIAS_SILU, ME_MSE
+  float* Zout;         // ME_BIAS_SILU: z; ME_MSE: dL/dz
+  const float* Zin;    // ME_DSILU: z; ME_MSE: target
+  float* rowsum;       // when set: sum_k A(i,k), the gradient of the bias
+  double* lpart;       // ME_MSE: squared differences of each block; with `loss`: their sum goes there
+  float* loss;
+  int nlpart;
+};
+struct alignas(16) MlpSmem {
+  float red[GW][GT][GT + 1];
+  float rs[GW][GT];
+  double ls[GW];
+};
 
 template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void mlp_gemm_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
-                                                       const float* __restrict__ B, int ldb, float* __restrict__ C,
-                                                       int ldc, const float* __restrict__ bias,
-                                                       float* __restrict__ Zout, const float* __restrict__ Zin) {
-  __shared__ float As[MK][MT + 1];  // As[k][i]
-  __shared__ float Bs[MK][MT + 1];  // Bs[k][j]
-  const int i0 = blockIdx.y * MT, j0 = blockIdx.x * MT;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave >> 1, wn = wave & 1;
+__device__ __forceinline__ void mlp_tile(MlpSmem& s, const MlpGemm& g, int tile) {
+  const int nj = (g.N + GT - 1) / GT;
+  const int i0 = tile / nj * GT, j0 = tile % nj * GT;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, r = lane & 15, kg = 4 * (lane >> 4);
+  const bool sums = g.rowsum && j0 == 0;
   f4 acc[2][2];
+  float rsum[2] = {0.f, 0.f};
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = f4{0, 0, 0, 0};
-  for (int k0 = 0; k0 < K; k0 += MK) {
+  // 16-byte loads where k is contiguous and rows start 16-byte aligned
+  const bool va = !TA && (((uintptr_t)g.A | (uintptr_t)(4 * g.lda)) & 15) == 0;
+  const bool vb = TB && (((uintptr_t)g.B | (uintptr_t)(4 * g.ldb)) & 15) == 0;
+  auto load = [&](const float* X, int64_t ld, bool kcontig, bool vec, int x, int X1, int k) {
+    f4 v = {0, 0, 0, 0};
+    if (x >= X1) return v;
+    if (kcontig) {
+      const float* p = X + ld * x + k;
+      if (vec && k + 4 <= g.K) return *reinterpret_cast<const f4*>(p);
 #pragma unroll
-    for (int q = 0; q < MT * MK / 256; ++q) {
-      const int e = t + 256 * q;
-      int i, k;
-      if (TA) {
-        i = e % MT;
-        k = e / MT;
-      } else {
-        k = e % MK;
-        i = e / MK;
-      }
-      const int gi = i0 + i, gk = k0 + k;
-      float v = 0.f;
-      if (gi < M && gk < K) v = TA ? A[(int64_t)gk * lda + gi] : A[(int64_t)gi * lda + gk];
-      As[k][i] = v;
-      int j, kb;
-      if (TB) {
-        kb = e % MK;
-        j = e / MK;
-      } else {
-        j = e % MT;
-        kb = e / MT;
-      }
-      const int gj = j0 + j, gkb = k0 + kb;
-      float w = 0.f;
-      if (gj < N && gkb < K) w = TB ? B[(int64_t)gj * ldb + gkb] : B[(int64_t)gkb * ldb + gj];
-      Bs[kb][j] = w;
+      for (int e = 0; e < 4; ++e)
+        if (k + e < g.K) v[e] = p[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (k + e < g.K) v[e] = X[ld * (k + e) + x];
     }
-    __syncthreads();
+    return v;
+  };
+  f4 fa[2], fb[2];
+  auto fetch = [&](int k0) {
 #pragma unroll
-    for (int kk = 0; kk < MK; kk += 4) {
-      float av[2], bv[2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) av[a] = As[kk + (lane >> 4)][wm * 32 + a * 16 + (lane & 15)];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) bv[b] = Bs[kk + (lane >> 4)][wn * 32 + b * 16 + (lane & 15)];
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a], bv[b], acc[a][b], 0, 0, 0);
+    for (int q = 0; q < 2; ++q) {
+      fa[q] = load(g.A, g.lda, !TA, va, i0 + 16 * q + r, g.M, k0 + kg);
+      fb[q] = load(g.B, g.ldb, TB, vb, j0 + 16 * q + r, g.N, k0 + kg);
     }
-    __syncthreads();
+  };
+  fetch(16 * wave);
+  for (int k0 = 16 * wave; k0 < g.K; k0 += 16 * GW) {
+    const f4 a0 = fa[0], a1 = fa[1], b0 = fb[0], b1 = fb[1];
+    if (k0 + 16 * GW < g.K) fetch(k0 + 16 * GW);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[e], b0[e], acc[0][0], 0, 0, 0);
+      acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[e], b1[e], acc[0][1], 0, 0, 0);
+      acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[e], b0[e], acc[1][0], 0, 0, 0);
+      acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[e], b1[e], acc[1][1], 0, 0, 0);
+    }
+    if (sums) {
+      rsum[0] += (a0[0] + a0[1]) + (a0[2] + a0[3]);
+      rsum[1] += (a1[0] + a1[1]) + (a1[2] + a1[3]);
+    }
   }
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = i0 + wm * 32 + a * 16 + acc_row_f32(lane, v);
-        const int j = j0 + wn * 32 + b * 16 + (lane & 15);
-        if (i >= M || j >= N) continue;
-        const int64_t o = (int64_t)i * ldc + j;
-        float z = acc[a][b][v];
-        if (EPI == ME_BIAS || EPI == ME_BIAS_SILU) z += bias[j];
-        if (EPI == ME_BIAS_SILU) {
-          Zout[o] = z;
-          z = silu_f(z);
-        }
-        if (EPI == ME_DSILU) z *= dsilu_f(Zin[o]);
-        C[o] = z;
-      }
+      for (int v = 0; v < 4; ++v) s.red[wave][a * 16 + acc_row_f32(lane, v)][b * 16 + r] = acc[a][b][v];
+  if (sums) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      float x = rsum[q];
+      x += __shfl_xor(x, 16);
+      x += __shfl_xor(x, 32);
+      if (lane < 16) s.rs[wave][16 * q + lane] = x;
+    }
+  }
+  __syncthreads();
+  double sq = 0.0;
+#pragma unroll
+  for (int q = 0; q < GT * GT / (64 * GW); ++q) {
+    const int e = t + 64 * GW * q, ii = e / GT, jj = e % GT, i = i0 + ii, j = j0 + jj;
+    float z = 0.f;
+#pragma unroll
+    for (int w = 0; w < GW; ++w) z += s.red[w][ii][jj];
+    if (i >= g.M || j >= g.N) continue;
+    const int64_t o = (int64_t)i * g.ldc + j;
+    if (EPI == ME_BIAS || EPI == ME_BIAS_SILU || EPI == ME_MSE) z += g.bias[j];
+    if (EPI == ME_BIAS_SILU) {
+      g.Zout[o] = z;
+      z = silu_f(z);
+    }
+    if (EPI == ME_DSILU) z *= dsilu_f(g.Zin[o]);
+    if (EPI == ME_MSE) {  // dY = 2 (Y - T) / (B d)
+      const float d = z - g.Zin[o];
+      g.Zout[o] = (float)(2.0 * d * (1.0 / ((double)g.M * g.N)));
+      sq += (double)d * d;
+    } else {
+      g.C[o] = z;
+    }
+  }
+  if (sums && t < GT && i0 + t < g.M) {
+    float x = 0.f;
+#pragma unroll
+    for (int w = 0; w < GW; ++w) x += s.rs[w][t];
+    g.rowsum[i0 + t] = x;
+  }
+  // sums over the block in a fixed order: this tile's squares, or (the kernel
+  // after, its first block) those of all tiles into the loss
+  const bool fin = g.loss && EPI != ME_MSE && tile == 0;
+  if (EPI == ME_MSE || fin) {
+    if (fin)
+      for (int q = t; q < g.nlpart; q += 64 * GW) sq += g.lpart[q];
+    for (int o = 32; o > 0; o >>= 1) sq += __shfl_down(sq, o);
+    if (lane == 0) s.ls[wave] = sq;
+    __syncthreads();
+    if (t == 0) {
+      double x = 0.0;
+      for (int w = 0; w < GW; ++w) x += s.ls[w];
+      if (fin) *g.loss = (float)x;
+      else g.lpart[tile] = x * (1.0 / ((double)g.M * g.N));
+    }
+  }
 }
 
 template <bool TA, bool TB, int EPI>
-static ecalj_status mlp_gemm(ecalj_ctx* h, int M, int N, int K, const float* A, int lda, const float* B, int ldb,
-                             float* C, int ldc, const float* bias = nullptr, float* Zout = nullptr,
-                             const float* Zin = nullptr) {
-  if (M <= 0 || N <= 0) return ECALJ_OK;
-  dim3 grid((N + MT - 1) / MT, (M + MT - 1) / MT);
-  if (grid.y > 65535) return ECALJ_ERR_DIM;
-  hipLaunchKernelGGL((mlp_gemm_kernel<TA, TB, EPI>), grid, dim3(256), 0, h->stream, M, N, K, A, lda, B, ldb, C, ldc,
-                     bias, Zout, Zin);
+__global__ __launch_bounds__(64 * GW) void mlp_gemm_kernel(MlpGemm g) {
+  __shared__ MlpSmem s;
+  mlp_tile<TA, TB, EPI>(s, g, blockIdx.x);
+}
+
+// Backward of one layer in one launch: the first nw blocks form dW = dZ^T H
+// (and the bias gradient), the others dZ of the layer before.
+__global__ __launch_bounds__(64 * GW) void mlp_backward_kernel(MlpGemm gw, int nw, MlpGemm gz) {
+  __shared__ MlpSmem s;
+  if ((int)blockIdx.x < nw) mlp_tile<true, false, ME_STORE>(s, gw, blockIdx.x);
+  else mlp_tile<false, false, ME_DSILU>(s, gz, blockIdx.x - nw);
+}
+
+static int64_t mlp_tiles(int M, int N) { return (int64_t)((M + GT - 1) / GT) * ((N + GT - 1) / GT); }
+
+template <bool TA, bool TB, int EPI>
+static ecalj_status mlp_gemm(ecalj_ctx* h, const MlpGemm& g) {
+  if (g.M <= 0 || g.N <= 0) return ECALJ_OK;
+  const int64_t tiles = mlp_tiles(g.M, g.N);
+  if ((g.M + MT - 1) / MT > 65535 || tiles > 0x7fffffff) return ECALJ_ERR_DIM;
+  hipLaunchKernelGGL((mlp_gemm_kernel<TA, TB, EPI>), dim3((unsigned)tiles), dim3(64 * GW), 0, h->stream, g);
   ECALJ_HIP(hipGetLastError());
   return ECALJ_OK;
 }
@@ -210,35 +292,6 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(int M, int N, int K, con
 }
 
 // ---------------------------------------------------------------- small kernels
-// dY = 2 (Y - T) / (B d); loss = mean (Y - T)^2, reduced in a fixed order (one block)
-__global__ __launch_bounds__(256) void mse_kernel(const float* __restrict__ y, const float* __restrict__ tg,
-                                                  int64_t n, float* __restrict__ dy, float* __restrict__ loss) {
-  __shared__ double red[256];
-  const double nrm = 1.0 / (double)n;
-  double s = 0.0;
-  for (int64_t e = threadIdx.x; e < n; e += 256) {
-    const float d = y[e] - tg[e];
-    dy[e] = (float)(2.0 * d * nrm);
-    s += (double)d * d;
-  }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0 && loss) *loss = (float)(red[0] * nrm);
-}
-
-// db[j] = sum_i dz[i*ld + j], fixed order
-__global__ void colsum_kernel(const float* __restrict__ dz, int rows, int cols, int ld, float* __restrict__ db) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= cols) return;
-  float s = 0.f;
-  for (int i = 0; i < rows; ++i) s += dz[(int64_t)i * ld + j];
-  db[j] = s;
-}
-
 __global__ void adam_kernel(int64_t n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
                             float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
@@ -361,16 +414,23 @@ ecalj_status ecalj_mlp_nparam(int nlayer, const int* dims, int64_t* nparam) {
   return ECALJ_OK;
 }
 
-// workspace: Z_l and H_{l+1} per layer (B x d[l+1] floats each), then dZ ping-pong (2 x B x maxw)
-static ecalj_status mlp_work(ecalj_ctx* h, const NetShape& s, int batch, float** w) {
+// workspace: Z_l and H_{l+1} per layer (B x d[l+1] floats each), then dZ
+// ping-pong (2 x B x maxw) and the loss partials (one double per output tile)
+static int64_t mlp_floats(const NetShape& s, int batch) {
   int64_t n = 0;
   for (int l = 0; l < s.L; ++l) n += 2LL * batch * s.d[l + 1];
-  n += 2LL * batch * s.maxw;
+  return (n + 2LL * batch * s.maxw + 1) / 2 * 2;
+}
+static ecalj_status mlp_work(ecalj_ctx* h, const NetShape& s, int batch, float** w) {
+  const int64_t n = mlp_floats(s, batch) + 2 * mlp_tiles(batch, s.d[s.L]);
   return slot_ensure(h, ecalj_ctx::S_MLP, sizeof(float) * (size_t)n, (void**)w);
 }
 
+// target != nullptr: the last layer writes dL/dy of the mean squared error to
+// dy and its tiles' shares of the loss to lpart (y itself is not needed).
 static ecalj_status mlp_forward_ws(ecalj_ctx* h, const NetShape& s, const float* p, const float* x, int B,
-                                   float* ws, float* y, std::vector<const float*>* Hs, std::vector<float*>* Zs) {
+                                   float* ws, float* y, std::vector<const float*>* Hs, std::vector<float*>* Zs,
+                                   const float* target = nullptr, float* dy = nullptr, double* lpart = nullptr) {
   const float* hin = x;
   float* cur = ws;
   for (int l = 0; l < s.L; ++l) {
@@ -382,11 +442,25 @@ static ecalj_status mlp_forward_ws(ecalj_ctx* h, const NetShape& s, const float*
     cur += 2LL * B * dout;
     if (Hs) Hs->push_back(hin);
     if (Zs) Zs->push_back(Z);
+    MlpGemm g{};
+    g.M = B; g.N = dout; g.K = din;
+    g.A = hin; g.lda = din;
+    g.B = W; g.ldb = din;
+    g.ldc = dout;
+    g.bias = b;
     if (l < s.L - 1) {
-      ECALJ_TRY((mlp_gemm<false, true, ME_BIAS_SILU>(h, B, dout, din, hin, din, W, din, H, dout, b, Z)));
+      g.C = H;
+      g.Zout = Z;
+      ECALJ_TRY((mlp_gemm<false, true, ME_BIAS_SILU>(h, g)));
       hin = H;
+    } else if (target) {
+      g.Zin = target;
+      g.Zout = dy;
+      g.lpart = lpart;
+      ECALJ_TRY((mlp_gemm<false, true, ME_MSE>(h, g)));
     } else {
-      ECALJ_TRY((mlp_gemm<false, true, ME_BIAS>(h, B, dout, din, hin, din, W, din, y ? y : Z, dout, b)));
+      g.C = y;
+      ECALJ_TRY((mlp_gemm<false, true, ME_BIAS>(h, g)));
     }
   }
   return ECALJ_OK;
@@ -417,29 +491,40 @@ ecalj_status ecalj_mlp_grad_dev(ecalj_handle h, int nlayer, const int* dims, con
   float* g = (float*)grad;
   std::vector<const float*> Hs;
   std::vector<float*> Zs;
-  ECALJ_TRY(mlp_forward_ws(h, s, p, (const float*)x, B, ws, nullptr, &Hs, &Zs));
   int64_t used = 0;
   for (int l = 0; l < s.L; ++l) used += 2LL * B * s.d[l + 1];
   float* dz = ws + used;
   float* dz2 = dz + (int64_t)B * s.maxw;
-  const int dL = s.d[s.L];
-  hipLaunchKernelGGL(mse_kernel, dim3(1), dim3(256), 0, h->stream, Zs[s.L - 1], (const float*)target,
-                     (int64_t)B * dL, dz, (float*)loss);
-  ECALJ_HIP(hipGetLastError());
+  double* lpart = (double*)(ws + mlp_floats(s, B));
+  ECALJ_TRY(mlp_forward_ws(h, s, p, (const float*)x, B, ws, nullptr, &Hs, &Zs, (const float*)target, dz, lpart));
   for (int l = s.L - 1; l >= 0; --l) {
     const int din = s.d[l], dout = s.d[l + 1];
-    const float* W = p + s.off[l];
-    float* gW = g + s.off[l];
-    float* gb = gW + (int64_t)dout * din;
-    // dW = dZ^T H  (dout x din)
-    ECALJ_TRY((mlp_gemm<true, false, ME_STORE>(h, dout, din, B, dz, dout, Hs[l], din, gW, din)));
-    hipLaunchKernelGGL(colsum_kernel, dim3((dout + 127) / 128), dim3(128), 0, h->stream, dz, B, dout, dout, gb);
-    ECALJ_HIP(hipGetLastError());
-    if (l > 0) {  // dZ_{l-1} = (dZ W) * silu'(Z_{l-1})
-      ECALJ_TRY((mlp_gemm<false, false, ME_DSILU>(h, B, din, dout, dz, dout, W, din, dz2, din, nullptr, nullptr,
-                                                  Zs[l - 1])));
-      std::swap(dz, dz2);
+    MlpGemm w{};  // dW = dZ^T H  (dout x din), db = column sums of dZ
+    w.M = dout; w.N = din; w.K = B;
+    w.A = dz; w.lda = dout;
+    w.B = Hs[l]; w.ldb = din;
+    w.C = g + s.off[l]; w.ldc = din;
+    w.rowsum = w.C + (int64_t)dout * din;
+    if (l == s.L - 1) {
+      w.lpart = lpart;
+      w.nlpart = (int)mlp_tiles(B, dout);
+      w.loss = (float*)loss;
     }
+    if (l == 0) {
+      ECALJ_TRY((mlp_gemm<true, false, ME_STORE>(h, w)));
+      break;
+    }
+    MlpGemm z{};  // dZ_{l-1} = (dZ W) * silu'(Z_{l-1})
+    z.M = B; z.N = din; z.K = dout;
+    z.A = dz; z.lda = dout;
+    z.B = p + s.off[l]; z.ldb = din;
+    z.C = dz2; z.ldc = din;
+    z.Zin = Zs[l - 1];
+    const int64_t nw = mlp_tiles(dout, din), nz = mlp_tiles(B, din);
+    if (nw + nz > 0x7fffffff) return ECALJ_ERR_DIM;
+    hipLaunchKernelGGL(mlp_backward_kernel, dim3((unsigned)(nw + nz)), dim3(64 * GW), 0, h->stream, w, (int)nw, z);
+    ECALJ_HIP(hipGetLastError());
+    std::swap(dz, dz2);
   }
   return ECALJ_OK;
 }
