@@ -345,6 +345,7 @@ ecalj_status ecalj_destroy(ecalj_handle h) {
   }
   if (h->d_ppb) (void)hipFree(h->d_ppb);
   if (h->d_ppb2) (void)hipFree(h->d_ppb2);
+  ppb_planes_free(h);
   if (h->d_ppbc) (void)hipFree(h->d_ppbc);
   if (h->d_vcousq) (void)hipFree(h->d_vcousq);
   if (h->d_zcousq) (void)hipFree(h->d_zcousq);
@@ -581,6 +582,8 @@ ecalj_status ecalj_dev_phase_similarity(ecalj_handle h, const void* a, int ngb, 
 // ------------------------------------------------------------------ state
 ecalj_status ecalj_set_ppb(ecalj_handle h, int natom, const int* nv, const int* mdim, const double* ppb) {
   if (!h || natom < 1 || !nv || !mdim || !ppb) return ECALJ_ERR_ARG;
+  for (int a = 0; a < natom; ++a)
+    if (nv[a] < 0 || mdim[a] < 0) return ECALJ_ERR_DIM;  // before any state changes
   int64_t tot = 0;
   h->nv.assign(nv, nv + natom);
   h->mdim.assign(mdim, mdim + natom);
@@ -588,7 +591,6 @@ ecalj_status ecalj_set_ppb(ecalj_handle h, int natom, const int* nv, const int* 
   h->ndima_used = 0;
   h->ngb_ppb = 0;
   for (int a = 0; a < natom; ++a) {
-    if (nv[a] < 0 || mdim[a] < 0) return ECALJ_ERR_DIM;
     h->ppb_off[a] = tot;
     tot += (int64_t)nv[a] * nv[a] * mdim[a];
     h->ndima_used += nv[a];
@@ -603,6 +605,7 @@ ecalj_status ecalj_set_ppb(ecalj_handle h, int natom, const int* nv, const int* 
   h->d_ppbc = nullptr;
   if (h->d_ppb) (void)hipFree(h->d_ppb);
   if (h->d_ppb2) (void)hipFree(h->d_ppb2);
+  ppb_planes_free(h);
   h->d_ppb = h->d_ppb2 = nullptr;
   const size_t bytes = sizeof(double) * std::max<int64_t>(tot, 1);
   if (hipMalloc(&h->d_ppb, bytes) != hipSuccess) return ECALJ_ERR_NOMEM;
@@ -809,9 +812,8 @@ static ecalj_status zmel_impl(ecalj_ctx* h, const double* phase, int ndima, int 
           g.batch = bm; g.div = bm;
         }
         if (mode == ECALJ_PREC_BF16X3)
-          ECALJ_TRY(zmel_p_bf3(h, (int)nvmd, g.N, nv, h->d_ppb2 + h->ppb_off[ap], nvmd,
-                               (const ecalj::cf*)cphim + ias, ndima, g.batch > 1 ? sm : 0, true, (ecalj::cf*)T, nvmd,
-                               g.batch > 1 ? nvmd * nm : 0, g.batch));
+          ECALJ_TRY(zmel_p_bf3(h, ap, g.N, (const ecalj::cf*)cphim + ias, ndima, g.batch > 1 ? sm : 0, true,
+                               (ecalj::cf*)T, g.batch > 1 ? nvmd * nm : 0, g.batch));
         else
           ECALJ_TRY(gemm(h, g));
         GemmCall z;  // per (n,k): zmel(ims+I, voff+n, m) = phase * sum_b T[b + nv*I + nvmd*(n + nm*k)] cphiq_k(ias+b, m)

@@ -43,8 +43,8 @@ struct alignas(16) SigSmem {
 // (A: 4 planes of MP x QBK per (v, ks); B: 4 planes of NCP x QBK per ks).
 // NW = 8 puts two waves on every SIMD: one wave alone issues a 16x16x32
 // bf16 MFMA only every ~30 cycles, two interleave to ~20.
-// AREAL: the A operand is real (its imaginary planes are zero and are not
-// multiplied): 6 MFMAs per 16x16 tile and k slice instead of 12.
+// AREAL: the A operand is real and has two planes (hi, lo) instead of four: 6
+// MFMAs per 16x16 tile and k slice instead of 12.
 template <int BN, int NSTG, int NW, bool AREAL = false>
 __device__ __forceinline__ void sig_tile(SigSmem<BN, NSTG>& s, const unsigned short* __restrict__ Ak,
                                          const unsigned short* __restrict__ Bk, const double* __restrict__ g,
@@ -55,9 +55,10 @@ __device__ __forceinline__ void sig_tile(SigSmem<BN, NSTG>& s, const unsigned sh
   static_assert(NW == 4 || NW == 8, "four or eight waves");
   constexpr int NT = NW * 64, WN = NW / 2;
   constexpr int TM = 4, TN = BN / (16 * WN);          // 16x16 tiles per wave
-  constexpr int ARW = 4 * QBM * QBK * 2 / 1024 / NW;  // 1 KB A runs per wave and stage
+  constexpr int APL = AREAL ? 2 : 4;                  // A planes
+  constexpr int ARW = APL * QBM * QBK * 2 / 1024 / NW;  // 1 KB A runs per wave and stage
   constexpr int BRW = 4 * BN * QBK * 2 / 1024 / NW;   // 1 KB B runs per wave and stage
-  static_assert(TN >= 1 && ARW * NW == 4 * QBM * QBK * 2 / 1024 && BRW * NW == 4 * BN * QBK * 2 / 1024,
+  static_assert(TN >= 1 && ARW * NW == APL * QBM * QBK * 2 / 1024 && BRW * NW == 4 * BN * QBK * 2 / 1024,
                 "runs split evenly over the waves");
   constexpr int APP = QBM * QBK / 512, BPP = BN * QBK / 512;  // runs per plane
   const int t = threadIdx.x, lane = t & 63;
@@ -79,7 +80,7 @@ __device__ __forceinline__ void sig_tile(SigSmem<BN, NSTG>& s, const unsigned sh
 
   auto issue = [&](int st, int buf) {
     const int v = v0 + st / NS, ks = st % NS;
-    const unsigned short* a = A + ((int64_t)v * NS + ks) * 4 * apst;
+    const unsigned short* a = A + ((int64_t)v * NS + ks) * APL * apst;
     const unsigned short* bb = B + (int64_t)ks * 4 * bpst;
 #pragma unroll
     for (int q = 0; q < ARW; ++q) {

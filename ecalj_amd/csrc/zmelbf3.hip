@@ -119,7 +119,7 @@ ecalj_status zmel_z_bf3(ecalj_ctx* h, int M, int N, int K, const cf* A, int64_t 
 // X complex64 K-contiguous (X[k + ldb c], conjugated when conjB), per batch b
 // X_b = X + b x_s1, T_b = C + b c_s1; P shared by all batches.
 
-// real rows -> planes (imaginary planes zero); one thread per (ks, chunk, row), row fastest
+// real rows -> two planes (hi, lo); one thread per (ks, chunk, row), row fastest
 __global__ __launch_bounds__(256) void rsplit_kernel(const double* __restrict__ a, int64_t lda, int rows, int K,
                                                      int RP, int NS, unsigned short* __restrict__ dst) {
   typedef unsigned short us8v __attribute__((ext_vector_type(8)));
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void rsplit_kernel(const double* __restrict__ 
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot; e += (int64_t)gridDim.x * blockDim.x) {
     const int row = (int)(e % RP);
     const int ch = (int)((e / RP) % 4), ks = (int)(e / (4 * (int64_t)RP));
-    us8v rh, rl, z;
+    us8v rh, rl;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       const int kk = ks * QBK + 8 * ch + q;
@@ -137,13 +137,10 @@ __global__ __launch_bounds__(256) void rsplit_kernel(const double* __restrict__ 
       split_bf16(x, h, l);
       rh[q] = h;
       rl[q] = l;
-      z[q] = 0;
     }
-    unsigned short* D = dst + (int64_t)ks * 4 * pst + (int64_t)row * QBK + 8 * chunk_slot(row, ch);
+    unsigned short* D = dst + (int64_t)ks * 2 * pst + (int64_t)row * QBK + 8 * chunk_slot(row, ch);
     *reinterpret_cast<us8v*>(D) = rh;
     *reinterpret_cast<us8v*>(D + pst) = rl;
-    *reinterpret_cast<us8v*>(D + 2 * pst) = z;
-    *reinterpret_cast<us8v*>(D + 3 * pst) = z;
   }
 }
 
@@ -157,26 +154,75 @@ __global__ __launch_bounds__(512, 1) void zmel_p_kernel(const unsigned short* __
                             C + c_s1 * b, 0, ldc);
 }
 
-ecalj_status zmel_p_bf3(ecalj_ctx* h, int M, int N, int K, const double* P, int64_t lda, const cf* X,
-                        int64_t ldb, int64_t x_s1, bool conjB, cf* C, int64_t ldc, int64_t c_s1, int batch) {
+static int64_t ppb_plane_elems(const ecalj_ctx* h, int a) {
+  const int64_t nvmd = (int64_t)h->nv[a] * h->mdim[a];
+  return 2 * (nvmd + QBM - 1) / QBM * QBM * pad_to(h->nv[a], QBK);
+}
+
+// bf16 planes of atom a's ppb (the relaid copy): a weight of every zmel call
+// until the next set_ppb, so the split (0.98 ms at C3, more than either GEMM)
+// runs once per atom and is kept, 4 bytes per element of ppb.  The build is
+// waited for, so that calls on another stream find it complete.  Without room
+// for it, or under capture before it was built, *out stays null.
+static ecalj_status ppb_planes(ecalj_ctx* h, int a, const unsigned short** out) {
+  *out = nullptr;
+  const int nv = h->nv[a];
+  const int64_t nvmd = (int64_t)nv * h->mdim[a], el = ppb_plane_elems(h, a);
+  if (nvmd > 0x7fffffff - QBM) return ECALJ_ERR_DIM;
+  if (h->ppb_pl.size() != h->nv.size()) h->ppb_pl.assign(h->nv.size(), nullptr);
+  if (!h->ppb_pl[a]) {
+    if (h->capturing) return ECALJ_OK;
+    void* p = nullptr;
+    if (hipMalloc(&p, sizeof(unsigned short) * (size_t)el) != hipSuccess) {
+      (void)hipGetLastError();
+      return ECALJ_OK;
+    }
+    h->ppb_pl[a] = (unsigned short*)p;
+    const int MP = pad_to((int)nvmd, QBM), NS = pad_to(nv, QBK) / QBK;
+    const int64_t tot = (int64_t)NS * 4 * MP;
+    hipLaunchKernelGGL(rsplit_kernel, dim3((unsigned)std::min<int64_t>((tot + 255) / 256, 65536 * 4)), dim3(256), 0,
+                       h->stream, h->d_ppb2 + h->ppb_off[a], nvmd, (int)nvmd, nv, MP, NS, h->ppb_pl[a]);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(h->stream) != hipSuccess) {
+      (void)hipFree(p);
+      h->ppb_pl[a] = nullptr;
+      return ECALJ_ERR_HIP;
+    }
+  }
+  *out = h->ppb_pl[a];
+  return ECALJ_OK;
+}
+
+void ppb_planes_free(ecalj_ctx* h) {
+  for (unsigned short* p : h->ppb_pl)
+    if (p) (void)hipFree(p);
+  h->ppb_pl.clear();
+}
+
+ecalj_status zmel_p_bf3(ecalj_ctx* h, int a, int N, const cf* X, int64_t ldb, int64_t x_s1, bool conjB, cf* C,
+                        int64_t c_s1, int batch) {
+  const int K = h->nv[a], M = (int)((int64_t)K * h->mdim[a]);
+  const int64_t lda = M, ldc = M;
   if (M < 1 || N < 1 || batch < 1) return ECALJ_OK;
   if (K < 1 || batch > 65535) return ECALJ_ERR_DIM;
   const int MP = pad_to(M, QBM), NCP = pad_to(N, 128), NS = pad_to(K, QBK) / QBK;
-  if ((int64_t)MP / QBM > 0x7fffffff) return ECALJ_ERR_DIM;
-  const int64_t ape = 4LL * NS * MP * QBK, bpe = 4LL * NS * NCP * QBK;
-  unsigned short *as, *bs;
-  ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_ZPA, sizeof(unsigned short) * (size_t)ape, (void**)&as));
+  const int64_t bpe = 4LL * NS * NCP * QBK;
+  const unsigned short* as;
+  unsigned short* bs;
+  ECALJ_TRY(ppb_planes(h, a, &as));
+  if (!as) {  // split for this call
+    unsigned short* sp;
+    ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_ZPA, sizeof(unsigned short) * (size_t)ppb_plane_elems(h, a), (void**)&sp));
+    const int64_t tot = (int64_t)NS * 4 * MP;
+    hipLaunchKernelGGL(rsplit_kernel, dim3((unsigned)std::min<int64_t>((tot + 255) / 256, 65536 * 4)), dim3(256), 0,
+                       h->stream, h->d_ppb2 + h->ppb_off[a], lda, M, K, MP, NS, sp);
+    ECALJ_HIP(hipGetLastError());
+    as = sp;
+  }
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_ZPB, sizeof(unsigned short) * (size_t)bpe * batch + sizeof(double) * NCP,
                         (void**)&bs));
   double* ones = reinterpret_cast<double*>(bs + (size_t)bpe * batch);
   hipLaunchKernelGGL(ones_kernel, dim3((NCP + 255) / 256), dim3(256), 0, h->stream, ones, NCP);
   ECALJ_HIP(hipGetLastError());
-  {
-    const int64_t tot = (int64_t)NS * 4 * MP;
-    const int blocks = (int)std::min<int64_t>((tot + 255) / 256, 65536 * 4);
-    hipLaunchKernelGGL(rsplit_kernel, dim3(blocks), dim3(256), 0, h->stream, P, lda, M, K, MP, NS, as);
-    ECALJ_HIP(hipGetLastError());
-  }
   {
     const int64_t tot = (int64_t)NS * NCP * 4 * batch;
     const int blocks = (int)std::min<int64_t>((tot + 255) / 256, 65536 * 4);
