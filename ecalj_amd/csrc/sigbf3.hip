@@ -576,6 +576,11 @@ __global__ __launch_bounds__(256) void split_b_kernel(const TIN* __restrict__ bm
   }
 }
 
+static __global__ __launch_bounds__(256) void fill_kernel(double* __restrict__ p, int n, double x) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = x;
+}
+
 template <class TIN>
 static ecalj_status split_a(ecalj_ctx* h, const void* a, int64_t lda, int64_t a_stride, int m, int k, bool herm,
                             int MP, int NS, unsigned short* as, int64_t as_stride, int nb) {
@@ -610,11 +615,11 @@ ecalj_status qgemm_bf3(ecalj_ctx* h, int nb, int m, int ncol, int k, const QOper
   double* w;
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_QA, sizeof(unsigned short) * (size_t)ape * na, (void**)&as));
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_QB, sizeof(unsigned short) * (size_t)bpe * nbb, (void**)&bs));
-  std::vector<unsigned char> wb(sizeof(double) * (size_t)ncol);
-  for (int c = 0; c < ncol; ++c) std::memcpy(wb.data() + sizeof(double) * c, &alpha, sizeof(double));
-  unsigned char* dw = nullptr;
-  ECALJ_TRY(upload_blob(h, ecalj_ctx::S_QW, wb, &dw));
-  w = (double*)dw;
+  // the weights by a fill: an upload through pinned staging waits for the one
+  // before it, which held the host back to the GPU four times per W build
+  ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_QW, sizeof(double) * (size_t)ncol, (void**)&w));
+  hipLaunchKernelGGL(fill_kernel, dim3((ncol + 255) / 256), dim3(256), 0, h->stream, w, ncol, alpha);
+  ECALJ_HIP(hipGetLastError());
   if (A.wide) ECALJ_TRY(split_a<cd>(h, A.p, A.ld, A.stride, m, k, A.herm, MP, NS, as, ape, na));
   else ECALJ_TRY(split_a<cf>(h, A.p, A.ld, A.stride, m, k, A.herm, MP, NS, as, ape, na));
   if (B.wide) ECALJ_TRY(split_b<cd>(h, B.p, B.ld, B.stride, k, ncol, B.herm, NCP, NS, bs, bpe, nbb));
