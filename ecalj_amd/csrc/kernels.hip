@@ -218,101 +218,161 @@ ecalj_status x0_herk(ecalj_ctx* h, int mode, const void* z, const int64_t* d_col
 //   out(e, v) = i dscale(v0+v) rcxq(e, v0+v) + sum_iw coef(v, iw) rcxq(e, iw)
 //                                                              (real axis, dscale != null)
 // for the output chunk v in [v0, v0+nv); coef(v, iw) = coef[v + ldc*(iw-1)]
-// (chunk base already applied), zero-padded so that NV coefficients can be
-// read for every chunk: the FMA loop runs over all NV outputs without a
-// per-output test.  FP64 accumulation, complex128 output; rcxq complex128
-// or complex64.  With `scale`, rcxq(:, iw) *= scale(iw) is stored back (the
-// reference scales rcxq in place once).
-template <int NV, class T>
-__global__ __launch_bounds__(256) void hilbert_kernel(T* __restrict__ rcxq, int64_t slice, int nwhis,
-                                                      int nv, int ldc, const double* __restrict__ coef,
-                                                      const double* __restrict__ scale, int v0,
-                                                      const double* __restrict__ dscale,
-                                                      cd* __restrict__ out, int64_t n) {
-  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  double ar[NV], ai[NV];
-#pragma unroll
-  for (int v = 0; v < NV; ++v) { ar[v] = 0.0; ai[v] = 0.0; }
-  // four bins per round: their loads are issued before any store-back, so
-  // four reads of rcxq per lane are in flight (the loop is latency bound)
-  int iw = 1;
-  for (; iw + 3 <= nwhis; iw += 4) {
-    double xr[4], xi[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) ld_c2(rcxq + e + slice * (iw + u), xr[u], xi[u]);
-    if (scale) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const double s = scale[iw + u - 1];
-        st_c(rcxq + e + slice * (iw + u), s * xr[u], s * xi[u]);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const double* c = coef + (int64_t)ldc * (iw + u - 1);
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        ar[v] += c[v] * xr[u];
-        ai[v] += c[v] * xi[u];
-      }
-    }
-  }
-  for (; iw <= nwhis; ++iw) {
-    double xr, xi;
-    ld_c2(rcxq + e + slice * iw, xr, xi);
-    if (scale) {
-      const double s = scale[iw - 1];
-      st_c(rcxq + e + slice * iw, s * xr, s * xi);
-    }
-    const double* c = coef + (int64_t)ldc * (iw - 1);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      ar[v] += c[v] * xr;
-      ai[v] += c[v] * xi;
-    }
-  }
-  if (dscale) {  // i*dscale*rcxq(:, it): slot it of rcxq is the bin centred at freq_r(it); slot 0 the zero frequency
-#pragma unroll
-    for (int v = 0; v < NV; ++v)
-      if (v < nv) {
-        double xr, xi;
-        ld_c2(rcxq + e + slice * (v0 + v), xr, xi);
-        const double s = dscale[v0 + v];
-        ar[v] -= s * xi;
-        ai[v] += s * xr;
-      }
-  }
-#pragma unroll
-  for (int v = 0; v < NV; ++v)
-    if (v < nv) out[e + n * v] = cd{ar[v], ai[v]};
-}
+// (chunk base already applied), zero-padded to a multiple of 32 outputs.  FP64
+// accumulation, complex128 output; rcxq complex128 or complex64.  With
+// `scale`, rcxq(:, iw) *= scale(iw) is stored back (the reference scales rcxq
+// in place once).
+//
+// A (outputs x bins) times (bins x elements) product on the FP64 MFMA: a wave
+// owns 64 elements, lane (j, g) reads elements 4j..4j+3 (one run of 32 or 64
+// bytes) of bin 4 it + g, and element 4j + t is column j of column tile t; the
+// coefficients of 16 outputs are one vector load per 4 bins.  NX further
+// outputs (17 and 21 are usual: nf + 1) are summed in the lanes that hold their
+// bins and added up at the end, which costs NX/16 of a row tile instead of a
+// whole one.  The next round's loads are in flight during this round's
+// products.  One thread per element with scalar coefficient loads, each waited
+// for, took 0.60 ms at C2 (0.86 GB read, 17 outputs), with twice the loads in
+// flight 0.56; this takes 0.22 (3.9 TB/s).
+typedef double d2a8 __attribute__((ext_vector_type(2), aligned(8)));
+typedef float f4a8 __attribute__((ext_vector_type(4), aligned(8)));
 
-template <int NV, class T>
-static void hilbert_launch(ecalj_ctx* h, T* rcxq, int64_t slice, int nwhis, int nv, int ldc, const double* coef,
-                           const double* scale, int v0, const double* dscale, cd* out, int64_t n) {
-  const dim3 grid((unsigned)((n + 255) / 256));
-  hipLaunchKernelGGL((hilbert_kernel<NV, T>), grid, dim3(256), 0, h->stream, rcxq, slice, nwhis, nv, ldc, coef,
-                     scale, v0, dscale, out, n);
+template <int NRT, int NX, int U, class T>
+__global__ __launch_bounds__(256, 2) void hilbert_kernel(T* __restrict__ rcxq, int64_t slice, int nwhis, int nv,
+                                                         int ldc, const double* __restrict__ coef,
+                                                         const double* __restrict__ scale, int v0,
+                                                         const double* __restrict__ dscale, cd* __restrict__ out,
+                                                         int64_t n) {
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+  const int64_t w0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 64, e = w0 + 4 * j;
+  if (w0 >= n) return;
+  const bool full = e + 4 <= n;
+  const int left = full ? 4 : (int)max((int64_t)0, n - e);  // this lane's elements
+  struct V { T x[4]; };
+  auto load = [&](int bin, V& v) {
+    const T* p = rcxq + e + slice * bin;
+    if (full) {
+      if constexpr (sizeof(T) == 8) {
+        const f4a8 a = reinterpret_cast<const f4a8*>(p)[0], b = reinterpret_cast<const f4a8*>(p)[1];
+        v.x[0] = T{a[0], a[1]}, v.x[1] = T{a[2], a[3]}, v.x[2] = T{b[0], b[1]}, v.x[3] = T{b[2], b[3]};
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const d2a8 a = reinterpret_cast<const d2a8*>(p)[t];
+          v.x[t] = T{a[0], a[1]};
+        }
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) v.x[t] = t < left ? p[t] : T{0, 0};
+    }
+  };
+  d4 ar[NRT][4], ai[NRT][4];
+#pragma unroll
+  for (int r = 0; r < NRT; ++r)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) ar[r][t] = ai[r][t] = d4{0, 0, 0, 0};
+  double xr[NX ? NX : 1][4], xi[NX ? NX : 1][4];
+#pragma unroll
+  for (int x = 0; x < NX; ++x)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) xr[x][t] = xi[x][t] = 0.0;
+  const int nit = (nwhis + 3) / 4;
+  V cur[U], nxt[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) load(min(1 + 4 * u + g, nwhis), cur[u]);
+  for (int ib = 0; ib < nit; ib += U) {
+    double ca[U][NRT], cx[U][NX ? NX : 1];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int bin = 1 + 4 * (ib + u) + g;
+      const double* c = coef + (int64_t)ldc * (min(bin, nwhis) - 1);
+      const bool in = bin <= nwhis;  // beyond: zeros
+#pragma unroll
+      for (int r = 0; r < NRT; ++r) ca[u][r] = in ? c[16 * r + j] : 0.0;
+#pragma unroll
+      for (int x = 0; x < NX; ++x) cx[u][x] = in ? c[16 * NRT + x] : 0.0;
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the coefficients' loads go first, then the next round's data
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(min(1 + 4 * (ib + U + u) + g, nwhis), nxt[u]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int bin = 1 + 4 * (ib + u) + g;
+      if (scale && bin <= nwhis) {
+        const double s = scale[bin - 1];
+        T* p = rcxq + e + slice * bin;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (t < left) st_c(p + t, s * cur[u].x[t].re, s * cur[u].x[t].im);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const double re = bin <= nwhis ? cur[u].x[t].re : 0.0, im = bin <= nwhis ? cur[u].x[t].im : 0.0;
+#pragma unroll
+        for (int r = 0; r < NRT; ++r) {
+          ar[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ca[u][r], re, ar[r][t], 0, 0, 0);
+          ai[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ca[u][r], im, ai[r][t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int x = 0; x < NX; ++x) {
+          xr[x][t] += cx[u][x] * re;
+          xi[x][t] += cx[u][x] * im;
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+  }
+  // output v of the lane's element t; on the real axis i*dscale*rcxq(:, it):
+  // slot it of rcxq is the bin centred at freq_r(it), slot 0 the zero frequency
+  auto put = [&](int v, int t, double re, double im) {
+    if (v >= nv || t >= left) return;
+    if (dscale) {
+      const T x = rcxq[e + t + slice * (v0 + v)];
+      const double s = dscale[v0 + v];
+      re -= s * x.im;
+      im += s * x.re;
+    }
+    out[e + t + n * v] = cd{re, im};
+  };
+#pragma unroll
+  for (int r = 0; r < NRT; ++r)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) put(16 * r + acc_row_f64(lane, q), t, ar[r][t][q], ai[r][t][q]);
+#pragma unroll
+  for (int x = 0; x < NX; ++x)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      double re = xr[x][t], im = xi[x][t];
+      re += __shfl_xor(re, 16);
+      im += __shfl_xor(im, 16);
+      re += __shfl_xor(re, 32);
+      im += __shfl_xor(im, 32);
+      if (g == 0) put(16 * NRT + x, t, re, im);
+    }
 }
 
 template <class T>
 static ecalj_status hilbert_t(ecalj_ctx* h, T* rcxq, int64_t slice, int nwhis, int nv, int ldc, const double* d_coef,
                               const double* d_scale, const double* d_dscale, cd* out, int64_t n) {
-  // chunks of at most 32 outputs (64 FP64 accumulators per lane); each chunk
-  // re-reads rcxq.  The chunks run last to first, so that the one that stores
-  // the scaled rcxq (chunk 0) runs after every other chunk has read it.
+  constexpr int U = sizeof(T) == 8 ? 4 : 2;
+  const dim3 grid((unsigned)((n + 255) / 256));
+  // chunks of at most 32 outputs (two row tiles of FP64 accumulators); each
+  // chunk re-reads rcxq.  The chunks run last to first, so that the one that
+  // stores the scaled rcxq (chunk 0) runs after every other chunk has read it.
   for (int v0 = ((nv - 1) / 32) * 32; v0 >= 0; v0 -= 32) {
     const int c = std::min(32, nv - v0);
-    const double* sc = (v0 == 0) ? d_scale : nullptr;
-    if (c <= 8)
-      hilbert_launch<8, T>(h, rcxq, slice, nwhis, c, ldc, d_coef + v0, sc, v0, d_dscale, out + n * v0, n);
-    else if (c <= 16)
-      hilbert_launch<16, T>(h, rcxq, slice, nwhis, c, ldc, d_coef + v0, sc, v0, d_dscale, out + n * v0, n);
-    else if (c <= 24)  // nf + 1 = 17..24 imaginary frequencies: no FMAs on 8 padded outputs
-      hilbert_launch<24, T>(h, rcxq, slice, nwhis, c, ldc, d_coef + v0, sc, v0, d_dscale, out + n * v0, n);
-    else
-      hilbert_launch<32, T>(h, rcxq, slice, nwhis, c, ldc, d_coef + v0, sc, v0, d_dscale, out + n * v0, n);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, h->stream, rcxq, slice, nwhis, c, ldc, d_coef + v0,
+                         (v0 == 0) ? d_scale : nullptr, v0, d_dscale, out + n * v0, n);
+    };
+    if (c <= 16) go(hilbert_kernel<1, 0, U, T>);
+    else if (c == 17) go(hilbert_kernel<1, 1, U, T>);
+    else if (c <= 21) go(hilbert_kernel<1, 5, U / 2, T>);
+    else go(hilbert_kernel<2, 0, U, T>);
     ECALJ_HIP(hipGetLastError());
   }
   return ECALJ_OK;
