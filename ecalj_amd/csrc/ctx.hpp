@@ -86,6 +86,10 @@ struct ecalj_ctx {
   std::map<std::array<int64_t, 5>, int> tuned;
   std::string tune_log;
 
+  // coefficient tables of the last imaginary- and real-axis Hilbert transform
+  // (dpsion), kept with the meshes they were made from and compared by value
+  struct HilbertPlan { std::vector<double> mesh, blob; size_t ncoef = 0; } hilbert_plan[2];
+
   // kernel timing
   bool timing = false;
   struct EvPair { hipEvent_t a, b; };
