@@ -578,7 +578,7 @@ ecalj_status wc_form(ecalj_ctx* h, const cd* inv, const int* perm, const double*
 constexpr int GJB = 32;
 // Outer pivot block.  The trailing update of each outer step is a rank-GJO
 // GEMM (K = GJO), so the matrix is read and written n/GJO times instead of
-// n/GJB times; the GJO x GJO diagonal block is inverted by the GJB scheme.
+// n/GJB times; the GJO x GJO diagonal block is inverted by gj_inv_kernel.
 constexpr int GJO = 128;
 
 __global__ __launch_bounds__(256) void gj_diag_kernel(cd* __restrict__ a, int n, int64_t lda,
@@ -644,6 +644,81 @@ __global__ __launch_bounds__(256) void gj_diag_kernel(cd* __restrict__ a, int n,
     const int i = e % b, l = e / b;
     A[(k0 + i) + lda * (k0 + l)] = cd{i == l ? 1.0 : 0.0, 0.0};
   }
+}
+
+// In-place inverse, in order, of b x b matrices with b <= GJO: the whole matrix
+// in the registers of one block (thread (ti, tj) holds rows 16 a + ti of columns
+// 32 c + tj), one Gauss-Jordan step per row, row and column kk exchanged through
+// LDS (double-buffered: one barrier per step).  One block per matrix and 128 steps
+// of 1.1 us each bound it (32 elements per thread, of which the FP64 FMAs are 0.45
+// us).  138 us for a block of 128; in GJB-wide pivot blocks (a diagonal kernel, a
+// row panel and a trailing GEMM, twelve launches) it took 250-280.
+__global__ __launch_bounds__(512) void gj_inv_kernel(cd* __restrict__ a, int64_t lda, int64_t astride, int b,
+                                                     int* __restrict__ flag) {
+  __shared__ cd row[2][GJO], col[2][GJO];
+  const int tid = threadIdx.x, ti = tid & 15, tj = tid >> 4;
+  cd* A = a + astride * blockIdx.x;
+  cd y[8][4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int i = 16 * q + ti, j = 32 * c + tj;
+      y[q][c] = (i < b && j < b) ? A[i + lda * j] : cd{0.0, 0.0};
+    }
+#pragma unroll
+  for (int a0 = 0; a0 < 8; ++a0) {
+    const int c0 = a0 / 2;  // column block of column 16 a0 + t
+    const int nt = min(16, b - 16 * a0);
+    for (int t = 0; t < nt; ++t) {
+      const int kk = 16 * a0 + t, buf = t & 1;
+      const bool mine = tj == (kk & 31);
+      if (ti == t)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) row[buf][32 * c + tj] = y[a0][c];
+      if (mine)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) col[buf][16 * q + ti] = y[q][c0];
+      __syncthreads();
+      const cd piv = row[buf][kk];
+      if (!(fabs(piv.re) + fabs(piv.im) > 2e-300) && !(hypot(piv.re, piv.im) > 1e-300)) {
+        if (tid == 0) *flag = 1;
+      }
+      const double mag = piv.re * piv.re + piv.im * piv.im;
+      const double dr = piv.re / mag, di = -piv.im / mag;  // 1/piv
+      cd xs[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const cd x = row[buf][32 * c + tj];
+        xs[c] = cd{x.re * dr - x.im * di, x.re * di + x.im * dr};
+      }
+      // column kk: 0 - f / piv, and 1 / piv at the pivot
+      if (mine) {
+        xs[c0] = cd{dr, di};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) y[q][c0] = cd{0.0, 0.0};
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const cd f = col[buf][16 * q + ti];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          y[q][c].re = fma(f.im, xs[c].im, fma(-f.re, xs[c].re, y[q][c].re));
+          y[q][c].im = fma(-f.im, xs[c].re, fma(-f.re, xs[c].im, y[q][c].im));
+        }
+      }
+      if (ti == t)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) y[a0][c] = xs[c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int i = 16 * q + ti, j = 32 * c + tj;
+      if (i < b && j < b) A[i + lda * j] = y[q][c];
+    }
 }
 
 // Row exchanges for pivot block K = [k0, k0+b), b <= GJO (partial pivoting,
@@ -934,22 +1009,20 @@ ecalj_status gj_unscramble(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astr
   return ECALJ_OK;
 }
 
-// One level: pivot blocks of GJB columns.
+// One level, n <= GJO with pivoting: pivot blocks of GJB columns.
 static ecalj_status gj_inverse_1(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astride, int nmat, int* ipiv) {
-  const bool pivot = ipiv != nullptr;
   cd *pinv, *cp;
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_GJP, sizeof(cd) * GJB * GJB * nmat, (void**)&pinv));
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_GJC, sizeof(cd) * (size_t)n * GJB * nmat, (void**)&cp));
   for (int k0 = 0; k0 < n; k0 += GJB) {
     const int b = std::min(GJB, n - k0);
-    if (pivot) {  // choose and apply the row exchanges of this block (cp is free until gj_diag)
-      hipLaunchKernelGGL(gj_panel_kernel, dim3(nmat), dim3(256), 0, h->stream, a, n, lda, astride, k0, b, cp, ipiv,
-                         h->d_flag);
-      ECALJ_HIP(hipGetLastError());
-      hipLaunchKernelGGL(gj_swap_kernel, dim3((n + 255) / 256, nmat), dim3(256), 0, h->stream, a, n, lda, astride,
-                         k0, b, ipiv);
-      ECALJ_HIP(hipGetLastError());
-    }
+    // choose and apply the row exchanges of this block (cp is free until gj_diag)
+    hipLaunchKernelGGL(gj_panel_kernel, dim3(nmat), dim3(256), 0, h->stream, a, n, lda, astride, k0, b, cp, ipiv,
+                       h->d_flag);
+    ECALJ_HIP(hipGetLastError());
+    hipLaunchKernelGGL(gj_swap_kernel, dim3((n + 255) / 256, nmat), dim3(256), 0, h->stream, a, n, lda, astride,
+                       k0, b, ipiv);
+    ECALJ_HIP(hipGetLastError());
     hipLaunchKernelGGL(gj_diag_kernel, dim3(nmat), dim3(256), 0, h->stream, a, n, lda, astride, k0, b, pinv, cp,
                        h->d_flag);
     ECALJ_HIP(hipGetLastError());
@@ -1000,7 +1073,9 @@ __global__ void gj_outer_copy_kernel(const cd* __restrict__ a, int n, int64_t ld
 
 static size_t round256(size_t b) { return ((b ? b : 256) + 255) & ~(size_t)255; }
 
-// The slot requests of gj_inverse (pivot) + gj_unscramble, in their order.
+// The slot requests of gj_inverse (pivot) + gj_unscramble, in their order; the
+// last two of n > GJO leave room for the diagonal blocks' panels, which no
+// kernel needs: the sizes that a no-allocation call takes depend on this sum.
 size_t zminv_scratch_bytes(int64_t n, int64_t nmat) {
   const size_t z = sizeof(cd), m = (size_t)nmat, N = (size_t)n;
   size_t t = round256(sizeof(int) * 2 * N * m);                             // S_GJPIV
@@ -1008,7 +1083,7 @@ size_t zminv_scratch_bytes(int64_t n, int64_t nmat) {
     t += round256(z * GJB * GJB * m) + round256(z * N * GJB * m);           // S_GJP, S_GJC
   } else {
     t += round256(z * GJO * GJO * m) + 3 * round256(z * N * GJO * m);       // S_GJD, S_GJOC, S_GJR, S_GJW
-    t += round256(z * GJB * GJB * m) + round256(z * (size_t)GJO * GJB * m); // gj_inverse_1 of the diagonal blocks
+    t += round256(z * GJB * GJB * m) + round256(z * (size_t)GJO * GJB * m);
   }
   return t + round256(z * N * N * m);                                       // S_TMP2 of gj_unscramble
 }
@@ -1023,7 +1098,10 @@ ecalj_status gj_inverse(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astride
   // Two levels above GJO: outer blocks of GJO columns.  With pivoting, the
   // exchanges of an outer block come from a blocked LU of its panel (32-wide
   // sub-panels on a copy), then the exchanged block is eliminated in order.
-  if (n <= GJO) {
+  if (n <= GJO && !pivot) {
+    hipLaunchKernelGGL(gj_inv_kernel, dim3(nmat), dim3(512), 0, h->stream, a, lda, astride, n, h->d_flag);
+    ECALJ_HIP(hipGetLastError());
+  } else if (n <= GJO) {
     ECALJ_TRY(gj_inverse_1(h, a, n, lda, astride, nmat, ipiv));
   } else {
     cd *D, *Cp, *R, *W = nullptr;
@@ -1069,7 +1147,9 @@ ecalj_status gj_inverse(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astride
                          dim3(256), 0, h->stream, a, n, lda, astride, k0, b, nmat, D, Cp, R);
       ECALJ_HIP(hipGetLastError());
       // D <- D^-1 (in order: the matrices taking this path are safe to eliminate without exchanges)
-      ECALJ_TRY(gj_inverse_1(h, D, b, GJO, (int64_t)GJO * GJO, nmat, nullptr));
+      hipLaunchKernelGGL(gj_inv_kernel, dim3(nmat), dim3(512), 0, h->stream, D, (int64_t)GJO, (int64_t)GJO * GJO, b,
+                         h->d_flag);
+      ECALJ_HIP(hipGetLastError());
       // A[K,:] = D^-1 R   (A[K,K] becomes D^-1)
       GemmCall r;
       r.M = b; r.N = n; r.K = b;
