@@ -893,37 +893,153 @@ __global__ __launch_bounds__(256) void gj_panel_lu_kernel(cd* __restrict__ w, in
   }
 }
 
-// For the panel columns j in [c0+b, bw): the sub-panel's exchanges, then
-// U12 = L11^-1 W[r0:r0+b, j] (L11 unit lower triangular).  One thread per (matrix, column).
-__global__ void gj_panel_fix_kernel(cd* __restrict__ w, int n, int r0, int c0, int b, int bw, int k0,
-                                    const int* __restrict__ ipiv, int nmat) {
-  const int ncol = bw - c0 - b;
-  const int64_t tot = (int64_t)ncol * nmat;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int mat = (int)(e / ncol), j = c0 + b + (int)(e % ncol);
-    cd* Wm = w + (int64_t)n * GJO * mat;
-    cd* col = Wm + (int64_t)n * j;
-    const int* P = ipiv + (int64_t)n * mat;
-    for (int kk = 0; kk < b; ++kk) {
-      const int r = r0 + kk, p = P[k0 + r] - k0;
-      if (p != r) {
-        const cd x = col[r];
-        col[r] = col[p];
-        col[p] = x;
+// The same with the sub-panel in registers, one row per thread (mm <= GJ_LU_ROWS
+// rows): the rows stay where they are and `pos` says where the exchanges have
+// put them, so an exchange moves nothing and the store at the end places the
+// rows.  The pivot row is broadcast through LDS.  The chain of b columns bounds
+// it (search, broadcast, update, two barriers each): 65 us at 600 rows and 32
+// columns, 45 at 250, where the panel in memory takes 309 and 140.  More rows
+// than fit the registers stay with the panel in memory.
+constexpr int GJ_LU_ROWS = 768;  // 12 waves, three per SIMD: 168 registers, 128 of them the row
+__device__ __forceinline__ double row_max16(double v) {
+  // maximum over the lane's 16: rotations by 8, 4, 2, 1
+#define ECALJ_ROR_MAX(N)                                                                          \
+  {                                                                                               \
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + N, 0xf, 0xf, false); \
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + N, 0xf, 0xf, false); \
+    v = fmax(v, __hiloint2double(hi, lo));                                                        \
+  }
+  ECALJ_ROR_MAX(8)
+  ECALJ_ROR_MAX(4)
+  ECALJ_ROR_MAX(2)
+  ECALJ_ROR_MAX(1)
+#undef ECALJ_ROR_MAX
+  return v;
+}
+// smallest idx among the lanes with v == m (at least one)
+__device__ __forceinline__ int first_of_max(double v, double m, int idx) {
+  unsigned long long eq = __ballot(v == m);
+  int best = __builtin_amdgcn_readlane(idx, __ffsll(eq) - 1);
+  for (eq &= eq - 1; eq; eq &= eq - 1) best = min(best, __builtin_amdgcn_readlane(idx, __ffsll(eq) - 1));
+  return best;
+}
+__global__ __launch_bounds__(GJ_LU_ROWS) void gj_panel_lu_reg_kernel(cd* __restrict__ w, int n, int m, int r0, int c0,
+                                                                     int b, int k0, int* __restrict__ ipiv,
+                                                                     int* __restrict__ flag) {
+  __shared__ double red_v[16];
+  __shared__ int red_i[16];
+  __shared__ cd prow[GJB];
+  cd* W = w + (int64_t)n * GJO * blockIdx.x + r0 + (int64_t)n * c0;
+  int* P = ipiv + (int64_t)n * blockIdx.x;
+  const int mm = m - r0, tid = threadIdx.x, lane = tid & 63, nwave = blockDim.x >> 6;
+  const bool has = tid < mm;
+  cd y[GJB];
+#pragma unroll
+  for (int j = 0; j < GJB; ++j) y[j] = (has && j < b) ? W[tid + (int64_t)n * j] : cd{0.0, 0.0};
+  if (tid < 16) red_v[tid] = -1.0, red_i[tid] = mm;
+  __syncthreads();  // every load above is done before the stores at the end
+  int pos = has ? tid : -1;
+#pragma unroll
+  for (int kk = 0; kk < GJB; ++kk) {
+    if (kk < b) {
+      const double s = fabs(y[kk].re) + fabs(y[kk].im);
+      const double v = (pos >= kk && s >= 0.0) ? s : -1.0;  // never a NaN
+      double mx = row_max16(v);
+      mx = fmax(mx, __shfl_xor(mx, 16));
+      mx = fmax(mx, __shfl_xor(mx, 32));
+      const int wi = first_of_max(v, mx, pos >= kk ? pos : mm);
+      if (lane == 0) {
+        red_v[tid >> 6] = mx;
+        red_i[tid >> 6] = wi;
       }
-    }
-    const cd* L = Wm + r0 + (int64_t)n * c0;
-    for (int i = 1; i < b; ++i) {
-      double sr = col[r0 + i].re, si = col[r0 + i].im;
-      for (int kk = 0; kk < i; ++kk) {
-        const cd l = L[i + (int64_t)n * kk], u = col[r0 + kk];
-        sr -= l.re * u.re - l.im * u.im;
-        si -= l.re * u.im + l.im * u.re;
+      __syncthreads();
+      const double rv = red_v[lane & 15];
+      const double vm = row_max16(rv);
+      int ip = first_of_max(rv, vm, red_i[lane & 15]);
+      if (!(vm > 1e-300)) {  // zero (or NaN) column: singular
+        if (tid == 0) *flag = 1;
+        ip = kk;
       }
-      col[r0 + i] = cd{sr, si};
+      if (pos == ip) {
+        P[k0 + r0 + kk] = k0 + r0 + ip;
+#pragma unroll
+        for (int j = kk; j < GJB; ++j) prow[j] = y[j];
+      }
+      pos = (pos == ip) ? kk : (pos == kk) ? ip : pos;
+      __syncthreads();
+      const cd piv = prow[kk];
+      const double mag = piv.re * piv.re + piv.im * piv.im;
+      if (mag > 0.0 && pos > kk) {
+        const double dr = piv.re / mag, di = -piv.im / mag;
+        const cd x = y[kk];
+        const cd l = cd{x.re * dr - x.im * di, x.re * di + x.im * dr};
+        y[kk] = l;
+#pragma unroll
+        for (int j = kk + 1; j < GJB; ++j) {
+          const cd u = prow[j];
+          y[j] = cd{y[j].re - (l.re * u.re - l.im * u.im), y[j].im - (l.re * u.im + l.im * u.re)};
+        }
+      }
     }
   }
+  if (has)
+#pragma unroll
+    for (int j = 0; j < GJB; ++j)
+      if (j < b) W[pos + (int64_t)n * j] = y[j];
+}
+
+// For the panel columns j in [c0+b, bw): the sub-panel's exchanges, then
+// U12 = L11^-1 W[r0:r0+b, j] (L11 unit lower triangular).  One lane per column,
+// its b rows in registers, L11 in LDS.  The exchanges as the permutation they
+// make: row kk comes from src[kk], and a row of the first b that they put
+// beyond them goes to dst.  (Exchange by exchange and with L11 from memory, a
+// chain of some 500 dependent loads took 102 us, whatever the size; now 25-30.)
+__global__ __launch_bounds__(64) void gj_panel_fix_kernel(cd* __restrict__ w, int n, int r0, int c0, int b, int bw,
+                                                          int k0, const int* __restrict__ ipiv) {
+  __shared__ cd L[GJB][GJB];  // L[kk][i]
+  __shared__ int piv[GJB], src[GJB], dst[GJB];
+  const int tid = threadIdx.x;
+  cd* Wm = w + (int64_t)n * GJO * blockIdx.y;
+  const int* P = ipiv + (int64_t)n * blockIdx.y;
+  for (int e = tid; e < GJB * GJB; e += 64) {
+    const int i = e % GJB, kk = e / GJB;
+    L[kk][i] = (kk < i && i < b) ? Wm[(r0 + i) + (int64_t)n * (c0 + kk)] : cd{0.0, 0.0};
+  }
+  if (tid < b) piv[tid] = P[k0 + r0 + tid] - k0 - r0;
+  __syncthreads();
+  if (tid < b) {
+    int f = tid, g = tid;  // where row tid goes; which row ends at tid
+    for (int t = 0; t < b; ++t) {
+      const int p = piv[t], u = b - 1 - t, q = piv[u];
+      f = (f == t) ? p : (f == p) ? t : f;
+      g = (g == u) ? q : (g == q) ? u : g;
+    }
+    dst[tid] = f;
+    src[tid] = g;
+  }
+  __syncthreads();
+  const int j = c0 + b + blockIdx.x * 64 + tid;
+  if (j >= bw) return;
+  cd* col = Wm + (int64_t)n * j + r0;
+  cd x[GJB];
+#pragma unroll
+  for (int i = 0; i < GJB; ++i) x[i] = (i < b) ? col[src[i]] : cd{0.0, 0.0};
+  for (int i = 0; i < b; ++i)
+    if (dst[i] >= b) col[dst[i]] = col[i];
+#pragma unroll
+  for (int kk = 0; kk < GJB; ++kk) {
+    int o = 0;  // column kk of L11 is read when x[kk] is ready: all of it at once would spill
+    asm volatile("" : "+v"(o), "+v"(x[kk].re));
+#pragma unroll
+    for (int i = kk + 1; i < GJB; ++i) {
+      const cd l = L[kk][i + o], u = x[kk];
+      x[i].re -= l.re * u.re - l.im * u.im;
+      x[i].im -= l.re * u.im + l.im * u.re;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < GJB; ++i)
+    if (i < b) col[i] = x[i];
 }
 
 // Apply the exchanges of block K to whole rows (all n columns).
@@ -1120,14 +1236,17 @@ ecalj_status gj_inverse(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astride
         ECALJ_HIP(hipGetLastError());
         for (int c0 = 0; c0 < b; c0 += GJB) {
           const int bs = std::min(GJB, b - c0);
-          hipLaunchKernelGGL(gj_panel_lu_kernel, dim3(nmat), dim3(256), 0, h->stream, W, n, m, c0, c0, bs, k0, ipiv,
-                             h->d_flag);
+          if (m - c0 <= GJ_LU_ROWS)
+            hipLaunchKernelGGL(gj_panel_lu_reg_kernel, dim3(nmat), dim3((m - c0 + 63) / 64 * 64), 0, h->stream, W, n,
+                               m, c0, c0, bs, k0, ipiv, h->d_flag);
+          else
+            hipLaunchKernelGGL(gj_panel_lu_kernel, dim3(nmat), dim3(256), 0, h->stream, W, n, m, c0, c0, bs, k0, ipiv,
+                               h->d_flag);
           ECALJ_HIP(hipGetLastError());
           const int right = b - c0 - bs;
           if (right <= 0) continue;
-          const int64_t tf = (int64_t)right * nmat;
-          hipLaunchKernelGGL(gj_panel_fix_kernel, dim3((unsigned)std::min<int64_t>((tf + 255) / 256, 65536)),
-                             dim3(256), 0, h->stream, W, n, c0, c0, bs, b, k0, ipiv, nmat);
+          hipLaunchKernelGGL(gj_panel_fix_kernel, dim3((right + 63) / 64, nmat), dim3(64), 0, h->stream, W, n, c0, c0,
+                             bs, b, k0, ipiv);
           ECALJ_HIP(hipGetLastError());
           if (m - c0 - bs <= 0) continue;
           GemmCall u;  // W[c0+bs:m, c0+bs:b] -= W[c0+bs:m, c0:c0+bs] W[c0:c0+bs, c0+bs:b]
