@@ -498,81 +498,62 @@ size_t sig_bf3_a_elems_per_k(int n, int nw1) {
 // op(X) = X, or X^H when the flag is set.  A stride / B stride 0: one operand
 // shared by every batch (split once).
 
-// A planes [b][((ks*4 + p)*MP + I)*32 + slot]; one thread per (b, ks, chunk, I), I fastest
-template <class TIN>
-__global__ __launch_bounds__(256) void split_a_kernel(const TIN* __restrict__ a, int64_t lda, int64_t a_stride,
-                                                      int m, int k, int herm, int MP, int NS,
-                                                      unsigned short* __restrict__ as, int64_t as_stride, int nb) {
+// Planes [b][((ks*4 + p)*RP + r)*32 + slot] of x(r, J), r < nr, J < k:
+// JC: x = src[J + ld r] (the k index contiguous), else src[r + ld J]; conj flips
+// the imaginary part.  One thread per (b, ks, r, chunk), chunk fastest: a wave
+// writes 16 whole rows, 1 KB, of each plane, and reads runs of 32 elements (JC)
+// or of 16.  Memory-bound (at 1200 x 1200 x 21 complex64 it reads 242 MB and
+// writes 248: 81 us JC, 95 otherwise); with r fastest it took 650 and 249.
+template <class TIN, bool JC>
+__global__ __launch_bounds__(256) void split_rows_kernel(const TIN* __restrict__ src, int64_t ld, int64_t stride,
+                                                         int nr, int k, int conj, int RP, int NS,
+                                                         unsigned short* __restrict__ out, int64_t out_stride,
+                                                         int nb) {
   typedef unsigned short us8v __attribute__((ext_vector_type(8)));
-  const int64_t per = (int64_t)NS * 4 * MP, tot = per * nb;
-  const int64_t pst = (int64_t)MP * QBK;
+  typedef float f4a8 __attribute__((ext_vector_type(4), aligned(8)));
+  const int64_t per = (int64_t)NS * 4 * RP, tot = per * nb;
+  const int64_t pst = (int64_t)RP * QBK;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot; e += (int64_t)gridDim.x * blockDim.x) {
     const int b = (int)(e / per);
-    const int64_t r = e % per;
-    const int I = (int)(r % MP);
-    const int ch = (int)((r / MP) % 4), ks = (int)(r / (4 * (int64_t)MP));
+    const int u = (int)(e % per);  // per < 2^31: 4 NS RP of a matrix that fits memory
+    const int ch = u % 4, r = (u / 4) % RP, ks = (u / 4) / RP;
+    const int J0 = ks * QBK + 8 * ch;
+    float xr[8], xi[8];
+    if (JC && sizeof(TIN) == 8 && r < nr && J0 + 8 <= k) {
+      const f4a8* p = reinterpret_cast<const f4a8*>(src + stride * b + J0 + ld * r);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f4a8 v = p[q];
+        xr[2 * q] = v[0], xi[2 * q] = v[1], xr[2 * q + 1] = v[2], xi[2 * q + 1] = v[3];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int J = J0 + q;
+        xr[q] = xi[q] = 0.f;
+        if (r < nr && J < k) {
+          const TIN x = src[stride * b + (JC ? J + ld * r : r + ld * J)];
+          xr[q] = (float)x.re;
+          xi[q] = (float)x.im;
+        }
+      }
+    }
     us8v rh, rl, ih, il;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      const int J = ks * QBK + 8 * ch + q;
-      float xr = 0.f, xi = 0.f;
-      if (I < m && J < k) {
-        const TIN x = herm ? a[a_stride * b + J + lda * I] : a[a_stride * b + I + lda * J];
-        xr = (float)x.re;
-        xi = herm ? -(float)x.im : (float)x.im;
-      }
       unsigned short h, l;
-      split_bf16(xr, h, l);
+      split_bf16(xr[q], h, l);
       rh[q] = h;
       rl[q] = l;
-      split_bf16(xi, h, l);
+      split_bf16(conj ? -xi[q] : xi[q], h, l);
       ih[q] = h;
       il[q] = l;
     }
-    unsigned short* A = as + as_stride * b + (int64_t)ks * 4 * pst + (int64_t)I * QBK + 8 * chunk_slot(I, ch);
-    *reinterpret_cast<us8v*>(A) = rh;
-    *reinterpret_cast<us8v*>(A + pst) = rl;
-    *reinterpret_cast<us8v*>(A + 2 * pst) = ih;
-    *reinterpret_cast<us8v*>(A + 3 * pst) = il;
-  }
-}
-
-// B planes [b][((ks*4 + p)*NCP + c)*32 + slot]; one thread per (b, ks, chunk, c), c fastest
-template <class TIN>
-__global__ __launch_bounds__(256) void split_b_kernel(const TIN* __restrict__ bm, int64_t ldb, int64_t b_stride,
-                                                      int k, int ncol, int herm, int NCP, int NS,
-                                                      unsigned short* __restrict__ bs, int64_t bs_stride, int nb) {
-  typedef unsigned short us8v __attribute__((ext_vector_type(8)));
-  const int64_t per = (int64_t)NS * 4 * NCP, tot = per * nb;
-  const int64_t pst = (int64_t)NCP * QBK;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < tot; e += (int64_t)gridDim.x * blockDim.x) {
-    const int b = (int)(e / per);
-    const int64_t r = e % per;
-    const int c = (int)(r % NCP);
-    const int ch = (int)((r / NCP) % 4), ks = (int)(r / (4 * (int64_t)NCP));
-    us8v rh, rl, ih, il;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int J = ks * QBK + 8 * ch + q;
-      float xr = 0.f, xi = 0.f;
-      if (c < ncol && J < k) {
-        const TIN x = herm ? bm[b_stride * b + c + ldb * J] : bm[b_stride * b + J + ldb * c];
-        xr = (float)x.re;
-        xi = herm ? -(float)x.im : (float)x.im;
-      }
-      unsigned short h, l;
-      split_bf16(xr, h, l);
-      rh[q] = h;
-      rl[q] = l;
-      split_bf16(xi, h, l);
-      ih[q] = h;
-      il[q] = l;
-    }
-    unsigned short* B = bs + bs_stride * b + (int64_t)ks * 4 * pst + (int64_t)c * QBK + 8 * chunk_slot(c, ch);
-    *reinterpret_cast<us8v*>(B) = rh;
-    *reinterpret_cast<us8v*>(B + pst) = rl;
-    *reinterpret_cast<us8v*>(B + 2 * pst) = ih;
-    *reinterpret_cast<us8v*>(B + 3 * pst) = il;
+    unsigned short* P = out + out_stride * b + (int64_t)ks * 4 * pst + (int64_t)r * QBK + 8 * chunk_slot(r, ch);
+    *reinterpret_cast<us8v*>(P) = rh;
+    *reinterpret_cast<us8v*>(P + pst) = rl;
+    *reinterpret_cast<us8v*>(P + 2 * pst) = ih;
+    *reinterpret_cast<us8v*>(P + 3 * pst) = il;
   }
 }
 
@@ -581,24 +562,22 @@ static __global__ __launch_bounds__(256) void fill_kernel(double* __restrict__ p
   if (i < n) p[i] = x;
 }
 
-template <class TIN>
-static ecalj_status split_a(ecalj_ctx* h, const void* a, int64_t lda, int64_t a_stride, int m, int k, bool herm,
-                            int MP, int NS, unsigned short* as, int64_t as_stride, int nb) {
-  const int64_t tot = (int64_t)NS * 4 * MP * nb;
+// rows of A: x(I, J) = op(A)(I, J); rows of B: x(c, J) = op(B)(J, c)
+static ecalj_status split_rows(ecalj_ctx* h, const QOperand& X, bool jc, int nr, int k, int RP, int NS,
+                               unsigned short* out, int64_t out_stride, int nb) {
+  const int64_t tot = (int64_t)NS * 4 * RP * nb;
   const int blocks = (int)std::min<int64_t>((tot + 255) / 256, 65536);
-  hipLaunchKernelGGL(split_a_kernel<TIN>, dim3(blocks), dim3(256), 0, h->stream, (const TIN*)a, lda, a_stride, m, k,
-                     herm ? 1 : 0, MP, NS, as, as_stride, nb);
-  ECALJ_HIP(hipGetLastError());
-  return ECALJ_OK;
-}
-
-template <class TIN>
-static ecalj_status split_b(ecalj_ctx* h, const void* b, int64_t ldb, int64_t b_stride, int k, int ncol, bool herm,
-                            int NCP, int NS, unsigned short* bs, int64_t bs_stride, int nb) {
-  const int64_t tot = (int64_t)NS * 4 * NCP * nb;
-  const int blocks = (int)std::min<int64_t>((tot + 255) / 256, 65536);
-  hipLaunchKernelGGL(split_b_kernel<TIN>, dim3(blocks), dim3(256), 0, h->stream, (const TIN*)b, ldb, b_stride, k,
-                     ncol, herm ? 1 : 0, NCP, NS, bs, bs_stride, nb);
+  auto go = [&](auto kern, auto* p) {
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, h->stream, p, X.ld, X.stride, nr, k, X.herm ? 1 : 0, RP, NS,
+                       out, out_stride, nb);
+  };
+  if (X.wide) {
+    if (jc) go(split_rows_kernel<cd, true>, (const cd*)X.p);
+    else go(split_rows_kernel<cd, false>, (const cd*)X.p);
+  } else {
+    if (jc) go(split_rows_kernel<cf, true>, (const cf*)X.p);
+    else go(split_rows_kernel<cf, false>, (const cf*)X.p);
+  }
   ECALJ_HIP(hipGetLastError());
   return ECALJ_OK;
 }
@@ -620,10 +599,8 @@ ecalj_status qgemm_bf3(ecalj_ctx* h, int nb, int m, int ncol, int k, const QOper
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_QW, sizeof(double) * (size_t)ncol, (void**)&w));
   hipLaunchKernelGGL(fill_kernel, dim3((ncol + 255) / 256), dim3(256), 0, h->stream, w, ncol, alpha);
   ECALJ_HIP(hipGetLastError());
-  if (A.wide) ECALJ_TRY(split_a<cd>(h, A.p, A.ld, A.stride, m, k, A.herm, MP, NS, as, ape, na));
-  else ECALJ_TRY(split_a<cf>(h, A.p, A.ld, A.stride, m, k, A.herm, MP, NS, as, ape, na));
-  if (B.wide) ECALJ_TRY(split_b<cd>(h, B.p, B.ld, B.stride, k, ncol, B.herm, NCP, NS, bs, bpe, nbb));
-  else ECALJ_TRY(split_b<cf>(h, B.p, B.ld, B.stride, k, ncol, B.herm, NCP, NS, bs, bpe, nbb));
+  ECALJ_TRY(split_rows(h, A, A.herm, m, k, MP, NS, as, ape, na));
+  ECALJ_TRY(split_rows(h, B, !B.herm, ncol, k, NCP, NS, bs, bpe, nbb));
   // the 8-wave 128 x 128 variant (the tuner's choice at the Sigma_c shapes); the output has leading dimension m
   return sig_launch_t<128, 2, 8>(h, nb, m, ncol, 1, MP, NS, NCP, as, A.stride ? ape : 0, bs, B.stride ? bpe : 0, w,
                                  0, C, c_stride, false);
