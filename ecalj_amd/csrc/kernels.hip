@@ -580,6 +580,13 @@ constexpr int GJB = 32;
 // GEMM (K = GJO), so the matrix is read and written n/GJO times instead of
 // n/GJB times; the GJO x GJO diagonal block is inverted by gj_inv_kernel.
 constexpr int GJO = 128;
+// Up to this order the outer blocks are half as wide: the updates of a small
+// matrix cost a launch, not memory, and two inverses of 64 take less than one of
+// 128 (2 x 41 us against 130).  13 matrices in order, W build: 436 against 469 us
+// at n = 150, 1040 against 1102 at 300, 1614 against 1683 at 400, no gain at 500;
+// pivoted 766 / 845, 1766 / 1914, 2594 / 2807.  One block alone (n <= GJO) is
+// inverted in one launch (284 us against 348 at 128).
+constexpr int GJ_SMALL = 400;
 
 __global__ __launch_bounds__(256) void gj_diag_kernel(cd* __restrict__ a, int n, int64_t lda,
                                                       int64_t astride, int k0, int b,
@@ -646,77 +653,89 @@ __global__ __launch_bounds__(256) void gj_diag_kernel(cd* __restrict__ a, int n,
   }
 }
 
-// In-place inverse, in order, of b x b matrices with b <= GJO: the whole matrix
-// in the registers of one block (thread (ti, tj) holds rows 16 a + ti of columns
-// 32 c + tj), one Gauss-Jordan step per row, row and column kk exchanged through
-// LDS (double-buffered: one barrier per step).  One block per matrix and 128 steps
-// of 1.1 us each bound it (32 elements per thread, of which the FP64 FMAs are 0.45
-// us).  138 us for a block of 128; in GJB-wide pivot blocks (a diagonal kernel, a
-// row panel and a trailing GEMM, twelve launches) it took 250-280.
-__global__ __launch_bounds__(512) void gj_inv_kernel(cd* __restrict__ a, int64_t lda, int64_t astride, int b,
-                                                     int* __restrict__ flag) {
-  __shared__ cd row[2][GJO], col[2][GJO];
+// 1 / x (x > 0): the hardware estimate and two Newton steps, an ulp; the exact
+// division where the estimate's range ends.  A third of the division's latency.
+__device__ __forceinline__ double fast_rcp(double x) {
+  if (!(x > 1e-290 && x < 1e290)) return 1.0 / x;
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
+// In-place inverse, in order, of b x b matrices with b <= 16 NQ: the whole matrix
+// in the registers of one block (thread (ti, tj) holds rows 16 q + ti of columns
+// NTJ c + tj), one Gauss-Jordan step per row, row and column kk exchanged through
+// LDS (double-buffered: one barrier per step).  One block per matrix and the
+// chain of steps bound it: NQ = 8, 512 threads of 8 x 4 elements, 1.0 us per step
+// (its FP64 FMAs alone 0.45), 130 us for a block of 128; NQ = 4, 256 threads of
+// 4 x 4, 41 us for a block of 64.  In GJB-wide pivot blocks (a diagonal kernel, a
+// row panel and a trailing GEMM, twelve launches) a block of 128 took 250-280.
+template <int NQ, int NTJ>
+__global__ __launch_bounds__(16 * NTJ) void gj_inv_kernel(cd* __restrict__ a, int64_t lda, int64_t astride, int b,
+                                                          int* __restrict__ flag) {
+  constexpr int NC = 16 * NQ / NTJ, N = 16 * NQ;
+  __shared__ cd row[2][N], col[2][N];
   const int tid = threadIdx.x, ti = tid & 15, tj = tid >> 4;
   cd* A = a + astride * blockIdx.x;
-  cd y[8][4];
+  cd y[NQ][NC];
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int i = 16 * q + ti, j = 32 * c + tj;
+    for (int q = 0; q < NQ; ++q) {
+      const int i = 16 * q + ti, j = NTJ * c + tj;
       y[q][c] = (i < b && j < b) ? A[i + lda * j] : cd{0.0, 0.0};
     }
 #pragma unroll
-  for (int a0 = 0; a0 < 8; ++a0) {
-    const int c0 = a0 / 2;  // column block of column 16 a0 + t
+  for (int a0 = 0; a0 < NQ; ++a0) {
+    const int c0 = 16 * a0 / NTJ;  // column block of column 16 a0 + t
     const int nt = min(16, b - 16 * a0);
     for (int t = 0; t < nt; ++t) {
       const int kk = 16 * a0 + t, buf = t & 1;
-      const bool mine = tj == (kk & 31);
+      const bool mine = tj == kk % NTJ;
       if (ti == t)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) row[buf][32 * c + tj] = y[a0][c];
+        for (int c = 0; c < NC; ++c) row[buf][NTJ * c + tj] = y[a0][c];
       if (mine)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) col[buf][16 * q + ti] = y[q][c0];
+        for (int q = 0; q < NQ; ++q) col[buf][16 * q + ti] = y[q][c0];
       __syncthreads();
       const cd piv = row[buf][kk];
       if (!(fabs(piv.re) + fabs(piv.im) > 2e-300) && !(hypot(piv.re, piv.im) > 1e-300)) {
         if (tid == 0) *flag = 1;
       }
-      const double mag = piv.re * piv.re + piv.im * piv.im;
-      const double dr = piv.re / mag, di = -piv.im / mag;  // 1/piv
-      cd xs[4];
+      const double rm = fast_rcp(piv.re * piv.re + piv.im * piv.im);
+      const double dr = piv.re * rm, di = -piv.im * rm;  // 1/piv
+      cd xs[NC];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const cd x = row[buf][32 * c + tj];
+      for (int c = 0; c < NC; ++c) {
+        const cd x = row[buf][NTJ * c + tj];
         xs[c] = cd{x.re * dr - x.im * di, x.re * di + x.im * dr};
       }
       // column kk: 0 - f / piv, and 1 / piv at the pivot
       if (mine) {
         xs[c0] = cd{dr, di};
 #pragma unroll
-        for (int q = 0; q < 8; ++q) y[q][c0] = cd{0.0, 0.0};
+        for (int q = 0; q < NQ; ++q) y[q][c0] = cd{0.0, 0.0};
       }
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
+      for (int q = 0; q < NQ; ++q) {
         const cd f = col[buf][16 * q + ti];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < NC; ++c) {
           y[q][c].re = fma(f.im, xs[c].im, fma(-f.re, xs[c].re, y[q][c].re));
           y[q][c].im = fma(-f.im, xs[c].re, fma(-f.re, xs[c].im, y[q][c].im));
         }
       }
       if (ti == t)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) y[a0][c] = xs[c];
+        for (int c = 0; c < NC; ++c) y[a0][c] = xs[c];
     }
   }
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int i = 16 * q + ti, j = 32 * c + tj;
+    for (int q = 0; q < NQ; ++q) {
+      const int i = 16 * q + ti, j = NTJ * c + tj;
       if (i < b && j < b) A[i + lda * j] = y[q][c];
     }
 }
@@ -1204,6 +1223,15 @@ size_t zminv_scratch_bytes(int64_t n, int64_t nmat) {
   return t + round256(z * N * N * m);                                       // S_TMP2 of gj_unscramble
 }
 
+static ecalj_status gj_inv(ecalj_ctx* h, cd* a, int b, int64_t lda, int64_t astride, int nmat) {
+  if (b <= 64)
+    hipLaunchKernelGGL((gj_inv_kernel<4, 16>), dim3(nmat), dim3(256), 0, h->stream, a, lda, astride, b, h->d_flag);
+  else
+    hipLaunchKernelGGL((gj_inv_kernel<8, 32>), dim3(nmat), dim3(512), 0, h->stream, a, lda, astride, b, h->d_flag);
+  ECALJ_HIP(hipGetLastError());
+  return ECALJ_OK;
+}
+
 ecalj_status gj_inverse(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astride, int nmat, const int** perm) {
   if (n == 0 || nmat == 0) return ECALJ_OK;
   if (nmat > 65535) return ECALJ_ERR_DIM;
@@ -1215,8 +1243,7 @@ ecalj_status gj_inverse(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astride
   // exchanges of an outer block come from a blocked LU of its panel (32-wide
   // sub-panels on a copy), then the exchanged block is eliminated in order.
   if (n <= GJO && !pivot) {
-    hipLaunchKernelGGL(gj_inv_kernel, dim3(nmat), dim3(512), 0, h->stream, a, lda, astride, n, h->d_flag);
-    ECALJ_HIP(hipGetLastError());
+    ECALJ_TRY(gj_inv(h, a, n, lda, astride, nmat));
   } else if (n <= GJO) {
     ECALJ_TRY(gj_inverse_1(h, a, n, lda, astride, nmat, ipiv));
   } else {
@@ -1225,8 +1252,9 @@ ecalj_status gj_inverse(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astride
     ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_GJOC, sizeof(cd) * (size_t)n * GJO * nmat, (void**)&Cp));
     ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_GJR, sizeof(cd) * (size_t)n * GJO * nmat, (void**)&R));
     if (pivot) ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_GJW, sizeof(cd) * (size_t)n * GJO * nmat, (void**)&W));
-    for (int k0 = 0; k0 < n; k0 += GJO) {
-      const int b = std::min(GJO, n - k0);
+    const int ob = n <= GJ_SMALL ? GJO / 2 : GJO;
+    for (int k0 = 0; k0 < n; k0 += ob) {
+      const int b = std::min(ob, n - k0);
       const int64_t tot = (int64_t)n * b * nmat;
       if (pivot) {
         const int m = n - k0;
@@ -1266,9 +1294,7 @@ ecalj_status gj_inverse(ecalj_ctx* h, cd* a, int n, int64_t lda, int64_t astride
                          dim3(256), 0, h->stream, a, n, lda, astride, k0, b, nmat, D, Cp, R);
       ECALJ_HIP(hipGetLastError());
       // D <- D^-1 (in order: the matrices taking this path are safe to eliminate without exchanges)
-      hipLaunchKernelGGL(gj_inv_kernel, dim3(nmat), dim3(512), 0, h->stream, D, (int64_t)GJO, (int64_t)GJO * GJO, b,
-                         h->d_flag);
-      ECALJ_HIP(hipGetLastError());
+      ECALJ_TRY(gj_inv(h, D, b, GJO, (int64_t)GJO * GJO, nmat));
       // A[K,:] = D^-1 R   (A[K,K] becomes D^-1)
       GemmCall r;
       r.M = b; r.N = n; r.K = b;

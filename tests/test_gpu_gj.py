@@ -1,5 +1,5 @@
 """The Gauss-Jordan inversion at the edges of its kernels: the in-register
-inverse of a diagonal block (tiles of 16 rows and 32 columns, blocks of 128)
+inverse of a diagonal block (tiles of 16 rows and 16 or 32 columns, blocks of 64 and 128)
 through the W build, and the pivoted panels (one row per thread up to 768 rows,
 32 columns each, exchanges as a permutation) through zminv.  FP64 against
 numpy: a backward-stable inverse is within n * cond * 2^-53 of it, below 1e-10
@@ -23,7 +23,7 @@ def crand(rng, *s):
     return rng.standard_normal(s) + 1j * rng.standard_normal(s)
 
 
-@pytest.mark.parametrize("n", [1, 15, 16, 17, 31, 33, 127, 128, 129, 145, 257])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 31, 33, 63, 64, 65, 127, 128, 129, 145, 193, 257, 400, 401])
 def test_in_order(h, n):
     print("in order", n, flush=True)
     rng = np.random.default_rng(n)
@@ -43,7 +43,7 @@ def test_in_order(h, n):
 
 
 @pytest.mark.parametrize("ties", [False, True])
-@pytest.mark.parametrize("n", [129, 161, 191, 256, 300, 769, 801, 897])
+@pytest.mark.parametrize("n", [129, 161, 191, 256, 300, 400, 401, 769, 801, 897])
 def test_pivoted(h, n, ties):
     print("pivoted", n, ties, flush=True)
     rng = np.random.default_rng(n)
