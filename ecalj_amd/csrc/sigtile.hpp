@@ -1,9 +1,10 @@
 // sigtile.hpp -- the block tile shared by the bf16x3 contractions: the
-// Sigma_c frequency contraction (sigbf3.hip), the chi0 bins (x0bf3.hip) and
-// the zmel GEMMs (zmelbf3.hip).  Operands are pre-split bf16 hi/lo planes,
-// pre-tiled per 32-wide k slice (rows of 64 bytes, the four 16-byte chunks
-// of row r stored in the order chunk ^ (((r >> 1) ^ (r >> 2)) & 3)), moved
-// global -> LDS with direct-to-LDS loads and multiplied on the bf16 MFMA.
+// Sigma_c frequency contraction (sigbf3.hip) and the zmel GEMMs
+// (zmelbf3.hip); the chi0 bins (x0bf3.hip) take the operands' layout with a
+// smaller tile.  Operands are pre-split bf16 hi/lo planes, pre-tiled per
+// 32-wide k slice (rows of 64 bytes, the four 16-byte chunks of row r stored
+// in the order chunk ^ (((r >> 1) ^ (r >> 2)) & 3)), moved global -> LDS with
+// direct-to-LDS loads and multiplied on the bf16 MFMA.
 #pragma once
 
 #include <algorithm>
@@ -49,8 +50,7 @@ template <int BN, int NSTG, int NW, bool AREAL = false>
 __device__ __forceinline__ void sig_tile(SigSmem<BN, NSTG>& s, const unsigned short* __restrict__ Ak,
                                          const unsigned short* __restrict__ Bk, const double* __restrict__ g,
                                          int n, int nw1, int v0, int nwg, int ncol, int MP, int NS, int NCP,
-                                         int I0, int c0, int accumulate, cf* __restrict__ C, int mirror = 0,
-                                         int64_t ldc = 0) {
+                                         int I0, int c0, int accumulate, cf* __restrict__ C, int64_t ldc = 0) {
   static_assert(NSTG == 2 || NSTG == 3, "two or three stages");
   static_assert(NW == 4 || NW == 8, "four or eight waves");
   constexpr int NT = NW * 64, WN = NW / 2;
@@ -225,11 +225,6 @@ __device__ __forceinline__ void sig_tile(SigSmem<BN, NSTG>& s, const unsigned sh
             *p = cf{o.re + tr[i][j][e], o.im + ti[i][j][e]};
           } else {
             *p = cf{tr[i][j][e], ti[i][j][e]};
-          }
-          if (mirror) {  // Hermitian output, off-diagonal tile: C(c, I) += conj
-            cf* q = C + c + ld * I;
-            const cf o = *q;
-            *q = cf{o.re + tr[i][j][e], o.im - ti[i][j][e]};
           }
         }
       }

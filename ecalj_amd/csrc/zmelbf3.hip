@@ -72,7 +72,7 @@ __global__ __launch_bounds__(512, 1) void zmel_bf3_kernel(const unsigned short* 
   const int b = blockIdx.z, r = blockIdx.x, c = blockIdx.y;
   const unsigned short* Bk = bs + (bdiv ? bpe * (b / bdiv) : 0);
   cf* Cb = C + (int64_t)(b % div) * c_s0 + (int64_t)(b / div) * c_s1;
-  sig_tile<128, 2, 8>(s, as + ape * b, Bk, ones, M, 1, 0, 1, N, MP, NS, NCP, r * QBM, c * 128, 0, Cb, 0, ldc);
+  sig_tile<128, 2, 8>(s, as + ape * b, Bk, ones, M, 1, 0, 1, N, MP, NS, NCP, r * QBM, c * 128, 0, Cb, ldc);
 }
 
 ecalj_status zmel_z_bf3(ecalj_ctx* h, int M, int N, int K, const cf* A, int64_t lda, int64_t a_s0, int64_t a_s1,
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(512, 1) void zmel_p_kernel(const unsigned short* __
   __shared__ SigSmem<128, 2> s;
   const int b = blockIdx.z, r = blockIdx.x, c = blockIdx.y;
   sig_tile<128, 2, 8, true>(s, as, bs + bpe * b, ones, M, 1, 0, 1, N, MP, NS, NCP, r * QBM, c * 128, 0,
-                            C + c_s1 * b, 0, ldc);
+                            C + c_s1 * b, ldc);
 }
 
 static int64_t ppb_plane_elems(const ecalj_ctx* h, int a) {
