@@ -130,10 +130,15 @@ __device__ __forceinline__ void d6_stage(D6Acc& c, const d2* a, const d2* b, int
 }
 
 // The stage wait and barrier: every load but the `left` newest has landed in
-// every wave, and every wave has left the stage before.
+// every wave, and every wave has left the stage before: its LDS reads have
+// returned (lgkmcnt 0) before the barrier, after which that stage's buffer is
+// loaded anew.  (The reads' values are there anyway when their products run,
+// so this costs nothing; without it only the compiler's order of the products
+// would keep the reads ahead of the barrier.)
 template <int LEFT>
 __device__ __forceinline__ void d6_wait() {
-  ECALJ_WAIT_VMCNT(LEFT);
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt((LEFT & 0xF) | ((LEFT >> 4) << 14) | (0x7 << 4));  // vmcnt(LEFT) lgkmcnt(0)
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_barrier();
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
