@@ -60,6 +60,7 @@ ecalj_status slot_ensure(ecalj_ctx* h, int slot, size_t bytes, void** out) {
     }
     size_t want = bytes + bytes / 8;
     if (hipMalloc(&h->slot[slot], want) != hipSuccess) {
+      (void)hipGetLastError();  // (the next launch check is not to report it)
       h->slot[slot] = nullptr;
       return ECALJ_ERR_NOMEM;
     }
@@ -67,6 +68,16 @@ ecalj_status slot_ensure(ecalj_ctx* h, int slot, size_t bytes, void** out) {
   }
   *out = h->slot[slot];
   return ECALJ_OK;
+}
+
+// Gives a slot's memory back (after the stream's work on it).
+void slot_release(ecalj_ctx* h, int slot) {
+  if (!h->slot[slot]) return;
+  (void)hipStreamSynchronize(h->stream);
+  (void)hipFree(h->slot[slot]);
+  h->slot[slot] = nullptr;
+  h->slot_bytes[slot] = 0;
+  ++h->state_gen;
 }
 
 ecalj_status timing_begin(ecalj_ctx* h, int kclass, int* idx) {

@@ -90,6 +90,10 @@ struct ecalj_ctx {
   // (dpsion), kept with the meshes they were made from and compared by value
   struct HilbertPlan { std::vector<double> mesh, blob; size_t ncoef = 0; } hilbert_plan[2];
 
+  // scratch limit of one group of k of the Sigma_c modes; halved when the device
+  // has no room for such a group
+  size_t sig_mode_cap = (size_t)16 << 30;
+
   // kernel timing
   bool timing = false;
   struct EvPair { hipEvent_t a, b; };
@@ -100,6 +104,7 @@ struct ecalj_ctx {
 namespace ecalj {
 
 ecalj_status slot_ensure(ecalj_ctx* h, int slot, size_t bytes, void** out);
+void slot_release(ecalj_ctx* h, int slot);
 void rot_free(ecalj_ctx* h);
 // Device buffer owned by one host-pointer entry point (freed on return).
 struct DevBuf {

@@ -3,6 +3,7 @@
 // extents match the buffers it was given before it is issued.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <vector>
 
@@ -1474,8 +1475,29 @@ static ecalj_status sig_final_partials(ecalj_ctx* h, const T* cz, const T* zmel,
 
 // Scratch of one group of internal k-points (operands + czmelwc).  The mode
 // form keeps the planes of every group of columns and takes twice as much, so
-// that a launch still holds several k (C3: 6 of 12).
-constexpr size_t kSigScratch = (size_t)8 << 30, kSigModeScratch = (size_t)16 << 30;
+// that a launch still holds several k (C3: 6 of 12).  A k whose planes alone
+// pass the limit (one of 21 frequencies: from n = 2150 in FP64, 3350 in bf16x3)
+// takes the plain contraction, which keeps one plane per frequency.
+// ECALJ_SIG_MODE_SCRATCH (bytes) sets a lower limit (tests of the grouping).
+constexpr size_t kSigScratch = (size_t)8 << 30;
+static size_t sig_mode_cap(const ecalj_ctx* h) {
+  size_t cap = h->sig_mode_cap;
+  if (const char* e = std::getenv("ECALJ_SIG_MODE_SCRATCH")) {
+    const long long v = std::atoll(e);
+    if (v > 0) cap = std::min(cap, (size_t)v);
+  }
+  return cap;
+}
+
+// After a failed request for the mode form's scratch: try again with groups of
+// half the size (kept in the handle, so later calls do not ask in vain), or not
+// with modes at all (under capture nothing grows).
+static bool sig_modes_retry(ecalj_ctx* h, ecalj_status st, size_t asked) {
+  if (st != ECALJ_ERR_NOMEM) return false;
+  slot_release(h, ecalj_ctx::S_WH);
+  h->sig_mode_cap = std::min(h->sig_mode_cap, asked) / 2;
+  return true;
+}
 
 template <int MODE, class T>
 static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int n, int nm, int ntq, int niw,
@@ -1492,19 +1514,6 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   const int ncol = nm * ntq;
   const int64_t nn = (int64_t)n * n;
   T *wh, *cz, *part;
-  // W unpacked (or, for bf16x3, split into bf16 planes) per internal k;
-  // processed in groups to bound scratch memory
-  const bool modes = sig_modes_pays(h, MODE, n, (int64_t)ncol * nbatch, nw1);
-  const size_t wh_bytes_per = modes ? sig_modes_bytes(MODE, n, nm, ntq, nw1)
-                              : (MODE == MBF3) ? sig_bf3_bytes_per_k(n, ncol, nw1) : sizeof(T) * nn * nw1;
-  const size_t cz_bytes_per = sizeof(T) * (size_t)n * ncol;
-  const size_t cap = modes ? kSigModeScratch : kSigScratch;
-  int group = (int)std::max<size_t>(1, std::min<size_t>(nbatch, cap / (wh_bytes_per + cz_bytes_per)));
-  group = std::min(group, 65535);
-  if (modes) group = (nbatch + (nbatch + group - 1) / group - 1) / ((nbatch + group - 1) / group);  // even parts
-  const std::vector<int> nms(modes ? group : 0, nm);
-  ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_WH, wh_bytes_per * group, (void**)&wh));
-  ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_CZ, cz_bytes_per * group, (void**)&cz));
   // final product: split-K partials of czmelwc^H zmel (K = n*nm per internal k)
   const int64_t R = (int64_t)n * nm;
   const bool direct = MODE == MBF3 && ntq <= kSigFinalMax;
@@ -1512,6 +1521,28 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   const int chunks = (int)((R + KC - 1) / KC);
   const int np = ntq * ntq;
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_PART, sizeof(T) * (size_t)np * chunks * nbatch, (void**)&part));
+  // W unpacked (or, for bf16x3, split into bf16 planes) per internal k;
+  // processed in groups to bound scratch memory
+  const size_t cz_bytes_per = sizeof(T) * (size_t)n * ncol;
+  const size_t mode_bytes_per = sig_modes_bytes(MODE, n, nm, ntq, nw1);
+  const size_t plain_bytes_per = (MODE == MBF3) ? sig_bf3_bytes_per_k(n, ncol, nw1) : sizeof(T) * nn * nw1;
+  bool modes = sig_modes_pays(h, MODE, n, (int64_t)ncol * nbatch, nw1);
+  int group;
+  for (;;) {
+    size_t cap = sig_mode_cap(h);
+    modes = modes && mode_bytes_per + cz_bytes_per <= cap;
+    if (!modes) cap = kSigScratch;
+    const size_t wh_bytes_per = modes ? mode_bytes_per : plain_bytes_per;
+    group = (int)std::max<size_t>(1, std::min<size_t>(nbatch, cap / (wh_bytes_per + cz_bytes_per)));
+    group = std::min(group, 65535);
+    if (modes) group = (nbatch + (nbatch + group - 1) / group - 1) / ((nbatch + group - 1) / group);  // even parts
+    ecalj_status st = slot_ensure(h, ecalj_ctx::S_WH, wh_bytes_per * group, (void**)&wh);
+    if (st == ECALJ_OK) st = slot_ensure(h, ecalj_ctx::S_CZ, cz_bytes_per * group, (void**)&cz);
+    if (st == ECALJ_OK) break;
+    if (!modes) return st;
+    modes = sig_modes_retry(h, st, (wh_bytes_per + cz_bytes_per) * group);
+  }
+  const std::vector<int> nms(modes ? group : 0, nm);
   const int64_t wstride = ldw * n * nw1;
   const int64_t tot = nn * nw1;
   const int ublocks = (int)std::min<int64_t>((tot + 255) / 256, 65536);
@@ -1583,25 +1614,6 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
   }
   const cf* z = (const cf*)zmel;
   const int np = ntq * ntq;
-  // scratch groups of consecutive k
-  const bool modes = sig_modes_pays(h, MBF3, n, zoff[nk], nw1);
-  const size_t cap = modes ? kSigModeScratch : kSigScratch;
-  std::vector<int> gstart{0};
-  size_t acc = 0;
-  size_t maxg = 0;
-  for (int k = 0; k < nk; ++k) {
-    const size_t b = (modes ? sig_modes_bytes(MBF3, n, nm[k], ntq, nw1)
-                            : sig_bf3_bytes_per_k(n, std::max(nm[k] * ntq, 1), nw1)) +
-                     sizeof(cf) * (size_t)n * nm[k] * ntq;
-    if (acc > 0 && acc + b > cap) {
-      gstart.push_back(k);
-      maxg = std::max(maxg, acc);
-      acc = 0;
-    }
-    acc += b;
-  }
-  maxg = std::max(maxg, acc);
-  gstart.push_back(nk);
   // chunks of the final product per k
   const bool direct = ntq <= kSigFinalMax;
   int64_t rows = 0, nparts = 0;
@@ -1622,11 +1634,40 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
   memcpy(blob.data() + tb, kst.data(), sizeof(int) * (nk + 1));
   unsigned char* dtab;
   ECALJ_TRY(upload_blob(h, ecalj_ctx::S_KST, blob, &dtab));
-  unsigned char* wh;
   cf* part;
-  ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_WH, maxg, (void**)&wh));
   ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_PART, sizeof(cf) * (size_t)np * std::max<int64_t>(nparts, 1),
                         (void**)&part));
+  // scratch groups of consecutive k
+  size_t worst = 0;
+  for (int k = 0; k < nk; ++k)
+    worst = std::max(worst, sig_modes_bytes(MBF3, n, nm[k], ntq, nw1) + sizeof(cf) * (size_t)n * nm[k] * ntq);
+  bool modes = sig_modes_pays(h, MBF3, n, zoff[nk], nw1);
+  std::vector<int> gstart;
+  unsigned char* wh;
+  for (;;) {
+    size_t cap = sig_mode_cap(h);
+    modes = modes && worst <= cap;
+    if (!modes) cap = kSigScratch;
+    gstart.assign(1, 0);
+    size_t acc = 0, maxg = 0;
+    for (int k = 0; k < nk; ++k) {
+      const size_t b = (modes ? sig_modes_bytes(MBF3, n, nm[k], ntq, nw1)
+                              : sig_bf3_bytes_per_k(n, std::max(nm[k] * ntq, 1), nw1)) +
+                       sizeof(cf) * (size_t)n * nm[k] * ntq;
+      if (acc > 0 && acc + b > cap) {
+        gstart.push_back(k);
+        maxg = std::max(maxg, acc);
+        acc = 0;
+      }
+      acc += b;
+    }
+    maxg = std::max(maxg, acc);
+    gstart.push_back(nk);
+    const ecalj_status st = slot_ensure(h, ecalj_ctx::S_WH, maxg, (void**)&wh);
+    if (st == ECALJ_OK) break;
+    if (!modes) return st;
+    modes = sig_modes_retry(h, st, maxg);
+  }
   for (size_t gi = 0; gi + 1 < gstart.size(); ++gi) {
     const int k0 = gstart[gi], k1 = gstart[gi + 1];
     cf* cz;
