@@ -1534,7 +1534,7 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
     if (!modes) cap = kSigScratch;
     const size_t wh_bytes_per = modes ? mode_bytes_per : plain_bytes_per;
     group = (int)std::max<size_t>(1, std::min<size_t>(nbatch, cap / (wh_bytes_per + cz_bytes_per)));
-    group = std::min(group, 65535);
+    group = std::min(group, modes ? sig_modes_max_k(nw1, ncol) : 65535);
     if (modes) group = (nbatch + (nbatch + group - 1) / group - 1) / ((nbatch + group - 1) / group);  // even parts
     ecalj_status st = slot_ensure(h, ecalj_ctx::S_WH, wh_bytes_per * group, (void**)&wh);
     if (st == ECALJ_OK) st = slot_ensure(h, ecalj_ctx::S_CZ, cz_bytes_per * group, (void**)&cz);
@@ -1639,8 +1639,11 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
                         (void**)&part));
   // scratch groups of consecutive k
   size_t worst = 0;
-  for (int k = 0; k < nk; ++k)
+  int maxk = nk;
+  for (int k = 0; k < nk; ++k) {
+    maxk = std::min(maxk, sig_modes_max_k(nw1, (int64_t)nm[k] * ntq));
     worst = std::max(worst, sig_modes_bytes(MBF3, n, nm[k], ntq, nw1) + sizeof(cf) * (size_t)n * nm[k] * ntq);
+  }
   bool modes = sig_modes_pays(h, MBF3, n, zoff[nk], nw1);
   std::vector<int> gstart;
   unsigned char* wh;
@@ -1654,7 +1657,7 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
       const size_t b = (modes ? sig_modes_bytes(MBF3, n, nm[k], ntq, nw1)
                               : sig_bf3_bytes_per_k(n, std::max(nm[k] * ntq, 1), nw1)) +
                        sizeof(cf) * (size_t)n * nm[k] * ntq;
-      if (acc > 0 && acc + b > cap) {
+      if (acc > 0 && (acc + b > cap || (modes && k - gstart.back() >= maxk))) {
         gstart.push_back(k);
         maxg = std::max(maxg, acc);
         acc = 0;

@@ -706,6 +706,11 @@ size_t sig_modes_bytes(int mode, int n, int nm, int ntq, int nw1) {
                (kModeMax * kModeMax * wt + sizeof(SigModeRank)) * groups + per_k + 4096);
 }
 
+// k-points whose (k, frequency) and (k, group) pairs fit one grid's y.
+int sig_modes_max_k(int nw1, int64_t ncol) {
+  return (int)std::max<int64_t>(1, 65535 / std::max<int64_t>(nw1, kModeGroups * (ncol / kModeSort + 1)));
+}
+
 // czmelwc of nk internal k-points (zmel, wgt, cz packed per k: n x nm[k] x ntq
 // and nw1 x nm[k] x ntq) in the storage type of the mode; scratch: the sum of
 // sig_modes_bytes.

@@ -113,3 +113,22 @@ def test_capture_after_a_plain_warm_up(orc, monkeypatch):  # noqa: F811
         gr.close()
     finally:
         h.close()
+
+
+@pytest.mark.parametrize("prec,nf,nk", [("f64", 20, 3300), ("f32", 20, 3300), ("f64", 7, 4200)])
+def test_more_k_than_one_grid_holds(orc, prec, nf, nk):  # noqa: F811
+    """(k, frequency) and (k, group) pairs beyond 65535: several launches."""
+    import ecalj_amd
+
+    ngb, nm, ntq = 8, 1, 2
+    four = [case(orc, 80 + k, ngb, nm, ntq, nf, "physical") for k in range(4)]
+    h = ecalj_amd.Handle(0, prec)
+    try:
+        call = uniform(h, prec, nk, ngb, nm, ntq, nf, [four[k % 4] for k in range(nk)])
+        plain = call("uniform").download()
+        h.set_tuning(MODES)
+        got = call("uniform").download()
+    finally:
+        h.close()
+    print(prec, nf, nk, relerr(got, plain), flush=True)
+    assert relerr(got, plain) < TOLS[prec]
