@@ -157,31 +157,50 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
   double* nrm = nrms + cbase;
   WT* gm = gms + cbase * nw1;
   WT* cf_ = coef + (int64_t)blockIdx.x * kModeMax * kModeMax;
-  if (t < kModeMax) {
+  if (t < 64) {  // the first wave
     double s = 0.0;
     if (t < nw1)
       for (int c = 0; c < kModeChunks; ++c) s += part[((int64_t)g.k * nw1 + t) * kModeChunks + c];
     s = sqrt(s);
-    // below FP32's normal range W rounds to zero or nearly so; a W with infinities
-    // or NaN goes unscaled, so that they reach every mode and the result
-    sv[t] = (s < 1e-36) ? 0.0 : (s < 1e300 ? s : 1.0);
+    // Only the ratios of the s_v matter (any positive s_v gives the product; they
+    // weigh its error), so they are taken relative to the largest, by a power of
+    // two: W of any scale gives the same digits.  A W at or near zero beside the
+    // others takes a floor; one whose norm is infinite or NaN, and all of them
+    // where every norm is zero, go unscaled, so that infinities and NaN reach
+    // every mode and the result.
+    double m = (s < 1e300) ? s : 0.0;
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+    int e = 0;
+    if (m > 0.0) (void)frexp(m, &e);
+    if (t < kModeMax) sv[t] = (m > 0.0 && s < 1e300) ? fmax(ldexp(s, -e), 1e-30) : 1.0;
   }
   for (int e = t; e < kModeMax * kModeMax; e += 512) cf_[e] = 0;
   __syncthreads();
   double best = 0.0;
   int bc = 0;
   for (int c = t; c < ncp; c += 512) {
-    double x[kModeMax], n2 = 0.0;
+    double x[kModeMax], m = 0.0;
+    bool bad = false;
     if (c < g.ncol) {
       const double* src = wgt + g.gsrc + (int64_t)nw1 * perm[cbase + c];
 #pragma unroll
       for (int v = 0; v < kModeMax; ++v) {
         x[v] = v < nw1 ? sv[v] * src[v] : 0.0;
-        n2 += x[v] * x[v];
+        m = fmax(m, fabs(x[v]));
+        bad |= !(fabs(x[v]) < __builtin_inf());
       }
     } else {
 #pragma unroll
       for (int v = 0; v < kModeMax; ++v) x[v] = 0.0;
+    }
+    // the norm of x / 2^e (its squares in range), inv = 1 / that norm
+    int e = 0;
+    if (m > 0.0 && !bad) (void)frexp(m, &e);
+    double n2 = 0.0;
+#pragma unroll
+    for (int v = 0; v < kModeMax; ++v) {
+      x[v] = bad ? __builtin_nan("") : ldexp(x[v], -e);
+      n2 += x[v] * x[v];
     }
     const double nr = sqrt(n2), inv = n2 > 0.0 ? 1.0 / nr : 0.0;
     double r2 = 0.0;
@@ -192,8 +211,8 @@ __global__ __launch_bounds__(512) void mode_basis_kernel(const SigMode* __restri
         X[(int64_t)v * ncp + c] = y;
         r2 += y * y;
       }
-    nrm[c] = nr;
-    gm[c] = n2 < 1e300 ? (WT)0 : (WT)__builtin_nanf("");  // (stays where no mode is found)
+    nrm[c] = ldexp(nr, e);
+    gm[c] = bad ? (WT)__builtin_nanf("") : (WT)0;  // (stays where no mode is found)
     if (r2 > best) {
       best = r2;
       bc = c;

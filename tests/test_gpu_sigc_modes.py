@@ -191,3 +191,37 @@ def test_modes_graph_replay_follows_its_inputs(orc):
         gr.close()
     finally:
         h.close()
+
+
+@pytest.mark.parametrize("wscale,gscale", [(1e-40, 1.0), (1e-170, 1.0), (1e170, 1e-20), (1.0, 1e-170), (1.0, 1e170)])
+def test_modes_f64_do_not_depend_on_the_scale(orc, wscale, gscale):
+    """FP64: W or the weights far from 1 in size, as the plain contraction takes
+    them; and frequencies whose W is zero or far smaller than the others'."""
+    import ecalj_amd
+
+    z, w, g = case(orc, 31, 130, 70, 6, 10, "physical")
+    w[:, :, 3] = 0.0
+    w[:, :, 4] *= 1e-60
+    ref = orc.sigc_imag(z, w, g)
+    h = ecalj_amd.Handle(0, "f64")
+    try:
+        h.set_tuning(MODES)
+        got = h.sigc(z, np.asfortranarray(wscale * w), np.asfortranarray(gscale * g))
+    finally:
+        h.close()
+    err = relerr(got / wscale / gscale, ref)
+    print(wscale, gscale, err, flush=True)
+    assert err < TOLS["f64"]
+
+
+@pytest.mark.parametrize("prec", ["bf16x3", "f32", "f64"])
+def test_modes_with_w_zero(orc, prec):
+    import ecalj_amd
+
+    z, w, g = case(orc, 32, 130, 70, 6, 10, "physical")
+    h = ecalj_amd.Handle(0, prec)
+    try:
+        h.set_tuning(MODES)
+        assert (h.sigc(z, np.zeros_like(w), g) == 0.0).all()
+    finally:
+        h.close()
