@@ -225,3 +225,45 @@ def test_modes_with_w_zero(orc, prec):
         assert (h.sigc(z, np.zeros_like(w), g) == 0.0).all()
     finally:
         h.close()
+
+
+@pytest.mark.parametrize("prec,exact", [("f64", np.longdouble), ("f32", np.float64)])
+@pytest.mark.parametrize("ngb,nf", [(64, 16), (96, 20), (40, 9)])
+def test_modes_err_no_more_than_the_plain_form(orc, prec, exact, ngb, nf):
+    """Few rows per element of Sigma, so that the contraction's rounding shows
+    beside the final product's; W positive, as screened interactions are, so
+    that its sums over the frequencies grow.  The elements' errors in norm
+    against wider sums (some 1500 of them, so their norm scatters by 3%)."""
+    import ecalj_amd
+
+    rng = np.random.default_rng(ngb)
+    nm, ntq = 8, 40
+    b = crand(rng, ngb, ngb)
+    x = np.concatenate([[0.0], (1.0 - np.polynomial.legendre.leggauss(nf)[0]) / (1.0 + np.polynomial.legendre.leggauss(nf)[0])])
+    w = np.asfortranarray((b @ b.conj().T)[:, :, None] / (1.0 + x ** 2))
+    z = crand(rng, ngb, nm, ntq)
+    if prec == "f32":
+        z = z.astype(np.complex64).astype(np.complex128)
+    g = np.asfortranarray(physical_weights(orc, rng, nm, ntq, nf))
+    for v in range(nf + 1):  # Hermitian to the last bit: the contraction reads the upper triangle
+        w[:, :, v] = np.triu(w[:, :, v], 1) + np.triu(w[:, :, v], 1).conj().T + np.diag(np.diag(w[:, :, v]).real)
+    zr, zi = (a.reshape(ngb, -1, order="F").astype(exact) for a in (z.real, z.imag))
+    cr, ci = np.zeros_like(zr), np.zeros_like(zr)
+    for v in range(nf + 1):
+        wr, wi, gv = w[:, :, v].real.astype(exact), w[:, :, v].imag.astype(exact), g[v].ravel(order="F").astype(exact)
+        cr += gv * (wr @ zr - wi @ zi)
+        ci += gv * (wr @ zi + wi @ zr)
+    a, b = (cr + 1j * ci).reshape(ngb * nm, ntq, order="F"), (zr + 1j * zi).reshape(ngb * nm, ntq, order="F")
+    ref = a.conj().T @ b
+    off = ~np.eye(ntq, dtype=bool)  # (the diagonal's imaginary part is clipped)
+    err = {}
+    h = ecalj_amd.Handle(0, prec)
+    try:
+        for name, mode in (("modes", MODES), ("plain", 6)):
+            h.set_tuning(mode)
+            d = (h.sigc(z, w, g) - ref)[off]
+            err[name] = float(np.sqrt((np.abs(d) ** 2).sum()) / np.sqrt((np.abs(ref[off]) ** 2).sum()))
+    finally:
+        h.close()
+    print(prec, ngb, nf, err, flush=True)
+    assert err["modes"] < err["plain"]
