@@ -654,13 +654,18 @@ __global__ __launch_bounds__(256) void gj_diag_kernel(cd* __restrict__ a, int n,
   }
 }
 
-// 1 / x (x > 0): the hardware estimate and two Newton steps, an ulp; the exact
-// division where the estimate's range ends.  A third of the division's latency.
-__device__ __forceinline__ double fast_rcp(double x) {
-  if (!(x > 1e-290 && x < 1e290)) return 1.0 / x;
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(fma(-x, r, 1.0), r, r);
-  return fma(fma(-x, r, 1.0), r, r);
+// 1 / z = conj(z) / |z|^2 with the digits of the two divisions: the hardware's
+// estimate of 1 / |z|^2, two Newton steps, and each quotient corrected by its
+// residual (which leaves it the division's in all but rare last bits).  Beyond
+// the estimate's range the divisions themselves.  A third of their latency.
+__device__ __forceinline__ cd fast_inv(cd z) {
+  const double m = z.re * z.re + z.im * z.im;
+  if (!(m > 1e-290 && m < 1e290)) return cd{z.re / m, -z.im / m};
+  double r = __builtin_amdgcn_rcp(m);
+  r = fma(fma(-m, r, 1.0), r, r);
+  r = fma(fma(-m, r, 1.0), r, r);
+  const double p = z.re * r, q = -z.im * r;
+  return cd{fma(fma(-m, p, z.re), r, p), fma(fma(-m, q, -z.im), r, q)};
 }
 
 // In-place inverse, in order, of b x b matrices with b <= 16 NQ: the whole matrix
@@ -704,8 +709,8 @@ __global__ __launch_bounds__(16 * NTJ) void gj_inv_kernel(cd* __restrict__ a, in
       if (!(fabs(piv.re) + fabs(piv.im) > 2e-300) && !(hypot(piv.re, piv.im) > 1e-300)) {
         if (tid == 0) *flag = 1;
       }
-      const double rm = fast_rcp(piv.re * piv.re + piv.im * piv.im);
-      const double dr = piv.re * rm, di = -piv.im * rm;  // 1/piv
+      const cd pinv = fast_inv(piv);
+      const double dr = pinv.re, di = pinv.im;
       cd xs[NC];
 #pragma unroll
       for (int c = 0; c < NC; ++c) {

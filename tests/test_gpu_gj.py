@@ -60,6 +60,25 @@ def test_pivoted(h, n, ties):
     assert np.abs(g - ref).max() < tol * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("scale", [1.0, 1e-120, 1e120, 1e-155])
+def test_pivot_reciprocals(h, scale):
+    """A diagonal matrix: every pivot's reciprocal alone (all other products are
+    with 0 and 1) has the digits of the two divisions conj(d) / |d|^2, up to an
+    odd last bit; at 1e-155 |d|^2 is subnormal and its divisions are exact."""
+    from fractions import Fraction
+
+    print("reciprocals", scale, flush=True)
+    n = 769
+    d = crand(np.random.default_rng(3), n) * scale
+    got = np.diag(h.zminv(np.asfortranarray(np.diag(d))))
+    same = np.zeros(n, bool)
+    for a, b in ((d.real, d.imag), (d.imag, d.real)):  # |d|^2 with either square's rounding fused away
+        m = np.array([float(Fraction(x) ** 2 + Fraction(float(y * y))) for x, y in zip(a, b)])
+        same |= got == d.conj().real / m + 1j * (d.conj().imag / m)
+    print("the divisions' digits:", same.mean(), flush=True)
+    assert same.mean() > 0.99
+
+
 @pytest.mark.parametrize("bad", [0.0, np.nan])
 def test_singular_column(h, bad):
     import ecalj_amd
