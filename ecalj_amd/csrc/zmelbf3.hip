@@ -163,7 +163,9 @@ static int64_t ppb_plane_elems(const ecalj_ctx* h, int a) {
 // until the next set_ppb, so the split (0.98 ms at C3, more than either GEMM)
 // runs once per atom and is kept, 4 bytes per element of ppb.  The build is
 // waited for, so that calls on another stream find it complete.  Without room
-// for it, or under capture before it was built, *out stays null.
+// for it, or under capture before it was built (set_ppb came between), *out
+// stays null and the call splits into S_ZPA, which every build leaves large
+// enough for any atom.
 static ecalj_status ppb_planes(ecalj_ctx* h, int a, const unsigned short** out) {
   *out = nullptr;
   const int nv = h->nv[a];
@@ -171,8 +173,14 @@ static ecalj_status ppb_planes(ecalj_ctx* h, int a, const unsigned short** out) 
   if (nvmd > 0x7fffffff - QBM) return ECALJ_ERR_DIM;
   if (h->ppb_pl.size() != h->nv.size()) h->ppb_pl.assign(h->nv.size(), nullptr);
   if (!h->ppb_pl[a]) {
-    if (h->capturing) return ECALJ_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (h->capturing || (hipStreamIsCapturing(h->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone))
+      return ECALJ_OK;
+    int64_t most = 0;
+    for (size_t b = 0; b < h->nv.size(); ++b) most = std::max(most, ppb_plane_elems(h, (int)b));
     void* p = nullptr;
+    ECALJ_TRY(slot_ensure(h, ecalj_ctx::S_ZPA, sizeof(unsigned short) * (size_t)most, &p));
+    p = nullptr;
     if (hipMalloc(&p, sizeof(unsigned short) * (size_t)el) != hipSuccess) {
       (void)hipGetLastError();
       return ECALJ_OK;

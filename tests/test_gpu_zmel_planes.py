@@ -1,6 +1,9 @@
-"""The bf16 planes of ppb that zmel keeps in the handle: rebuilt after every
-set_ppb, per atom and through the rotated-atom map, complete for a call on
-another stream, and the same results when a graph replays them."""
+"""The bf16 planes of ppb that zmel keeps in the handle: rebuilt per atom after
+every set_ppb, complete for a call on another stream, the same results when a
+graph replays them, and split anew in a graph captured before they are built.
+(The rotated-atom map: test_gpu_zmel_core.py.)"""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -69,3 +72,76 @@ def test_planes_in_a_graph():
         gr.close()
     finally:
         h.close()
+
+
+def test_capture_between_set_ppb_and_the_next_call():
+    """Warmed up, then new ppb: the capture cannot build the planes it keeps, and
+    each replay splits ppb; the eager call after it builds them."""
+    import ecalj_amd
+
+    rng = np.random.default_rng(4)
+    nv, md, nm, nq = [40, 24], [50, 70], 4, 60
+    flat = lambda: np.concatenate([rng.standard_normal((v, v, m)).ravel(order="F") for v, m in zip(nv, md)])
+    h = ecalj_amd.Handle(0, "bf16x3")
+    try:
+        h.set_ppb(nv, md, flat())
+        cm, cq = h.to_dev(crand(rng, sum(nv), nm)), h.to_dev(crand(rng, sum(nv), nq))
+        out = h.array((sum(md), nm, nq), np.complex64)
+        call = lambda: h.zmel_dev(cm, cq, out, nm=nm, nq=nq, ndima=sum(nv), zmelconjg=True)
+        call()
+        before = out.download()
+        h.set_ppb(nv, md, flat())
+        h.graph_begin()
+        try:
+            call()
+        finally:
+            gr = h.graph_end()
+        got = []
+        for _ in range(2):
+            out.zero()
+            gr.launch()
+            h.sync()
+            got.append(out.download())
+        gr.close()
+        call()
+        want = out.download()
+        assert not np.array_equal(want, before)
+        assert np.array_equal(got[0], want) and np.array_equal(got[1], want)
+    finally:
+        h.close()
+
+
+def test_planes_on_another_stream():
+    import ecalj_amd
+
+    rng = np.random.default_rng(5)
+    nv, md, nm, nq = 200, 220, 3, 50
+    h = ecalj_amd.Handle(0, "bf16x3")
+    lib = ecalj_amd.lib()
+    st = ctypes.c_void_p()
+    try:
+        ppb = rng.standard_normal((nv, nv, md))
+        cm, cq = h.to_dev(crand(rng, nv, nm)), h.to_dev(crand(rng, nv, nq))
+        out = h.array((md, nm, nq), np.complex64)
+        call = lambda: h.zmel_dev(cm, cq, out, nm=nm, nq=nq, ndima=nv, zmelconjg=True)
+        h.set_ppb([nv], [md], ppb)
+        call()
+        call()
+        want = out.download()
+        assert lib.hipStreamCreate(ctypes.byref(st)) == 0
+        for _ in range(3):
+            h.set_ppb([nv], [md], ppb)
+            out.zero()
+            h.sync()
+            call()  # builds the planes on the handle's own stream
+            h.sync()  # (the call's own scratch is of its stream)
+            h.set_stream(st.value)
+            out.zero()
+            call()
+            h.sync()
+            assert np.array_equal(out.download(), want)
+            h.set_stream(None)
+    finally:
+        h.close()
+        if st.value:
+            lib.hipStreamDestroy(st)
