@@ -156,7 +156,7 @@ __global__ __launch_bounds__(512, 1) void zmel_p_kernel(const unsigned short* __
 
 static int64_t ppb_plane_elems(const ecalj_ctx* h, int a) {
   const int64_t nvmd = (int64_t)h->nv[a] * h->mdim[a];
-  return 2 * (nvmd + QBM - 1) / QBM * QBM * pad_to(h->nv[a], QBK);
+  return 2 * ((nvmd + QBM - 1) / QBM * QBM) * pad_to(h->nv[a], QBK);
 }
 
 // bf16 planes of atom a's ppb (the relaid copy): a weight of every zmel call
