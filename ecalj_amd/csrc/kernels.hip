@@ -1532,6 +1532,8 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   const size_t mode_bytes_per = sig_modes_bytes(MODE, n, nm, ntq, nw1);
   const size_t plain_bytes_per = (MODE == MBF3) ? sig_bf3_bytes_per_k(n, ncol, nw1) : sizeof(T) * nn * nw1;
   bool modes = sig_modes_pays(h, MODE, n, (int64_t)ncol * nbatch, nw1);
+  // the FP64 modes move whole elements of zmel to LDS, 16 bytes at a time
+  if (MODE == M64) modes = modes && (uintptr_t)zmel % 16 == 0;
   int group;
   for (;;) {
     size_t cap = sig_mode_cap(h);

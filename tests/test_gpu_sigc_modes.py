@@ -267,3 +267,26 @@ def test_modes_err_no_more_than_the_plain_form(orc, prec, exact, ngb, nf):
         h.close()
     print(prec, ngb, nf, err, flush=True)
     assert err["modes"] < err["plain"]
+
+
+def test_modes_f64_zmel_at_an_odd_multiple_of_8_bytes(orc):
+    """The FP64 modes load zmel in whole 16-byte elements; one that starts between
+    them takes the plain contraction (as the FP64 GEMM's rule does)."""
+    import ecalj_amd
+
+    ngb, nm, ntq, nf = 130, 70, 6, 10
+    z, w, g = case(orc, 33, ngb, nm, ntq, nf, "physical")
+    h = ecalj_amd.Handle(0, "f64")
+    try:
+        flat = np.concatenate([[0.0], z.ravel(order="F").view(float)])
+        dz, da, dw, dg, s = h.to_dev(flat), h.to_dev(z), h.to_dev(w), h.to_dev(g), h.array((ntq, ntq))
+        out = []
+        for mode, p in ((6, da.ptr), (MODES, dz.ptr + 8)):
+            h.set_tuning(mode)
+            s.zero()
+            h.sigc_dev(1, p, ngb, nm, ntq, nf, dw, dg, s)
+            out.append(s.download())
+    finally:
+        h.close()
+    assert relerr(out[1], orc.sigc_imag(z, w, g)) < TOLS["f64"]
+    assert np.array_equal(out[0], out[1])  # the plain form's digits
