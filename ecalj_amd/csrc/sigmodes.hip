@@ -697,12 +697,13 @@ static int mode_group_tiles(int T, double f) {
 // fewer than 8 leave too little to save.  Work: the order, the bases and the
 // extra launches take about 0.2 ms, so the plain contraction has to take more
 // than about twice that (2e11 flop in the bf16x3 form, 4e10 in FP64 and FP32).
-// Tuner mode kTuneModes asks for it at any size.
+// Tuner mode kTuneModes asks for it at any size, any other forced variant for
+// the plain contraction, in every form.
 bool sig_modes_pays(const ecalj_ctx* h, int mode, int n, int64_t cols, int nw1) {
   if (nw1 > kModeMax || n < 2 || n > 13000) return false;  // n: what LdMode divides by
   if (mode == MBF3 && h->sigc_fp8) return false;
   if (h->tune_mode == kTuneModes) return true;
-  if (mode == MBF3 && h->tune_mode != 0) return false;
+  if (h->tune_mode != 0) return false;
   return nw1 >= 8 && 8.0 * n * n * nw1 * (double)cols >= (mode == MBF3 ? 2e11 : 4e10);
 }
 

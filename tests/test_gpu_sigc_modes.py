@@ -290,3 +290,23 @@ def test_modes_f64_zmel_at_an_odd_multiple_of_8_bytes(orc):
         h.close()
     assert relerr(out[1], orc.sigc_imag(z, w, g)) < TOLS["f64"]
     assert np.array_equal(out[0], out[1])  # the plain form's digits
+
+
+@pytest.mark.parametrize("prec", ["bf16x3", "f32", "f64"])
+def test_tuner_mode_chooses_the_form(orc, prec):
+    """A call large enough for the modes: mode 0 takes them, as 13 does; any other
+    forced variant takes the plain contraction."""
+    import ecalj_amd
+
+    ngb, nm, ntq, nf = (500, 300, 20, 16) if prec == "bf16x3" else (300, 205, 16, 16)
+    z, w, g = case(orc, 34, ngb, nm, ntq, nf, "physical")
+    h = ecalj_amd.Handle(0, prec)
+    try:
+        out = {}
+        for mode in (0, MODES, 6):
+            h.set_tuning(mode)
+            out[mode] = h.sigc(z, w, g)
+    finally:
+        h.close()
+    assert np.array_equal(out[0], out[MODES])
+    assert (out[6] != out[0]).any() and relerr(out[6], out[0]) < TOLS[prec]
