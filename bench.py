@@ -163,7 +163,6 @@ def run_form(qp, precision, steps, warmup, tuning=0):
     from ecalj_amd.qsgw import QPointGPU
 
     g = QPointGPU(qp, precision)
-    tuning_mode = tuning
     if tuning:
         g.h.set_tuning(tuning)
     log(f"bench[{precision}]: setup run (W_c at internal k from the first W_c(q))")
@@ -188,7 +187,7 @@ def run_form(qp, precision, steps, warmup, tuning=0):
     g.h.kernel_timing(False)
     _, _, _, eqp = g.results()
     log(f"bench[{precision}]: {steps} steps in {dt:.3f} s -> {dt / steps * 1e3:.1f} ms per q-point")
-    info = {"s_per_q": dt / steps, "ktimes": ktimes, "eqp": eqp, "nwhis": g.nwhis, "tuning": tuning, "forced": tuning_mode,
+    info = {"s_per_q": dt / steps, "ktimes": ktimes, "eqp": eqp, "nwhis": g.nwhis, "tuning": tuning,
             "npb": int(sum(g.ix.iwend - g.ix.iwini + 1))}
     g.close()
     del g
@@ -614,15 +613,14 @@ def roofline(fl, info, precision, steps, config="C2"):
     elif precision == "bf16x3" and var and var.startswith("vin4"):
         kname = ("sigv4_kernel (bf16x3 Sigma_c, frequency-inner, four real products per complex product: "
                  "W_c(iv)^H x frequency-weighted zmel, all internal k)")
-    # no tuner line and no forced variant: the launch ran over the frequency modes
-    modes = precision in ("f64", "f32") or (precision == "bf16x3" and not var and info.get("forced", 0) in (0, 13))
+    modes = "sigc_modes " in (info.get("tuning") or "")  # the library's report names the shapes that ran over the modes
     if modes:
-        kname = {"bf16x3": "sig3m_modes_kernel", "f64": "zgemm64_kernel over the modes"}.get(precision, "mode GEMM") + (
+        kname = {"bf16x3": "sig3m_modes_kernel", "f64": "mode_gemm64_kernel"}.get(precision, "mode_gemm_kernel") + (
             " (Sigma_c over frequency modes: combined W^H x weighted zmel, all internal k)")
     tr = MEASURED_TRAFFIC.get((config, precision, var))
     r = {"kernel": kname,
          "bound": "mfma", "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
-         "frac": round(achieved / peak, 4), "traffic": tr[0] if tr else None,
+         "frac": None if modes else round(achieved / peak, 4), "traffic": tr[0] if tr else None,
          "flop_per_launch": flop_launch, "avg_launch_ms": round(avg_s * 1e3, 4)}
     if tr:
         r["traffic_unit"] = "bytes per launch (HBM/fabric reads + writes, calibrated counters)"
@@ -643,7 +641,7 @@ def roofline(fl, info, precision, steps, config="C2"):
     if modes:
         r["note"] = ("achieved counts the complex flops of the contraction over every frequency (8 per complex MAC); "
                      "the frequency modes need only rank / frequencies of them (about a third in bf16x3, two thirds "
-                     "in FP64), so frac can exceed 1 and is no utilisation of the matrix cores")
+                     "in FP64), so it is no utilisation of the matrix cores and frac stays empty")
     return r
 
 

@@ -130,7 +130,7 @@ ecalj_status check_flag(ecalj_ctx* h);
 ecalj_status upload_blob(ecalj_ctx* h, int slot, const std::vector<unsigned char>& v, unsigned char** out);
 
 // ---- kernel-variant tuner
-enum TuneOp { TUNE_SIGC_BF3 = 0, TUNE_SIGC_BF3_GROUPED = 1 };
+enum TuneOp { TUNE_SIGC_BF3 = 0, TUNE_SIGC_BF3_GROUPED = 1, TUNE_SIGC_MODES = 2 };
 typedef std::array<int64_t, 5> TuneKey;
 bool tune_lookup(ecalj_ctx* h, const TuneKey& k, int* var);
 void tune_store(ecalj_ctx* h, const TuneKey& k, int var, const char* op, const std::vector<const char*>& names,

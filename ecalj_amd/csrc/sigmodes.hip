@@ -29,6 +29,7 @@
 // as 1.5 column tiles at one rank.
 #include <algorithm>
 #include <cmath>
+#include <cstdio>
 #include <cstring>
 #include <vector>
 
@@ -700,7 +701,7 @@ static int mode_group_tiles(int T, double f) {
 // Tuner mode kTuneModes asks for it at any size, any other forced variant for
 // the plain contraction, in every form.
 bool sig_modes_pays(const ecalj_ctx* h, int mode, int n, int64_t cols, int nw1) {
-  if (nw1 > kModeMax || n < 2 || n > 13000) return false;  // n: what LdMode divides by
+  if (nw1 > kModeMax || n < 2 || n > 13000) return false;  // n: what LdMode divides by (beyond it the planes pass the scratch limit in every form)
   if (mode == MBF3 && h->sigc_fp8) return false;
   if (h->tune_mode == kTuneModes) return true;
   if (h->tune_mode != 0) return false;
@@ -789,6 +790,14 @@ static ecalj_status sig_modes_t(ecalj_ctx* h, int nk, const int* nm, int ntq, co
       G = std::max(G, per);
       ncpmax = std::max(ncpmax, m.ncp);
     }
+  const TuneKey key{TUNE_SIGC_MODES, n, cols, nw1, nk};  // one line of the report per shape
+  int seen;
+  if (!tune_lookup(h, key, &seen)) {
+    h->tuned[key] = 0;
+    char line[128];
+    snprintf(line, sizeof line, "sigc_modes [%d %lld %d %d]: frequency modes\n", n, (long long)cols, nw1, nk);
+    h->tune_log += line;
+  }
   const int64_t npair = (int64_t)NS * (NS + 1) / 2;
   const int64_t blocks = 8LL * G * (((int64_t)runs.size() * R + 7) / 8);
   if (blocks > 0x7fffffff || npair > 0x7fffffff || nk > 65535 || (int64_t)nw1 * nk > 65535 || ng > 65535)

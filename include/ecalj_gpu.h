@@ -89,8 +89,8 @@ ecalj_status ecalj_kernel_time(ecalj_handle h, int kclass, double* ms, int64_t* 
  * calls of 8 to 24 frequencies run in frequency modes instead (every form but
  * fp8; no tuner run); mode 13 asks for that at any size, any other k > 0 for
  * the plain contraction, also in FP64 and FP32, which have one variant of it.
- * ecalj_tuning_report writes the decisions so far, one line per shape, as a
- * NUL-terminated string of at most len bytes. */
+ * ecalj_tuning_report writes the decisions so far, one line per shape (also
+ * for a shape that ran in frequency modes), as a NUL-terminated string of at most len bytes. */
 ecalj_status ecalj_set_tuning(ecalj_handle h, int mode);
 
 /* HIP graphs of the handle's stream (no counterpart in the reference, which

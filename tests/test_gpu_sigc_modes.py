@@ -303,9 +303,11 @@ def test_tuner_mode_chooses_the_form(orc, prec):
     h = ecalj_amd.Handle(0, prec)
     try:
         out = {}
-        for mode in (0, MODES, 6):
+        for mode in (6, 0, MODES):
             h.set_tuning(mode)
             out[mode] = h.sigc(z, w, g)
+            # the report names the shapes that ran over the modes, once each
+            assert h.tuning_report().count(f"sigc_modes [{ngb} ") == (0 if mode == 6 else 1)
     finally:
         h.close()
     assert np.array_equal(out[0], out[MODES])

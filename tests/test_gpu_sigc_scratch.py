@@ -79,6 +79,7 @@ def test_one_k_beyond_the_limit_takes_the_plain_form():
         before = free_bytes()
         h.sigc_dev(1, z, ngb, 1, 1, nf, w, g, s)
         h.sync()
+        assert "sigc_modes" not in h.tuning_report()
         taken = before - free_bytes()
         assert s.download()[0] == 0.0
     finally:
