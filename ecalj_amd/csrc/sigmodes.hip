@@ -34,17 +34,15 @@
 #include <vector>
 
 #include "gemm64.hpp"
+#include "moderule.hpp"
 #include "sig3mtile.hpp"
 
 namespace ecalj {
 
 constexpr int kModeMax = Q3NW;    // frequencies, and therefore modes, of one launch
 constexpr int kModeChunks = 16;   // partial sums of one W norm
-// Planes kept per k, in units of its frequencies: the mean rank times the
-// groups (C3: 12 groups of 6 modes; FP64 at C2: 13 of 11), with room to spare
 template <class WT>
-__host__ __device__ constexpr int mode_pool_planes() { return sizeof(WT) == 4 ? 6 : 11; }
-constexpr int kModeSort = 16384;  // columns of one sort (128 KB of LDS)
+__host__ __device__ constexpr int mode_pool_planes(int nw1) { return mode_planes(sizeof(WT) == 8, nw1); }
 // Largest residual of a column's weights, relative: 2^-25, the rounding of a
 // weight to FP32; FP64: 2^-51, the weights' own rounding with that of the steps.
 template <class G>
@@ -301,10 +299,10 @@ __global__ __launch_bounds__(256) void mode_pack_kernel(const SigMode* __restric
     if (i == (int)blockIdx.x) before = tot;
     tot += rank[i].raw;
   }
-  const bool fits = tot <= mode_pool_planes<WT>() * nw1;
+  const bool fits = tot <= mode_pool_planes<WT>(nw1);
   SigModeRank* r = rank + blockIdx.x;
   const int R = fits ? r->raw : nw1;
-  WT* cp = coefp + ((int64_t)g.k * mode_pool_planes<WT>() * nw1 + (fits ? before : 0)) * kModeMax;
+  WT* cp = coefp + ((int64_t)g.k * mode_pool_planes<WT>(nw1) + (fits ? before : 0)) * kModeMax;
   if (threadIdx.x == 0) {
     r->rank = R;
     r->poff = fits ? before : 0;
@@ -371,7 +369,7 @@ __global__ __launch_bounds__(512, 4) void mode_planes_kernel(const cd* __restric
                       8 * chunk_slot(row, wc);
   const bool put = wo == 0 || a < b;
   const int P = nplane[k];
-  const float* c0 = coefp + (int64_t)k * mode_pool_planes<float>() * nw1 * kModeMax;
+  const float* c0 = coefp + (int64_t)k * mode_pool_planes<float>(nw1) * kModeMax;
   for (int p = 0; p < P; p += 2) {
     float2(*T)[32][34] = tr[(p >> 1) & 1];
 #pragma unroll
@@ -501,7 +499,7 @@ __global__ __launch_bounds__(512) void mode_full_kernel(const cd* __restrict__ w
   const int NK = (n + 7) / 8 * 8;
   const int64_t nn = (int64_t)n * NK;
   T* A = as + pool * kpool[k];
-  const V* c0 = coefp + (int64_t)k * mode_pool_planes<V>() * nw1 * kModeMax;
+  const V* c0 = coefp + (int64_t)k * mode_pool_planes<V>(nw1) * kModeMax;
   for (int p = 0; p < P; ++p) {
     T(*L)[33] = tr[p & 1];
     const V* c = c0 + p * kModeMax;
@@ -684,16 +682,6 @@ __global__ __launch_bounds__(D6T, 4) void mode_gemm64_kernel(const SigMode* __re
 }
 
 // ---------------------------------------------------------------- host
-// Column tiles of the groups of one sort of T tiles: sqrt(f T) equal groups,
-// about the least of rank sum x tiles + the modes' cost.  bf16x3, f = 1.6:
-// a mode costs about 1.5 tiles at one rank (23 tiles: 6 groups, 90 tiles: 12);
-// FP64 / FP32 on 64-column tiles, f = 2.2: about 0.5 (45 tiles: 10 groups).
-constexpr int kModeGroups = 16;
-static int mode_group_tiles(int T, double f) {
-  const int G = std::max(1, std::min(kModeGroups, (int)(std::sqrt(f * T) + 0.5)));
-  return (T + G - 1) / G;
-}
-
 // Whether the mode form is taken.  Frequencies: one launch holds kModeMax;
 // fewer than 8 leave too little to save.  Work: the order, the bases and the
 // extra launches take about 0.2 ms, so the plain contraction has to take more
@@ -713,7 +701,7 @@ static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 // What one k of a call takes: elements of its plane pool, and whether its
 // zmel is copied in sorted order (bf16x3).
 static int64_t mode_planes_max(int mode, int nw1) {
-  return (int64_t)nw1 * (mode == M64 ? mode_pool_planes<double>() : mode_pool_planes<float>());
+  return mode_planes(mode == M64, nw1);
 }
 static int64_t mode_pool(int mode, int n, int nw1) {
   return mode_planes_max(mode, nw1) * (mode == MBF3 ? (int64_t)sig3m_a_elems_per_k(n, 1) : (int64_t)n * ((n + 7) / 8 * 8));
@@ -746,7 +734,6 @@ static ecalj_status sig_modes_t(ecalj_ctx* h, int nk, const int* nm, int ntq, co
                                 const cd* wc, int64_t ldw, int64_t w_stride, const double* wgt, T* cz,
                                 unsigned char* scratch) {
   constexpr int BN = MODE == MBF3 ? Q3BN : 64;
-  constexpr double GF = MODE == MBF3 ? 1.6 : 2.2;
   const int MP = pad_to(n, QBM), NP = pad_to(n, QBK), NS = NP / QBK, R = MODE == M32 ? (n + 63) / 64 : MP / QBM;
   const int64_t pool = mode_pool(MODE, n, nw1);
   std::vector<SigModeSort> sorts;
@@ -758,12 +745,12 @@ static ecalj_status sig_modes_t(ecalj_ctx* h, int nk, const int* nm, int ntq, co
   for (int k = 0; k < nk; ++k) {
     const int64_t N = (int64_t)nm[k] * ntq;
     if (N > 0x7fffffff / 2) return ECALJ_ERR_DIM;
-    const int TT = (int)((N + BN - 1) / BN), per = kModeSort / BN, parts = (TT + per - 1) / per;
+    const int TT = (int)((N + BN - 1) / BN), parts = mode_sorts(TT, BN);
     const int tp = parts ? (TT + parts - 1) / parts : 0;  // column tiles of one sort
     for (int t0 = 0; t0 < TT; t0 += tp) {
       const int tn = std::min(tp, TT - t0), cnt = (int)std::min<int64_t>(N - (int64_t)t0 * BN, (int64_t)tn * BN);
       sorts.push_back({co * nw1, cols, t0 * BN, cnt, tn * BN, 0});
-      const int gt = mode_group_tiles(tn, GF);
+      const int gt = mode_group_tiles(tn, parts, MODE == M64, MODE == MBF3, nw1);
       for (int g0 = 0; g0 < tn; g0 += gt) {
         const int gn = std::min(gt, tn - g0);
         grp.push_back({cols + g0 * BN, co * nw1, co * n, pools * pool, k, std::min(gn * BN, cnt - g0 * BN), gn * BN,
