@@ -1531,7 +1531,7 @@ static ecalj_status sig_contract_t(ecalj_ctx* h, int nbatch, const T* zmel, int 
   const size_t cz_bytes_per = sizeof(T) * (size_t)n * ncol;
   const size_t mode_bytes_per = sig_modes_bytes(MODE, n, nm, ntq, nw1);
   const size_t plain_bytes_per = (MODE == MBF3) ? sig_bf3_bytes_per_k(n, ncol, nw1) : sizeof(T) * nn * nw1;
-  bool modes = sig_modes_pays(h, MODE, n, (int64_t)ncol * nbatch, nw1);
+  bool modes = sig_modes_pays(h, MODE, n, nbatch, &nm, 0, ntq, nw1);
   // the FP64 modes move whole elements of zmel to LDS, 16 bytes at a time
   if (MODE == M64) modes = modes && (uintptr_t)zmel % 16 == 0;
   int group;
@@ -1651,7 +1651,7 @@ ecalj_status sig_contract_grouped(ecalj_ctx* h, int mode, int nk, const int* nm,
     maxk = std::min(maxk, sig_modes_max_k(nw1, (int64_t)nm[k] * ntq));
     worst = std::max(worst, sig_modes_bytes(MBF3, n, nm[k], ntq, nw1) + sizeof(cf) * (size_t)n * nm[k] * ntq);
   }
-  bool modes = sig_modes_pays(h, MBF3, n, zoff[nk], nw1);
+  bool modes = sig_modes_pays(h, MBF3, n, nk, nm, 1, ntq, nw1);
   std::vector<int> gstart;
   unsigned char* wh;
   for (;;) {

@@ -113,7 +113,7 @@ ecalj_status sig_final_bf3(ecalj_ctx* h, const cf* cz, const cf* z, int64_t R, i
 // one k, the k that one call takes (each of at most ncol columns), and czmelwc
 // of nk k-points packed one after the other.
 constexpr int kTuneModes = 13;  // tuner mode that asks for it
-bool sig_modes_pays(const ecalj_ctx* h, int mode, int n, int64_t cols, int nw1);
+bool sig_modes_pays(const ecalj_ctx* h, int mode, int n, int64_t nk, const int* nm, int step, int ntq, int nw1);
 size_t sig_modes_bytes(int mode, int n, int nm, int ntq, int nw1);
 int sig_modes_max_k(int nw1, int64_t ncol);
 ecalj_status sig_modes(ecalj_ctx* h, int mode, int nk, const int* nm, int ntq, const void* zmel, int n, int nw1,

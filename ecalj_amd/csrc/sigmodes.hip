@@ -682,18 +682,18 @@ __global__ __launch_bounds__(D6T, 4) void mode_gemm64_kernel(const SigMode* __re
 }
 
 // ---------------------------------------------------------------- host
-// Whether the mode form is taken.  Frequencies: one launch holds kModeMax;
-// fewer than 8 leave too little to save.  Work: the order, the bases and the
-// extra launches take about 0.2 ms, so the plain contraction has to take more
-// than about twice that (2e11 flop in the bf16x3 form, 4e10 in FP64 and FP32).
+// Whether the mode form is taken, for nk k-points of nm[step k] ntq columns:
+// 8 frequencies (fewer leave too little to save) to kModeMax (one launch holds
+// no more), and where it pays (moderule.hpp).  n: what LdMode divides by (beyond
+// it the planes pass the scratch limit in every form).
 // Tuner mode kTuneModes asks for it at any size, any other forced variant for
 // the plain contraction, in every form.
-bool sig_modes_pays(const ecalj_ctx* h, int mode, int n, int64_t cols, int nw1) {
-  if (nw1 > kModeMax || n < 2 || n > 13000) return false;  // n: what LdMode divides by (beyond it the planes pass the scratch limit in every form)
+bool sig_modes_pays(const ecalj_ctx* h, int mode, int n, int64_t nk, const int* nm, int step, int ntq, int nw1) {
+  if (nw1 > kModeMax || n < 2 || n > 13000) return false;
   if (mode == MBF3 && h->sigc_fp8) return false;
   if (h->tune_mode == kTuneModes) return true;
   if (h->tune_mode != 0) return false;
-  return nw1 >= 8 && 8.0 * n * n * nw1 * (double)cols >= (mode == MBF3 ? 2e11 : 4e10);
+  return nw1 >= 8 && mode_pays(mode == M64, mode == MBF3, n, nk, nm, step, ntq, nw1);
 }
 
 static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }

@@ -298,7 +298,7 @@ def test_tuner_mode_chooses_the_form(orc, prec):
     forced variant takes the plain contraction."""
     import ecalj_amd
 
-    ngb, nm, ntq, nf = (500, 300, 20, 16) if prec == "bf16x3" else (300, 205, 16, 16)
+    ngb, nm, ntq, nf = (512, 420, 24, 20) if prec == "bf16x3" else (300, 205, 16, 16)
     z, w, g = case(orc, 34, ngb, nm, ntq, nf, "physical")
     h = ecalj_amd.Handle(0, prec)
     try:

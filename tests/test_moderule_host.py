@@ -1,6 +1,6 @@
 """The sizes of the Sigma_c mode form (ecalj_amd/csrc/moderule.hpp, compiled
 here for the host with g++): the planes kept for the modes hold those of
-physical weights."""
+physical weights, and the form is taken where it was measured faster."""
 import ctypes as C
 import os
 import subprocess
@@ -27,6 +27,12 @@ def orc():
 
     oracle.build()
     return oracle
+
+
+def pays(rule, form, n, nms, ntq, nf):
+    nms = np.asarray(nms, np.int32)
+    return rule.moderule_pays(int(form == "f64"), int(form == "bf16x3"), n, len(nms),
+                              nms.ctypes.data_as(C.POINTER(C.c_int)), 1, ntq, nf + 1)
 
 
 def rank(x, tol):
@@ -69,3 +75,29 @@ def test_planes_hold_the_modes_of_physical_weights(rule, orc, form, nf, nm, ntq)
             total += rank(part[:, c:c + gt * bn], 2.0 ** -51 if f64 else 2.0 ** -25)
     print(form, nf, cols, "modes", total, "planes", rule.moderule_planes(f64, nf + 1))
     assert total <= rule.moderule_planes(f64, nf + 1)
+
+
+# (form, n, middle states per k, end states, frequencies - 1), us of the modes, us of the plain form (MI355X)
+MEASURED = [
+    ("f64", 300, [155] * 4, 10, 8, 2019, 1459), ("f64", 300, [205], 30, 12, 2270, 1712),
+    ("f64", 600, [155] * 2, 10, 8, 2948, 2315), ("f64", 60, [605] * 4, 32, 20, 3152, 1869),
+    ("f64", 300, [318], 36, 7, 3067, 2470), ("f64", 600, [159] * 8, 18, 16, 14400, 25450),
+    ("f32", 300, [605], 32, 7, 2296, 1937), ("f32", 60, [605] * 8, 32, 8, 1397, 1098),
+    ("f32", 300, [205] * 3, 20, 23, 1424, 3020), ("f32", 128, [305] * 8, 36, 20, 1685, 3114),
+    ("bf16x3", 200, [605] * 4, 32, 8, 1073, 764), ("bf16x3", 450, [605], 32, 7, 1068, 752),
+    ("bf16x3", 600, [65] * 8, 8, 16, 951, 752), ("bf16x3", 1200, [155], 18, 7, 849, 654),
+    ("bf16x3", 600, [159] * 16, 18, 16, 3380, 5077), ("bf16x3", 1200, [318] * 12, 36, 20, 28500, 66570),
+    ("bf16x3", 1080, [424, 158, 300, 250, 200, 350, 400, 180, 280], 16, 20, 10150, 20570),
+]
+
+
+@pytest.mark.parametrize("form,n,nms,ntq,nf,modes,plain", MEASURED)
+def test_the_faster_form_is_taken(rule, form, n, nms, ntq, nf, modes, plain):
+    assert bool(pays(rule, form, n, nms, ntq, nf)) == (modes < plain)
+
+
+def test_edges(rule):
+    assert not pays(rule, "bf16x3", 1200, [0, 0], 36, 20)          # no columns
+    assert not pays(rule, "f64", 100, [3], 2, 20)                  # too little work to be measured
+    assert pays(rule, "bf16x3", 1200, [0, 318, 0, 318], 36, 20)    # empty k between
+    assert not pays(rule, "bf16x3", 600, [3000], 40, 20)           # eight sorts: more modes than planes
