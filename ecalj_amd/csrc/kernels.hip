@@ -356,11 +356,70 @@ __global__ __launch_bounds__(256, 2) void hilbert_kernel(T* __restrict__ rcxq, i
     }
 }
 
+// The same for up to NV outputs with a thread per element, four bins' loads in
+// flight, the coefficients through the scalar cache: no 16-wide row tile to fill.
+template <int NV, class T>
+__global__ __launch_bounds__(256) void hilbert_few_kernel(T* __restrict__ rcxq, int64_t slice, int nwhis, int nv,
+                                                          int ldc, const double* __restrict__ coef,
+                                                          const double* __restrict__ scale, int v0,
+                                                          const double* __restrict__ dscale, cd* __restrict__ out,
+                                                          int64_t n) {
+  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  double ar[NV], ai[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) ar[v] = ai[v] = 0.0;
+  auto bins = [&](auto cnt, int iw) {
+    constexpr int N = decltype(cnt)::value;
+    T x[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) x[u] = rcxq[e + slice * (iw + u)];
+    if (scale) {
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const double s = scale[iw + u - 1];
+        st_c(rcxq + e + slice * (iw + u), s * x[u].re, s * x[u].im);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const double* c = coef + (int64_t)ldc * (iw + u - 1);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        ar[v] += c[v] * x[u].re;
+        ai[v] += c[v] * x[u].im;
+      }
+    }
+  };
+  int iw = 1;
+  for (; iw + 3 <= nwhis; iw += 4) bins(std::integral_constant<int, 4>{}, iw);
+  for (; iw <= nwhis; ++iw) bins(std::integral_constant<int, 1>{}, iw);
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+    if (v < nv) {
+      if (dscale) {
+        const T x = rcxq[e + slice * (v0 + v)];
+        const double s = dscale[v0 + v];
+        ar[v] -= s * x.im;
+        ai[v] += s * x.re;
+      }
+      out[e + n * v] = cd{ar[v], ai[v]};
+    }
+}
+
 template <class T>
 static ecalj_status hilbert_t(ecalj_ctx* h, T* rcxq, int64_t slice, int nwhis, int nv, int ldc, const double* d_coef,
                               const double* d_scale, const double* d_dscale, cd* out, int64_t n) {
   constexpr int U = sizeof(T) == 8 ? 4 : 2;
   const dim3 grid((unsigned)((n + 255) / 256));
+  // Outputs that the thread-per-element kernel takes: memory bounds both, the row
+  // tile of 16 the other more, from slices of 2 MB on; below, its chain of bins is
+  // the longer one.  Its time and the tile's (us, 130 bins): complex64, 600 x 600, 1
+  // output 89 / 116, 6 111 / 123, 8 145 / 125; 1000 x 1000, 8 252 / 284, 9 295 / 288;
+  // complex128, 400 x 400, 4 77 / 88, 5 94 / 89; 600 x 600, 8 173 / 183; 200 x 200, 1
+  // output 55 / 41.
+  const double slice_mb = 1e-6 * n * sizeof(T);
+  const int few = slice_mb >= 5 ? 8 : slice_mb >= 2 ? (sizeof(T) == 8 ? 6 : 4) : 0;
   // chunks of at most 32 outputs (two row tiles of FP64 accumulators); each
   // chunk re-reads rcxq.  The chunks run last to first, so that the one that
   // stores the scaled rcxq (chunk 0) runs after every other chunk has read it.
@@ -370,7 +429,8 @@ static ecalj_status hilbert_t(ecalj_ctx* h, T* rcxq, int64_t slice, int nwhis, i
       hipLaunchKernelGGL(kern, grid, dim3(256), 0, h->stream, rcxq, slice, nwhis, c, ldc, d_coef + v0,
                          (v0 == 0) ? d_scale : nullptr, v0, d_dscale, out + n * v0, n);
     };
-    if (c <= 16) go(hilbert_kernel<1, 0, U, T>);
+    if (c <= few) go(hilbert_few_kernel<8, T>);
+    else if (c <= 16) go(hilbert_kernel<1, 0, U, T>);
     else if (c == 17) go(hilbert_kernel<1, 1, U, T>);
     else if (c <= 21) go(hilbert_kernel<1, 5, U / 2, T>);
     else go(hilbert_kernel<2, 0, U, T>);

@@ -46,3 +46,31 @@ def test_dpsion_meshes(nwhis, niw, shape, prec, tol):
             assert rel(x[:, :, 1:], y[:, :, 1:]) < tol  # scaled in place
     finally:
         h.close()
+
+
+# slices from 2 MB (up to 4 or 6 outputs) and from 5 MB (up to 8) take a thread per element; bins around its
+# rounds of four; 33 outputs: one in the second chunk
+@pytest.mark.parametrize("prec,tol", [("f64", 1e-13), ("bf16x3", 2.0 ** -23)])
+@pytest.mark.parametrize("nwhis,niw,shape", [(1, 1, (700, 907)), (4, 4, (301, 500)), (5, 6, (500, 517)),
+                                             (7, 8, (700, 907)), (10, 9, (700, 907)), (6, 33, (700, 907))])
+def test_dpsion_few_outputs(nwhis, niw, shape, prec, tol):
+    import ecalj_amd
+    import oracle as orc
+
+    orc.build()
+    rng = np.random.default_rng(nwhis)
+    r = (rng.standard_normal((*shape, nwhis + 1), np.float32) + 1j * rng.standard_normal((*shape, nwhis + 1), np.float32))
+    r = np.asfortranarray(r.astype(np.complex128))
+    fr, nu = mesh(nwhis), np.concatenate([[0.0], np.sort(rng.uniform(0.01, 2.0, niw - 1))])
+    h = ecalj_amd.Handle(0, prec)
+    try:
+        x, y = r.copy(order="F"), r.copy(order="F")
+        g = h.dpsion_imag(x, fr, nu)
+        o = orc.dpsion_imag(y, fr, orc.imatt(nu, fr))
+        assert rel(g, o) < 1e-10
+        assert rel(x[:, :, 1:], y[:, :, 1:]) < tol
+        if nwhis > niw:  # the real axis' own term
+            w = np.linspace(0.0, 1.0, niw + 1)
+            assert rel(h.dpsion_real(r, fr, w), orc.dpsion_real(r, fr, orc.rmatt(w, fr))) < 1e-9
+    finally:
+        h.close()
