@@ -201,6 +201,7 @@ template <bool TA, bool TB, int EPI>
 static ecalj_status mlp_gemm(ecalj_ctx* h, const MlpGemm& g) {
   if (g.M <= 0 || g.N <= 0) return ECALJ_OK;
   const int64_t tiles = mlp_tiles(g.M, g.N);
+  // batches beyond 65535 row tiles of the inference kernel, which its grid cannot hold, are refused here too
   if ((g.M + MT - 1) / MT > 65535 || tiles > 0x7fffffff) return ECALJ_ERR_DIM;
   hipLaunchKernelGGL((mlp_gemm_kernel<TA, TB, EPI>), dim3((unsigned)tiles), dim3(64 * GW), 0, h->stream, g);
   ECALJ_HIP(hipGetLastError());

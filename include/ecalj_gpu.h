@@ -85,9 +85,9 @@ ecalj_status ecalj_kernel_time(ecalj_handle h, int kclass, double* ms, int64_t* 
  * always variant k.  Tuned kernels: the bf16x3 Sigma_c contraction (variants
  * 1 = 128x64 tiles, 3 stages, 4 waves; 2 = 128x128 tiles, 2 stages, 4 waves;
  * 3 = 128x128, 2 stages, 8 waves; 4 = variant 3 with the XCD-aware block
- * order), and its grouped form (variants 1-3; k > 3 wraps).  Large Sigma_c
- * calls of 8 to 24 frequencies run in frequency modes instead (every form but
- * fp8; no tuner run); mode 13 asks for that at any size, any other k > 0 for
+ * order), and its grouped form (variants 1-3; k > 3 wraps).  Sigma_c calls of
+ * 8 to 24 frequencies run in frequency modes instead where a model of both
+ * forms' times has them faster (every form but fp8; no tuner run); mode 13 asks for that at any size, any other k > 0 for
  * the plain contraction, also in FP64 and FP32, which have one variant of it.
  * ecalj_tuning_report writes the decisions so far, one line per shape (also
  * for a shape that ran in frequency modes), as a NUL-terminated string of at most len bytes. */
